@@ -149,24 +149,91 @@ __global__ __launch_bounds__(256) void residual_partial_kernel(const cplx *hpsi,
   }
 }
 
-__global__ void column_sum_kernel(const double *partial, int nchunk, int nst, double scale,
-                                  double *out) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nst) return;
-  double v = 0.0;
-  for (int c = 0; c < nchunk; c++) v += partial[((long)c * nst + b) * 2 + 0];
-  out[b] = scale * v;
+// Totals of the [nchunk][nst][2] partials, FIN_BT bands per workgroup: a thread
+// takes one band of chunks lane, lane + FIN_LANES, ... (eight bands of a chunk
+// are one 128-byte line), the lanes of a band are added by a butterfly within
+// each wave and the waves in order, so the order is fixed.  Bound by latency:
+// one thread per band walking the chunks, as this ran before, is a serial chain
+// of nchunk loads and adds (422 us a call for 1024 chunks x 256 bands, 106 us
+// for 456 x 48).  With non_local_energy_kernel in place of V_nl psi on the whole
+// grid, ham.energy, density, dipole and current of 36 x 36 x 90 x 48 bands take
+// 694 us against 1101.
+//   RATIO: eps[b] = sum of column 0 / sum of column 1, the latter also into
+//          norm[b] when given; else eps[b] = scale * sum of column 0
+constexpr int FIN_BT = 8;
+constexpr int FIN_LANES = 128;
+constexpr int FIN_WAVES = FIN_BT * FIN_LANES / 64;
+
+template <bool RATIO>
+__global__ __launch_bounds__(FIN_BT *FIN_LANES) void band_totals_kernel(
+    const double *__restrict__ partial, int nchunk, int nst, double scale, double *eps,
+    double *norm) {
+  __shared__ double red[FIN_WAVES][FIN_BT][2];
+  const int bb = threadIdx.x % FIN_BT, lane = threadIdx.x / FIN_BT;
+  const int b = blockIdx.x * FIN_BT + bb;
+  double v = 0.0, nn = 0.0;
+  if (b < nst) {
+#pragma unroll 4
+    for (int c = lane; c < nchunk; c += FIN_LANES) {
+      const double2 t = reinterpret_cast<const double2 *>(partial)[(long)c * nst + b];
+      v += t.x;
+      if constexpr (RATIO) nn += t.y;
+    }
+  }
+#pragma unroll
+  for (int w = FIN_BT; w < 64; w <<= 1) {
+    v += __shfl_xor(v, w, 64);
+    if constexpr (RATIO) nn += __shfl_xor(nn, w, 64);
+  }
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) < FIN_BT) {
+    red[wave][bb][0] = v;
+    red[wave][bb][1] = nn;
+  }
+  __syncthreads();
+  if (threadIdx.x < FIN_BT && b < nst) {
+    for (int w = 1; w < FIN_WAVES; w++) {
+      v += red[w][bb][0];
+      if constexpr (RATIO) nn += red[w][bb][1];
+    }
+    if constexpr (RATIO) {
+      eps[b] = v / nn;
+      if (norm) norm[b] = nn;
+    } else {
+      eps[b] = scale * v;
+    }
+  }
 }
 
-__global__ void energies_final_kernel(const double *partial, int nchunk, int nst, double *eps) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nst) return;
-  double v = 0.0, nn = 0.0;
-  for (int c = 0; c < nchunk; c++) {
-    v += partial[((long)c * nst + b) * 2 + 0];
-    nn += partial[((long)c * nst + b) * 2 + 1];
+// nl[b] = Re<V_nl psi_b|psi_b> / <psi_b|psi_b> from the projector coefficients
+// P = dV D p, p = sum_i M_i e^{i(k+A).r_i} psi(r_i): the sum over grid points of
+// conj(V_nl psi) psi is sum_{sphere, lm} dV D |p|^2 = sum |P|^2 / (dV D) (a
+// channel with D = 0 adds nothing).  nl holds the norms on entry.  The rows
+// (sphere, lm) are dealt over the lanes as in band_totals_kernel.
+__global__ __launch_bounds__(FIN_BT *FIN_LANES) void non_local_energy_kernel(
+    const cplx *__restrict__ P, const double *__restrict__ coeff, int nrows, int nst, double dV,
+    double *nl) {
+  __shared__ double red[FIN_WAVES][FIN_BT];
+  const int bb = threadIdx.x % FIN_BT, lane = threadIdx.x / FIN_BT;
+  const int b = blockIdx.x * FIN_BT + bb;
+  double v = 0.0;
+  if (b < nst) {
+#pragma unroll 4
+    for (int r = lane; r < nrows; r += FIN_LANES) {
+      const double d = coeff[r];
+      const cplx c = P[(long)r * nst + b];
+      if (d != 0.0) v += (c.x * c.x + c.y * c.y) / (dV * d);
+    }
   }
-  eps[b] = v / nn;
+#pragma unroll
+  for (int w = FIN_BT; w < 64; w <<= 1) v += __shfl_xor(v, w, 64);
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) < FIN_BT) red[wave][bb] = v;
+  __syncthreads();
+  if (threadIdx.x < FIN_BT && b < nst) {
+    for (int w = 1; w < FIN_WAVES; w++) v += red[w][bb];
+    nl[b] = v / nl[b];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -723,14 +790,15 @@ void exponential_2_for_1(handle &h, std::complex<double> z1, std::complex<double
 // The two launches of the band energies with their [nchunk][nst][2] partial
 // sums in `partial` (every entry the final kernel reads is written first)
 static void band_energies_with(handle &h, const cplx *hpsi, long hld, const cplx *psi, long ld,
-                               int nst, double *eps, double *partial) {
+                               int nst, double *eps, double *partial, double *norm = nullptr) {
   const int nchunk = (int)((h.npoint + EN_CHUNK - 1) / EN_CHUNK);
   dim3 grid(nchunk, (nst + EN_BT - 1) / EN_BT);
   hipLaunchKernelGGL(energies_partial_kernel, grid, dim3(256), 0, h.stream, hpsi, hld, psi, ld,
                      nst, h.npoint, partial);
   INQAMD_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(energies_final_kernel, dim3((nst + 63) / 64), dim3(64), 0, h.stream,
-                     (const double *)partial, nchunk, nst, eps);
+  hipLaunchKernelGGL(band_totals_kernel<true>, dim3((nst + FIN_BT - 1) / FIN_BT),
+                     dim3(FIN_BT * FIN_LANES), 0, h.stream, (const double *)partial, nchunk, nst,
+                     1.0, eps, norm);
   INQAMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -1194,23 +1262,29 @@ int inqamd_energy(inqamd_hamiltonian_t h, const void *psi, int nst, int ld, doub
     const cplx *f = (const cplx *)psi;
     // residual = H phi; eps = Re<residual|phi>/<phi|phi> (energy.hpp:74-75)
     hamiltonian_apply(*h, f, ld, h->hn, nst, nst, KA_CURRENT);
-    band_energies(*h, h->hn, nst, f, ld, nst, eps);
+    // (the norms wait in nl for the last kernel)
+    band_energies_with(*h, h->hn, nst, f, ld, nst, eps, h->partial, nl);
     // normres = dV |residual - eps phi|^2 (:76-77)
     const int nchunk = (int)((h->npoint + EN_CHUNK - 1) / EN_CHUNK);
     hipLaunchKernelGGL(residual_partial_kernel, dim3(nchunk, (nst + EN_BT - 1) / EN_BT),
                        dim3(256), 0, h->stream, (const cplx *)h->hn, (long)nst, f, (long)ld,
                        (const double *)eps, nst, h->npoint, h->partial);
     INQAMD_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(column_sum_kernel, dim3((nst + 63) / 64), dim3(64), 0, h->stream,
+    const dim3 fg((nst + FIN_BT - 1) / FIN_BT);
+    hipLaunchKernelGGL(band_totals_kernel<false>, fg, dim3(FIN_BT * FIN_LANES), 0, h->stream,
                        (const double *)h->partial, nchunk, nst, h->volume / (double)h->npoint,
-                       normres);
+                       normres, (double *)nullptr);
     INQAMD_HIP_CHECK(hipGetLastError());
-    // nl = Re<V_nl phi|phi>/<phi|phi> (:81-85)
-    INQAMD_HIP_CHECK(hipMemsetAsync(h->hn2, 0, (size_t)h->npoint * nst * sizeof(cplx), h->stream));
-    projector_phases(*h, KA_CURRENT);
-    projector_project_expand(*h, f, ld, nst, nullptr, 0, true);
-    projector_apply_coefficients(*h, h->hn2, nst, nst, KA_CURRENT);
-    band_energies(*h, h->hn2, nst, f, ld, nst, nl);
+    // nl = Re<V_nl phi|phi>/<phi|phi> (:81-85) from the coefficients, which the
+    // H application left in h->proj unless it kept V_nl phi per entry.  (V_nl phi
+    // was formed on the whole grid for it: a clear, the projector again, the
+    // scatter and a pass over both arrays.)
+    if (h->three_sweep && h->pt.nproj > 0 && !vnl_from_coefficients(*h))
+      projector_project_expand(*h, f, ld, nst, nullptr, 0, true);
+    hipLaunchKernelGGL(non_local_energy_kernel, fg, dim3(FIN_BT * FIN_LANES), 0, h->stream,
+                       (const cplx *)h->proj, (const double *)h->pt.coeff,
+                       h->pt.nproj * h->pt.max_nlm, nst, h->volume / (double)h->npoint, nl);
+    INQAMD_HIP_CHECK(hipGetLastError());
   });
 }
 
