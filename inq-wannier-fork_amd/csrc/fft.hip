@@ -268,7 +268,7 @@ static int reg_variant(const fft_pass_args &a) {
 
 void fft_launch_pass(const fft_pass_args &a, int mode, hipStream_t stream) {
   const int v = reg_variant(a);
-  if (v < 10 && fft_plan_launch(a, mode, a.nst >= 16 ? 16 : 8, stream)) return;
+  if (v < 10 && fft_plan_launch(a, mode, stream)) return;
   if (fft_reg_supported(a)) {
     fft_reg_launch(a, mode, v % 10, stream);
     return;

@@ -76,9 +76,9 @@ void fft_launch_pass(const fft_pass_args &a, int mode, hipStream_t stream);
 bool fft_reg_supported(const fft_pass_args &a);
 void fft_reg_launch(const fft_pass_args &a, int mode, int variant, hipStream_t stream);
 
-// Plan-specialised pass (fft_plan.hip) for the tabulated lengths and band
-// tiles B in {8, 16}; returns false when (len, B) has no instantiation.
-bool fft_plan_launch(const fft_pass_args &a, int mode, int B, hipStream_t stream);
+// Plan-specialised pass (fft_plan.hip) for the tabulated lengths; returns
+// false when the length has no instantiation.
+bool fft_plan_launch(const fft_pass_args &a, int mode, hipStream_t stream);
 
 // Arguments of the three-sweep local Hamiltonian (fft3.hip) on a band chunk
 // of a cubic L^3 grid.

@@ -64,6 +64,37 @@ __device__ __forceinline__ void dft<5>(cplx *v, int sign) {
 }
 
 template <>
+__device__ __forceinline__ void dft<7>(cplx *v, int sign) {
+  // cos and sin of 2 pi k/7, k = 1, 2, 3
+  constexpr double c[3] = {0.62348980185873353, -0.22252093395631440, -0.90096886790241913};
+  constexpr double s[3] = {0.78183148246802981, 0.97492791218182361, 0.43388373911755812};
+  cplx t[3], d[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    t[k] = cadd(v[k + 1], v[6 - k]);
+    d[k] = csub(v[k + 1], v[6 - k]);
+  }
+  const cplx v0 = v[0];
+  v[0] = cadd(v0, cadd(t[0], cadd(t[1], t[2])));
+#pragma unroll
+  for (int j = 1; j <= 3; j++) {
+    cplx m = v0, n = mk(0.0, 0.0);
+#pragma unroll
+    for (int k = 1; k <= 3; k++) {
+      const int r = (j * k) % 7;  // 2 pi j k/7 folded onto k = 1, 2, 3
+      const double cc = c[(r <= 3 ? r : 7 - r) - 1], ss = r <= 3 ? s[r - 1] : -s[6 - r];
+      m.x += cc * t[k - 1].x;
+      m.y += cc * t[k - 1].y;
+      n.x += ss * d[k - 1].x;
+      n.y += ss * d[k - 1].y;
+    }
+    n = mul_i(n, sign);
+    v[j] = cadd(m, n);
+    v[7 - j] = csub(m, n);
+  }
+}
+
+template <>
 __device__ __forceinline__ void dft<8>(cplx *v, int sign) {
   const double h = 0.70710678118654752440084436210485;  // 1/sqrt(2)
   cplx u[4], w[4];
@@ -85,7 +116,7 @@ __device__ __forceinline__ void dft<8>(cplx *v, int sign) {
   }
 }
 
-// cos and sin of 2 pi m / N for the composite butterflies (N = 6, 9, 12),
+// cos and sin of 2 pi m / N for the composite butterflies (N = 6, 9, 10, 12),
 // the correctly rounded doubles
 __host__ __device__ constexpr double unit_cos(int N, int m) {
   constexpr double c30 = 0.86602540378443860;  // cos(pi/6)
@@ -93,7 +124,9 @@ __host__ __device__ constexpr double unit_cos(int N, int m) {
   constexpr double c9[9] = {1.0, 0.76604444311897801, 0.17364817766693036, -0.5,
                             -0.93969262078590843, -0.93969262078590843, -0.5,
                             0.17364817766693036, 0.76604444311897801};
-  return N == 9 ? c9[m % 9] : c12[(m * (12 / N)) % 12];
+  constexpr double c36 = 0.80901699437494742, c72 = 0.30901699437494742;
+  constexpr double c10[10] = {1.0, c36, c72, -c72, -c36, -1.0, -c36, -c72, c72, c36};
+  return N == 9 ? c9[m % 9] : (N == 10 ? c10[m % 10] : c12[(m * (12 / N)) % 12]);
 }
 
 __host__ __device__ constexpr double unit_sin(int N, int m) {
@@ -102,7 +135,9 @@ __host__ __device__ constexpr double unit_sin(int N, int m) {
   constexpr double s9[9] = {0.0, 0.64278760968653936, 0.98480775301220802, c30,
                             0.34202014332566871, -0.34202014332566871, -c30,
                             -0.98480775301220802, -0.64278760968653936};
-  return N == 9 ? s9[m % 9] : s12[(m * (12 / N)) % 12];
+  constexpr double s36 = 0.58778525229247313, s72 = 0.95105651629515357;
+  constexpr double s10[10] = {0.0, s36, s72, s72, s36, 0.0, -s36, -s72, -s72, -s36};
+  return N == 9 ? s9[m % 9] : (N == 10 ? s10[m % 10] : s12[(m * (12 / N)) % 12]);
 }
 
 // Radix P*Q butterfly on registers by one Cooley-Tukey split: inputs
@@ -153,6 +188,11 @@ __device__ __forceinline__ void dft<6>(cplx *v, int sign) {
 template <>
 __device__ __forceinline__ void dft<9>(cplx *v, int sign) {
   dft_split<3, 3>(v, sign);
+}
+
+template <>
+__device__ __forceinline__ void dft<10>(cplx *v, int sign) {
+  dft_split<5, 2>(v, sign);
 }
 
 template <>

@@ -1,15 +1,25 @@
 // Plan-specialised register-resident pencil passes.
 //
-// Same algorithm as fft_reg.hip (first Stockham stage reads HBM into
-// registers, last stage writes registers to HBM, LDS only between stages),
-// but the radix sequence is a template parameter, so every stage's span,
+// The first Stockham stage reads HBM into registers, the last stage writes
+// registers to HBM, and LDS only exchanges data between stages, in place.  The
+// radix sequence is a template parameter, so every stage's span,
 // butterfly count and twiddle stride are compile-time constants and a kernel
 // holds only the registers its own radices need.  The Hpsi epilogue loads
 // the psi and V values of the elements a thread will write before the FFT
 // stages start, so their latency overlaps the transform.
 //
-// Instantiated for the grid lengths of the workloads (24 ... 96) and a few
-// small test sizes; other lengths use the runtime-plan kernels.
+// A workgroup takes PLAN_B consecutive columns of the pass, a column being one
+// (pencil, band) pair numbered pencil * nst + band: band counts that are no
+// multiple of the tile leave no idle lanes, and where the rows are compact
+// (ld = nst) a tile's accesses along x and y are whole aligned 256-byte runs
+// whatever the band count.  Bound by HBM: six passes of 230 MB at 45 x 54 x 80
+// x 37 bands take 253 us (5.4 TB/s, where a copy reaches 5.7), against 454 with
+// run-time plans for 45 and 54 and tiles of 16 bands (37 of 48 lanes) along
+// every axis; 64^3 x 128 1239 -> 1222 us, and one field of 64^3 (nst = 1, 15 of
+// 16 lanes idle before) 381 -> 237 us for its Hartree and PBE potentials.
+//
+// Instantiated for the lengths that factor into the butterflies below up to
+// 128; other lengths go to fft_dense.hip and fft.hip.
 
 #include "fft.hpp"
 #include "fft_dft.hpp"
@@ -17,30 +27,35 @@
 
 namespace inqamd {
 
-template <int B, int MODE, int R0, int R1, int R2>
-__global__ __launch_bounds__(plan_threads(R0 * R1 * R2, B)) void fft_plan_kernel(
+constexpr int PLAN_B = 16;
+
+template <int MODE, int R0, int R1, int R2>
+__global__ __launch_bounds__(plan_threads(R0 * R1 * R2, PLAN_B)) void fft_plan_kernel(
     const fft_pass_args a) {
   using P = plan3<R0, R1, R2>;
+  constexpr int B = PLAN_B;
   constexpr int LEN = P::LEN;
   constexpr int NT = plan_threads(LEN, B);
   constexpr int RL = P::NSTAGE == 1 ? R0 : (P::NSTAGE == 2 ? R1 : R2);  // last radix
   constexpr int NBL = LEN / RL;
   constexpr int NBFL = (NBL * B + NT - 1) / NT;
+  static_assert(NT % B == 0, "a thread works on one column");
   __shared__ cplx lds[LEN * B];
 
-  const int nbt = (a.nst + B - 1) / B;
-  long t = blockIdx.x;
-  const int bt = (int)(t % nbt);
-  t /= nbt;
-  const int o1 = (int)(t % a.c1);
-  const int o2 = (int)(t / a.c1);
+  // this thread's column; one past the last loads column 0 and stores nothing
+  const unsigned ncol = (unsigned)a.nst * (unsigned)a.c1 * (unsigned)a.c2;
+  const unsigned g = blockIdx.x * B + threadIdx.x % B;
+  const bool ok = g < ncol;
+  const unsigned q = (ok ? g : 0) / (unsigned)a.nst;
+  const int b = (int)((ok ? g : 0) - q * (unsigned)a.nst);
+  const int o2 = (int)(q / (unsigned)a.c1);
+  const int o1 = (int)(q - (unsigned)o2 * (unsigned)a.c1);
   const long base = o1 * a.s1 + o2 * a.s2;
-  const int b0 = bt * B;
+  const cplx *in = a.in + base * a.in_ld + b;
+  cplx *out = a.out + base * a.out_ld + b;
+  const long istep = a.stride * a.in_ld, ostep = a.stride * a.out_ld;
 
-  auto gl = [&](int i, int bb) -> cplx {
-    const int b = b0 + bb;
-    return b < a.nst ? a.in[(base + (long)i * a.stride) * a.in_ld + b] : mk(0.0, 0.0);
-  };
+  auto gl = [&](int i, int) -> cplx { return in[i * istep]; };
   auto ll = [&](int i, int bb) -> cplx { return lds[i * B + bb]; };
   auto ls = [&](int i, int bb, cplx v, int, int) { lds[i * B + bb] = v; };
 
@@ -48,40 +63,30 @@ __global__ __launch_bounds__(plan_threads(R0 * R1 * R2, B)) void fft_plan_kernel
     // prefetch V psi for the outputs of the last stage: thread element
     // (q, r) is pencil point j + r*NBL with j = w / B (span NBL = LEN/RL)
     cplx pre[NBFL][RL];
+    const cplx *psi = a.psi + base * a.psi_ld + b;
+    const double *V = a.V + base;
 #pragma unroll
     for (int q = 0; q < NBFL; q++) {
       const int w = threadIdx.x + q * NT;
-      const int j = w / B, bb = w % B, b = b0 + bb;
+      const int j = w / B;
 #pragma unroll
       for (int r = 0; r < RL; r++) {
         pre[q][r] = mk(0.0, 0.0);
-        if ((NBFL * NT == NBL * B || w < NBL * B) && b < a.nst) {
-          const long p = base + (long)(j + r * NBL) * a.stride;
-          const cplx ps = a.psi[p * a.psi_ld + b];
-          const double vp = a.V[p];
-          pre[q][r] = mk(vp * ps.x, vp * ps.y);
+        if (NBFL * NT == NBL * B || w < NBL * B) {
+          const long p = (long)(j + r * NBL) * a.stride;
+          pre[q][r] = cscale(V[p], psi[p * a.psi_ld]);
         }
       }
     }
     // the last stage stores butterfly slot (q, r) at pencil point j + r*NBL,
     // the point whose V psi was prefetched into pre[q][r]
-    auto gs = [&](int i, int bb, cplx v, int q, int r) {
-      const int b = b0 + bb;
-      const cplx add = pre[q][r];
-      if (b >= a.nst) return;
-      const long p = base + (long)i * a.stride;
-      v = cscale(a.scale, v);
-      v.x += add.x;
-      v.y += add.y;
-      a.out[p * a.out_ld + b] = v;
+    auto gs = [&](int i, int, cplx v, int q, int r) {
+      if (ok) out[i * ostep] = cadd(cscale(a.scale, v), pre[q][r]);
     };
     run_plan<P, R0, R1, R2, B, NT>(a.tw, a.sign, false, gl, ll, ls, gs, false);
   } else {
-    auto gs = [&](int i, int bb, cplx v, int, int) {
-      const int b = b0 + bb;
-      if (b >= a.nst) return;
-      const long p = base + (long)i * a.stride;
-      a.out[p * a.out_ld + b] = cscale(a.scale, v);
+    auto gs = [&](int i, int, cplx v, int, int) {
+      if (ok) out[i * ostep] = cscale(a.scale, v);
     };
     if constexpr (MODE == FFT_KINETIC) {
       const double inv2pi = 0.15915494309189533576888376337251;
@@ -111,58 +116,80 @@ __global__ __launch_bounds__(plan_threads(R0 * R1 * R2, B)) void fft_plan_kernel
 // ---------------------------------------------------------------------------
 // host: (length -> radix sequence) table
 // ---------------------------------------------------------------------------
-template <int B, int MODE, int R0, int R1, int R2>
-static void plan_launch(const fft_pass_args &a, hipStream_t stream) {
-  constexpr int NT = plan_threads(R0 * R1 * R2, B);
-  const long nbt = (a.nst + B - 1) / B;
-  const long nblocks = nbt * a.c1 * a.c2;
-  hipLaunchKernelGGL((fft_plan_kernel<B, MODE, R0, R1, R2>), dim3((unsigned)nblocks), dim3(NT), 0,
-                     stream, a);
+template <int MODE, int R0, int R1, int R2>
+static void plan_launch(const fft_pass_args &a, unsigned nblocks, hipStream_t stream) {
+  constexpr int NT = plan_threads(R0 * R1 * R2, PLAN_B);
+  hipLaunchKernelGGL((fft_plan_kernel<MODE, R0, R1, R2>), dim3(nblocks), dim3(NT), 0, stream, a);
   INQAMD_HIP_CHECK(hipGetLastError());
 }
 
+// Two stages wherever two butterflies of at most 12 reach the length: every
+// further stage is an LDS round trip and two barriers
 #define INQAMD_PLAN_TABLE(X) \
   X(8, 8, 1, 1)              \
+  X(9, 3, 3, 1)              \
+  X(10, 5, 2, 1)             \
   X(12, 4, 3, 1)             \
+  X(14, 7, 2, 1)             \
+  X(15, 5, 3, 1)             \
   X(16, 4, 4, 1)             \
-  X(20, 4, 5, 1)             \
-  X(24, 8, 3, 1)             \
-  X(30, 2, 3, 5)             \
+  X(18, 6, 3, 1)             \
+  X(20, 5, 4, 1)             \
+  X(21, 7, 3, 1)             \
+  X(24, 6, 4, 1)             \
+  X(25, 5, 5, 1)             \
+  X(27, 9, 3, 1)             \
+  X(28, 7, 4, 1)             \
+  X(30, 6, 5, 1)             \
   X(32, 8, 4, 1)             \
-  X(36, 4, 3, 3)             \
+  X(35, 7, 5, 1)             \
+  X(36, 6, 6, 1)             \
   X(40, 8, 5, 1)             \
-  X(48, 8, 2, 3)             \
-  X(60, 4, 3, 5)             \
+  X(42, 7, 6, 1)             \
+  X(45, 9, 5, 1)             \
+  X(48, 8, 6, 1)             \
+  X(49, 7, 7, 1)             \
+  X(50, 10, 5, 1)            \
+  X(54, 9, 6, 1)             \
+  X(56, 8, 7, 1)             \
+  X(60, 10, 6, 1)            \
+  X(63, 9, 7, 1)             \
   X(64, 8, 8, 1)             \
-  X(72, 8, 3, 3)             \
-  X(80, 8, 2, 5)             \
-  X(96, 8, 4, 3)
+  X(70, 10, 7, 1)            \
+  X(72, 9, 8, 1)             \
+  X(75, 5, 5, 3)             \
+  X(80, 10, 8, 1)            \
+  X(81, 9, 9, 1)             \
+  X(84, 12, 7, 1)            \
+  X(90, 10, 9, 1)            \
+  X(96, 12, 8, 1)            \
+  X(100, 10, 10, 1)          \
+  X(108, 12, 9, 1)           \
+  X(112, 8, 7, 2)            \
+  X(120, 12, 10, 1)          \
+  X(125, 5, 5, 5)            \
+  X(126, 9, 7, 2)            \
+  X(128, 8, 4, 4)
 
-template <int B, int MODE>
-static bool plan_dispatch_b(const fft_pass_args &a, hipStream_t stream) {
+template <int MODE>
+static bool plan_dispatch(const fft_pass_args &a, unsigned nblocks, hipStream_t stream) {
   switch (a.len) {
 #define INQAMD_PLAN_CASE(L, R0, R1, R2) \
-  case L: plan_launch<B, MODE, R0, R1, R2>(a, stream); return true;
+  case L: plan_launch<MODE, R0, R1, R2>(a, nblocks, stream); return true;
     INQAMD_PLAN_TABLE(INQAMD_PLAN_CASE)
 #undef INQAMD_PLAN_CASE
     default: return false;
   }
 }
 
-template <int MODE>
-static bool plan_dispatch(const fft_pass_args &a, int B, hipStream_t stream) {
-  switch (B) {
-    case 16: return plan_dispatch_b<16, MODE>(a, stream);
-    case 8: return plan_dispatch_b<8, MODE>(a, stream);
-    default: return false;
-  }
-}
-
-bool fft_plan_launch(const fft_pass_args &a, int mode, int B, hipStream_t stream) {
+bool fft_plan_launch(const fft_pass_args &a, int mode, hipStream_t stream) {
+  const long ncol = (long)a.nst * a.c1 * a.c2;
+  if (ncol > (1L << 31) - PLAN_B) return false;  // columns are numbered in 32 bits
+  const unsigned nblocks = (unsigned)((ncol + PLAN_B - 1) / PLAN_B);
   switch (mode) {
-    case FFT_PLAIN: return plan_dispatch<FFT_PLAIN>(a, B, stream);
-    case FFT_KINETIC: return plan_dispatch<FFT_KINETIC>(a, B, stream);
-    case FFT_EPILOGUE: return plan_dispatch<FFT_EPILOGUE>(a, B, stream);
+    case FFT_PLAIN: return plan_dispatch<FFT_PLAIN>(a, nblocks, stream);
+    case FFT_KINETIC: return plan_dispatch<FFT_KINETIC>(a, nblocks, stream);
+    case FFT_EPILOGUE: return plan_dispatch<FFT_EPILOGUE>(a, nblocks, stream);
     default: return false;
   }
 }
