@@ -255,24 +255,8 @@ static void launch_mode(const fft_pass_args &a, int B, hipStream_t stream) {
     launch_gen<MODE, false>(a, B, stream);
 }
 
-// Tile shape of the register-resident pass: band tile 16 for wide band
-// sets, 8 below 16 bands.  INQAMD_FFT_VARIANT overrides the choice (tuning).
-static int reg_variant(const fft_pass_args &a) {
-  static int forced = [] {
-    const char *e = getenv("INQAMD_FFT_VARIANT");
-    return e ? atoi(e) : -1;
-  }();
-  if (forced >= 0) return forced;
-  return a.nst >= 16 ? 0 : 3;
-}
-
 void fft_launch_pass(const fft_pass_args &a, int mode, hipStream_t stream) {
-  const int v = reg_variant(a);
-  if (v < 10 && fft_plan_launch(a, mode, stream)) return;
-  if (fft_reg_supported(a)) {
-    fft_reg_launch(a, mode, v % 10, stream);
-    return;
-  }
+  if (fft_plan_launch(a, mode, stream) || fft_dense_launch(a, mode, stream)) return;
   const int B = fft_band_tile(a.nst, a.len);
   if (2L * a.len * B * (long)sizeof(cplx) > 65536)
     throw error{ERR_UNSUPPORTED, "FFT axis too long for the LDS pencil pass"};

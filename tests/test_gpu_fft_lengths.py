@@ -1,6 +1,8 @@
 """Pencil passes over every axis length and over ragged column counts against
-the CPU oracle: every length with a butterfly plan on every axis, in the
-transforms and in the kinetic and V psi passes of H psi.
+the CPU oracle: lengths with a butterfly plan, lengths that go through the DFT
+matrix (primes, prime multiples, the shortest and the longest of its range, one
+beyond it), each on every axis, in the transforms and in the kinetic and V psi
+passes of H psi.
 
 Tolerance 1e-12 relative 2-norm, as for the other transforms.
 """
@@ -45,3 +47,16 @@ def check(device, n, nst):
 def test_planned_length(device, length):
     check(device, (length, 5, length) if length < 64 else (3, 4, length), 3)
     check(device, (4, length, 3), 17)
+
+
+@pytest.mark.parametrize("length", [1, 2, 3, 4, 5, 6, 7, 11, 13, 17, 29, 31, 32 + 1, 37, 44, 47, 52,
+                                    62, 67, 94, 95, 97, 127, 131, 133, 190, 191])
+def test_dft_matrix_length(device, length):
+    check(device, (length, 5, length) if length < 48 else (3, 2, length), 3)
+    check(device, (3, length, 2), 16)
+    check(device, (length, 2, 3), 1)
+
+
+@pytest.mark.parametrize("length", [144, 160, 192, 194])
+def test_beyond_both(device, length):
+    check(device, (2, length, 3), 9)
