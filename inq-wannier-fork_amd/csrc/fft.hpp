@@ -79,6 +79,9 @@ bool fft_plan_launch(const fft_pass_args &a, int mode, hipStream_t stream);
 // takes; false for the others.
 bool fft_dense_launch(const fft_pass_args &a, int mode, hipStream_t stream);
 
+// Powers H^n psi that a Taylor chain keeps before one sweep adds them to its sums
+constexpr int TAYLOR_PENDING = 3;
+
 // Arguments of the three-sweep local Hamiltonian (fft3.hip) on a band chunk
 // of a cubic L^3 grid.
 struct fft3_args {
@@ -114,14 +117,25 @@ struct fft3_args {
   const int *own_sph;     // [N] sphere of a point's first entry (0 where unowned)
   const double *ent_mat;  // [nent][4] projector values at the entry's point
   const cplx *phase_ent;  // [nent] e^{-i(k+A).r} of the call
-  // Taylor accumulations acc += c * hpsi (p == nullptr: unused), chunk-offset
+  // Taylor sums (acc1 == nullptr / acc2 == nullptr: unused), chunk-offset:
+  //   acc1 = src1 + sum_{j < npend} pc1[j] pend[j] + c1 hpsi, terms in this order
+  //   acc2 = acc2 + sum_{j < npend} pc2[j] pend[j] + c2 hpsi
+  // with src1 the old acc1 or the state that the sum starts from, and pend the
+  // earlier powers that no sum holds yet (each at its own points only, so hpsi
+  // may be written over pend[0])
   cplx *acc1;
   long acc1_ld;
+  const cplx *src1;
+  long src1_ld;
   double c1re, c1im;
-  int acc1_init;  // acc1 = psi + c1 * hpsi instead of acc1 += c1 * hpsi
   cplx *acc2;
   long acc2_ld;
   double c2re, c2im;
+  int npend;
+  const cplx *pend[TAYLOR_PENDING];
+  long pend_ld;
+  double pc1re[TAYLOR_PENDING], pc1im[TAYLOR_PENDING];
+  double pc2re[TAYLOR_PENDING], pc2im[TAYLOR_PENDING];
   // optional copy of psi's forward transform (before the kinetic factor),
   // band-major [nb][kz][kx][ky] like W, chunk-offset (nullptr: none)
   cplx *gdump;

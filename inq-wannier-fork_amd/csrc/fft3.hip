@@ -38,10 +38,12 @@ void xy_kin_kernel(const fft3_args a) {
 
 // TY: y values of a 64-column tile (8 or 16); a 32-column tile takes TY / 2
 // (the same bands per tile)
-constexpr int z_bwd_ty(int L, bool acc, int ty) { return z_bwd_cols(L, acc) == Z_COLS ? ty : ty / 2; }
+constexpr int z_bwd_ty(int L, bool taylor, int ty) {
+  return z_bwd_cols(L, taylor) == Z_COLS ? ty : ty / 2;
+}
 
-template <int R0, int R1, int R2, int TY, bool ACC, bool FWD = false>
-__global__ __launch_bounds__(z_bwd_threads(R0 * R1 * R2, ACC))
+template <int R0, int R1, int R2, int TY, bool ACC, bool FWD>
+__global__ __launch_bounds__(z_bwd_threads(R0 * R1 * R2, ACC || FWD))
 __attribute__((amdgpu_waves_per_eu(z_bwd_waves(R0 * R1 * R2))))
 void z_bwd_epi_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
@@ -49,20 +51,20 @@ void z_bwd_epi_kernel(const fft3_args a) {
   // the plain Hpsi's tiles dealt per XCD (64^3 x 256 Hpsi 1.495 -> 1.480
   // ms); the Taylor forms keep the natural order (their steps ran 1 % slower
   // dealt per XCD)
-  constexpr int TB = z_bwd_cols(L, ACC) / z_bwd_ty(L, ACC, TY);
-  const long t = ACC ? (long)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB);
-  z_bwd_epi_tile<R0, R1, R2, z_bwd_ty(L, ACC, TY), z_bwd_threads(L, ACC), ACC, false, FWD,
-                 z_bwd_cols(L, ACC)>(a, t, lds);
+  constexpr bool T = ACC || FWD;
+  constexpr int TB = z_bwd_cols(L, T) / z_bwd_ty(L, T, TY);
+  const long t = T ? (long)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB);
+  z_bwd_epi_tile<R0, R1, R2, z_bwd_ty(L, T, TY), z_bwd_threads(L, T), ACC, false, FWD,
+                 z_bwd_cols(L, T)>(a, t, lds);
 }
 
-// Launch shape of a z_bwd_epi variant (acc: the Taylor forms)
-template <int R0, int R1, int R2, int TY, bool ACC>
-struct z_bwd_shape {
-  static constexpr int L = R0 * R1 * R2, ZC = z_bwd_cols(L, ACC);
-  static long tiles(int nb) { return z_tiles<z_bwd_ty(L, ACC, TY), ZC>(L, nb); }
-  static constexpr size_t lds = z_bwd_lds(L, ZC);
-  static constexpr int threads = z_bwd_threads(L, ACC);
-};
+template <int R0, int R1, int R2, int TY, bool ACC, bool FWD>
+static void z_bwd_launch(const fft3_args &a, hipStream_t stream) {
+  constexpr int L = R0 * R1 * R2, ZC = z_bwd_cols(L, ACC || FWD);
+  const long tiles = z_tiles<z_bwd_ty(L, ACC || FWD, TY), ZC>(L, a.nb);
+  hipLaunchKernelGGL((z_bwd_epi_kernel<R0, R1, R2, TY, ACC, FWD>), dim3((unsigned)tiles),
+                     dim3(z_bwd_threads(L, ACC || FWD)), z_bwd_lds(L, ZC), stream, a);
+}
 
 // G-space Hpsi sweeps
 template <int R0, int R1, int R2, int TY>
@@ -127,10 +129,12 @@ static void prepare3() {
   ensure_lds(z_kin_kernel<R0, R1, R2, 8>, zl);
   ensure_lds(xy_fwd_kernel<R0, R1, R2, wide_threads(L)>, pl);
   const size_t zbp = z_bwd_lds(L, z_bwd_cols(L, false)), zba = z_bwd_lds(L, z_bwd_cols(L, true));
-  ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 8, false>, zbp);
-  ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 16, false>, zbp);
-  ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 8, true>, zba);
-  ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 16, true>, zba);
+  ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 8, false, false>, zbp);
+  ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 16, false, false>, zbp);
+  ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 8, true, false>, zba);
+  ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 16, true, false>, zba);
+  ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 8, false, true>, zba);
+  ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 16, false, true>, zba);
   ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 8, true, true>, zba);
   ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 16, true, true>, zba);
 }
@@ -154,17 +158,15 @@ static void launch3v(const fft3_args &a, hipStream_t stream, int sweep, bool fwd
     INQAMD_HIP_CHECK(hipGetLastError());
   }
   if (sweep < 0 || sweep == 2) {
-    using SA = z_bwd_shape<R0, R1, R2, TY, true>;
-    using SP = z_bwd_shape<R0, R1, R2, TY, false>;
-    if (fwd_next)
-      hipLaunchKernelGGL((z_bwd_epi_kernel<R0, R1, R2, TY, true, true>), dim3((unsigned)SA::tiles(a.nb)),
-                         dim3(SA::threads), SA::lds, stream, a);
-    else if (a.acc1 || a.acc2)
-      hipLaunchKernelGGL((z_bwd_epi_kernel<R0, R1, R2, TY, true>), dim3((unsigned)SA::tiles(a.nb)),
-                         dim3(SA::threads), SA::lds, stream, a);
+    const bool acc = a.acc1 != nullptr;
+    if (fwd_next && acc)
+      z_bwd_launch<R0, R1, R2, TY, true, true>(a, stream);
+    else if (fwd_next)
+      z_bwd_launch<R0, R1, R2, TY, false, true>(a, stream);
+    else if (acc)
+      z_bwd_launch<R0, R1, R2, TY, true, false>(a, stream);
     else
-      hipLaunchKernelGGL((z_bwd_epi_kernel<R0, R1, R2, TY, false>), dim3((unsigned)SP::tiles(a.nb)),
-                         dim3(SP::threads), SP::lds, stream, a);
+      z_bwd_launch<R0, R1, R2, TY, false, false>(a, stream);
     INQAMD_HIP_CHECK(hipGetLastError());
   }
 }

@@ -385,7 +385,7 @@ __device__ __forceinline__ void xy_fwd_plane(const fft3_args &a, long plane, cpl
 // ---------------------------------------------------------------------------
 // sweep 3: z backward, x 1/N + V psi, band-major W -> INQ layout
 // ---------------------------------------------------------------------------
-// ACC: the caller may pass Taylor accumulators (acc1/acc2); without it they
+// ACC: the caller passes Taylor sums (acc1, perhaps acc2); without it they
 // must be null and the epilogue is a plain store.
 // GS (G-space Hpsi): no z transform (the first sweep made it), only the
 // transposing write, whose epilogue adds 1/2 |G+k+A|^2 kin_in instead of
@@ -696,77 +696,89 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
       }
     }
   } else {
-    // The Taylor accumulators of G outputs are all loaded (an invalid output
-    // loads point 0, band gb0 and stores nothing), then the outputs and the
-    // updated accumulators are formed, then stored, each kind of store in a
-    // loop of its own: no store waits for a load behind it.
-    constexpr int G = NE <= 6 ? NE : (R0 >= 12 ? 2 : (NE + 1) / 2);
-    const cplx *s1 = a.acc1_init ? a.psi : a.acc1;
-    const long l1 = a.acc1_init ? a.ld : a.acc1_ld;
+    // The sums' sources and pending powers of G outputs are all loaded (an
+    // invalid output loads point 0, band gb0 and stores nothing), then the
+    // outputs and the sums are formed, then stored, each kind of store in a loop
+    // of its own: no store waits for a load behind it.  Two outputs are up to ten
+    // loads in flight and fit the registers beside pre[].
+    constexpr int G = 2;
+    const bool two = a.acc2 != nullptr;
+    const bool one_src = two && a.src1 == a.acc2 && a.src1_ld == a.acc2_ld;
 #pragma unroll
     for (int k0 = 0; k0 < NE; k0 += G) {
-      constexpr int GG = G;
-      cplx o1[GG], o2[GG], v[GG];
-      long pp[GG];
-      int cbk[GG];
-      bool ok[GG];
+      cplx o1[G], o2[G], v[G], pw[TAYLOR_PENDING][G];
+      long pp[G];
+      int cbk[G];
+      bool ok[G];
 #pragma unroll
-      for (int g = 0; g < GG; g++) {
+      for (int g = 0; g < G; g++) {
         const int e = threadIdx.x + (k0 + g) * NT;
         const int b = e % Z_TB, y = (e / Z_TB) % Z_TY, z = e / Z_COLS;
         ok[g] = k0 + g < NE && e < L * Z_COLS && y0 + y < L && cb0 + b < a.nb;
         pp[g] = ok[g] ? ((long)x * L + y0 + y) * L + z : 0;
         cbk[g] = gb0 + (ok[g] ? b : 0);
       }
-      if (a.acc1) {
 #pragma unroll
-        for (int g = 0; g < GG; g++) o1[g] = s1[pp[g] * l1 + cbk[g]];
-      }
-      if (a.acc2) {
+      for (int g = 0; g < G; g++) o1[g] = a.src1[pp[g] * a.src1_ld + cbk[g]];
+      if (two && !one_src) {
 #pragma unroll
-        for (int g = 0; g < GG; g++) o2[g] = a.acc2[pp[g] * a.acc2_ld + cbk[g]];
+        for (int g = 0; g < G; g++) o2[g] = a.acc2[pp[g] * a.acc2_ld + cbk[g]];
       }
 #pragma unroll
-      for (int g = 0; g < GG; g++) {
+      for (int j = 0; j < TAYLOR_PENDING; j++) {
+        if (j < a.npend) {
+#pragma unroll
+          for (int g = 0; g < G; g++) pw[j][g] = a.pend[j][pp[g] * a.pend_ld + cbk[g]];
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < G; g++) {
         const int e = threadIdx.x + (k0 + g) * NT;
         const int b = e % Z_TB, y = (e / Z_TB) % Z_TY, z = e / Z_COLS;
         v[g] = ok[g] ? result(k0 + g, b, y, z) : mk(0.0, 0.0);
       }
-      if (a.acc1) {
+      auto add = [](cplx &o, double cr, double ci, cplx t) {
+        o.x += cr * t.x - ci * t.y;
+        o.y += cr * t.y + ci * t.x;
+      };
+      if (one_src) {
 #pragma unroll
-        for (int g = 0; g < GG; g++) {
-          o1[g].x += a.c1re * v[g].x - a.c1im * v[g].y;
-          o1[g].y += a.c1re * v[g].y + a.c1im * v[g].x;
+        for (int g = 0; g < G; g++) o2[g] = o1[g];
+      }
+#pragma unroll
+      for (int j = 0; j < TAYLOR_PENDING; j++) {
+        if (j < a.npend) {
+#pragma unroll
+          for (int g = 0; g < G; g++) {
+            add(o1[g], a.pc1re[j], a.pc1im[j], pw[j][g]);
+            if (two) add(o2[g], a.pc2re[j], a.pc2im[j], pw[j][g]);
+          }
         }
       }
-      if (a.acc2) {
 #pragma unroll
-        for (int g = 0; g < GG; g++) {
-          o2[g].x += a.c2re * v[g].x - a.c2im * v[g].y;
-          o2[g].y += a.c2re * v[g].y + a.c2im * v[g].x;
-        }
+      for (int g = 0; g < G; g++) {
+        add(o1[g], a.c1re, a.c1im, v[g]);
+        if (two) add(o2[g], a.c2re, a.c2im, v[g]);
       }
       if (!a.skip_store) {
 #pragma unroll
-        for (int g = 0; g < GG; g++)
+        for (int g = 0; g < G; g++)
           if (ok[g]) a.hpsi[pp[g] * a.hld + cbk[g]] = v[g];
       }
       if constexpr (FWD) {
 #pragma unroll
-        for (int g = 0; g < GG; g++) {
+        for (int g = 0; g < G; g++) {
           const int e = threadIdx.x + (k0 + g) * NT;
           const int b = e % Z_TB, y = (e / Z_TB) % Z_TY, z = e / Z_COLS;
           if (ok[g]) lds[z * Z_COLS + zswz(b * Z_TY + y)] = v[g];
         }
       }
-      if (a.acc1) {
 #pragma unroll
-        for (int g = 0; g < GG; g++)
-          if (ok[g]) a.acc1[pp[g] * a.acc1_ld + cbk[g]] = o1[g];
-      }
-      if (a.acc2) {
+      for (int g = 0; g < G; g++)
+        if (ok[g]) a.acc1[pp[g] * a.acc1_ld + cbk[g]] = o1[g];
+      if (two) {
 #pragma unroll
-        for (int g = 0; g < GG; g++)
+        for (int g = 0; g < G; g++)
           if (ok[g]) a.acc2[pp[g] * a.acc2_ld + cbk[g]] = o2[g];
       }
     }
@@ -823,8 +835,11 @@ constexpr int z_bwd_waves(int L) { return L == 72 ? 4 : z_bwd_min_waves(L); }
 // (acc) keep 64 columns: with 32 the 96^3 ETRS step ran 103 -> 113 ms (the
 // form that transforms its output forward writes W in 64-byte runs of 4 y)
 // and 103.4 -> 104.3 ms with only the last order's form at 32.
-constexpr int z_bwd_cols(int L, bool acc) { return L == 96 && !acc ? 32 : Z_COLS; }
-constexpr int z_bwd_threads(int L, bool acc) { return L == 96 && !acc ? Z_NT : z_threads(L); }
+// taylor: a form that adds to Taylor sums or transforms its output forward
+constexpr int z_bwd_cols(int L, bool taylor) { return L == 96 && !taylor ? 32 : Z_COLS; }
+constexpr int z_bwd_threads(int L, bool taylor) {
+  return L == 96 && !taylor ? Z_NT : z_threads(L);
+}
 
 // Grid lengths with three-sweep kernels: (L, radices of the plan)
 #define INQAMD_FFT3_TABLE(X) \

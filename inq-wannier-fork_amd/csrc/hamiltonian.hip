@@ -370,15 +370,25 @@ static void local_passes(handle &h, const cplx *psi, long ld, cplx *hpsi, long h
     if (acc && acc->p1) {
       a.acc1 = acc->p1 + b0;
       a.acc1_ld = acc->ld1;
+      a.src1 = (acc->src1 ? acc->src1 : acc->p1) + b0;
+      a.src1_ld = acc->src1 ? acc->lds1 : acc->ld1;
       a.c1re = acc->c1re;
       a.c1im = acc->c1im;
-      a.acc1_init = acc->init1 ? 1 : 0;
-    }
-    if (acc && acc->p2) {
-      a.acc2 = acc->p2 + b0;
-      a.acc2_ld = acc->ld2;
-      a.c2re = acc->c2re;
-      a.c2im = acc->c2im;
+      if (acc->p2) {
+        a.acc2 = acc->p2 + b0;
+        a.acc2_ld = acc->ld2;
+        a.c2re = acc->c2re;
+        a.c2im = acc->c2im;
+      }
+      a.npend = acc->npend;
+      a.pend_ld = acc->ldpend;
+      for (int j = 0; j < acc->npend; j++) {
+        a.pend[j] = acc->pend[j] + b0;
+        a.pc1re[j] = acc->pc1[j].real();
+        a.pc1im[j] = acc->pc1[j].imag();
+        a.pc2re[j] = acc->pc2[j].real();
+        a.pc2im[j] = acc->pc2[j].imag();
+      }
     }
     if (acc && acc->gdump) {
       if (gskip) throw error{ERR_UNSUPPORTED, "band-group chunks with a transform dump"};
@@ -544,7 +554,7 @@ void hamiltonian_apply(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld
   }
   if (!h.three_sweep) {
     projector_apply_coefficients(h, hpsi, hld, nst, slot);
-    if (acc && acc->p1 && acc->init1) copy(h, psi, ld, acc->p1, acc->ld1, nst);
+    if (acc && acc->p1 && acc->src1) copy(h, acc->src1, acc->lds1, acc->p1, acc->ld1, nst);
     if (acc && acc->p1) shift(h, {acc->c1re, acc->c1im}, hpsi, hld, acc->p1, acc->ld1, nst);
     if (acc && acc->p2) shift(h, {acc->c2re, acc->c2im}, hpsi, hld, acc->p2, acc->ld2, nst);
   }
@@ -606,15 +616,26 @@ void copy(handle &h, const cplx *x, long xld, cplx *y, long yld, int nst) {
 }
 
 // Taylor chains on three-sweep grids (exponential.hpp:21-69): for
-// n = 1..order, H^n psi = H (H^{n-1} psi) with acc1 += c1_n H^n psi (acc1 =
-// in + c1_1 H in when init1) and acc2 += c2_n H^n psi, c_n = z^n / n!.  Run
+// n = 1..order, H^n in = H (H^{n-1} in) with p1 += c1_n H^n in (p1 = in + c1_1
+// H in when init1) and p2 += c2_n H^n in, c_n = z^n / n!.  Run
 // band chunk by band chunk with every order of a chunk on one stream: the
-// projector takes the chunk's bands of H^{n-1} psi, and each order's last
+// projector takes the chunk's bands of H^{n-1} in, and each order's last
 // sweep also transforms its output forward in z into W for the next order,
-// so no z_fwd sweep reads H^n psi back (16 B per point and band per order);
-// the last order writes only the accumulators.  Chunks alternate between two
-// streams.  The same arithmetic as one Hpsi per order: results are equal bit
-// for bit.  Needs V_nl psi from coefficients (or no projectors);
+// so no z_fwd sweep reads H^n in back (16 B per point and band per order).
+// Chunks alternate between two streams.
+//
+// The sums are formed in one sweep out of every four: up to three powers wait
+// in buffers of their own (H^n in is written in any case) and the fourth
+// order's sweep reads them with the sums' old values and adds all four terms,
+// in the order of the recurrence.  Adding each power in its own sweep reads and
+// writes every sum in every order: a Taylor-4 sum moved 496 B per point and
+// band where this moves 448, and the 2-for-1 sum 608 where this moves 464 (HBM
+// bounds every sweep): the interacting step of 64^3 x 256 bands 23.70 -> 20.53
+// ms, the ETRS step of 48^3 x 64 1670 -> 1575 us.  The last order's power is
+// not written.
+//
+// The same arithmetic as one Hpsi per order: results are equal bit for bit.
+// Needs V_nl psi from coefficients (or no projectors);
 // INQAMD_TAYLOR_CHAIN=0 runs one Hpsi per order.
 bool taylor_chain_ok(const handle &h) {
   static const bool enabled = [] {
@@ -626,7 +647,7 @@ bool taylor_chain_ok(const handle &h) {
 }
 
 // outs[n - 1] (ld nst) receives H^n in when given (nullptr: the handle's
-// ping-pong buffers, and for the last order nothing); dumps[n - 1] receives
+// buffers, and for the last order nothing); dumps[n - 1] receives
 // the forward transform of order n's input (H^{n-1} in), band-major, as the
 // x-y sweep computes it (taylor_acc::gdump; contiguous band chunks then).
 void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int slot, cplx *p1,
@@ -654,29 +675,44 @@ void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int s
     INQAMD_HIP_CHECK(hipEventRecord(h.ev_fork, h.stream));
     INQAMD_HIP_CHECK(hipStreamWaitEvent(h.aux, h.ev_fork, 0));
   }
-  cplx *buf[2] = {h.hn, h.hn2};
+  // power n sits in buffer (n - 1) % 3: of the (at most three) powers pending at
+  // order n only the oldest shares its buffer, and the sweep reads that one at
+  // each point before it writes there
+  static_assert(TAYLOR_PENDING == 3, "one buffer per pending power");
+  cplx *buf[TAYLOR_PENDING] = {h.hn, h.hn2, h.hn3};
   for (int c = 0; c < plan.n; c++) {
     const int b0 = plan.b0(c), nb = plan.nb(c);
     hipStream_t s = two && (c & 1) ? h.aux : h.stream;
     cplx *W = two ? h.work + (size_t)(c & 1) * plan.chunk * h.npoint : h.work;
     const cplx *src = in + b0;
     long sld = ild;
+    int first = 1;  // first power that no sum holds yet
     for (int n = 1; n <= order; n++) {
-      cplx *dst = (outs && outs[n - 1] ? outs[n - 1] : buf[n & 1]) + b0;
+      auto power = [&](int m) { return outs && outs[m - 1] ? outs[m - 1] : buf[(m - 1) % 3]; };
+      cplx *dst = power(n) + b0;
       const bool keep = n < order || (outs && outs[n - 1]);
       if (proj)
         projector_project_p4_chunk(h, src, sld, nst, b0, nb, plan.gskip, plan.glog, s,
                                    two ? (c & 1) : 0);
       taylor_acc acc;
-      acc.p1 = p1;
-      acc.ld1 = ld1;
-      acc.c1re = c1[n - 1].real();
-      acc.c1im = c1[n - 1].imag();
-      acc.init1 = init1 && n == 1;
-      acc.p2 = p2;
-      acc.ld2 = ld2;
-      acc.c2re = c2[n - 1].real();
-      acc.c2im = c2[n - 1].imag();
+      if (n == order || n - first == TAYLOR_PENDING) {
+        acc.p1 = p1;
+        acc.ld1 = ld1;
+        if (init1 && first == 1) acc.src1 = in, acc.lds1 = ild;
+        acc.c1re = c1[n - 1].real();
+        acc.c1im = c1[n - 1].imag();
+        acc.p2 = p2;
+        acc.ld2 = ld2;
+        acc.c2re = c2[n - 1].real();
+        acc.c2im = c2[n - 1].imag();
+        acc.ldpend = nst;
+        for (; first < n; first++) {
+          acc.pend[acc.npend] = power(first);
+          acc.pc1[acc.npend] = c1[first - 1];
+          acc.pc2[acc.npend++] = c2[first - 1];
+        }
+        first = n + 1;
+      }
       acc.gdump = dumps ? dumps[n - 1] : nullptr;
       if (n == 1)
         local_passes(h, src, sld, dst, nst, nb, slot, b0, nst, &acc, 0, s, W, plan.gskip,
@@ -742,7 +778,7 @@ void exponential_from(handle &h, std::complex<double> z, int order, const cplx *
     acc.ld1 = old;
     acc.c1re = coeff.real();
     acc.c1im = coeff.imag();
-    acc.init1 = iter == 1;
+    if (iter == 1) acc.src1 = in, acc.lds1 = ild;
     if (iter == 1) {
       hamiltonian_apply(h, in, ild, hn, tl, nst, slot, &acc);
     } else {
@@ -773,7 +809,7 @@ void exponential_2_for_1(handle &h, std::complex<double> z1, std::complex<double
     acc.ld1 = eld;
     acc.c1re = c1.real();
     acc.c1im = c1.imag();
-    acc.init1 = iter == 1;
+    if (iter == 1) acc.src1 = phi, acc.lds1 = ld;
     acc.p2 = phi;
     acc.ld2 = ld;
     acc.c2re = c2.real();
@@ -865,12 +901,12 @@ static void release(handle &h) {
   for (int a = 0; a < 3; a++)
     if (h.axis[a].tw) (void)hipFree(h.axis[a].tw), h.axis[a].tw = nullptr;
   for (void *p : {(void *)h.V, (void *)h.kA, (void *)h.work, (void *)h.hn, (void *)h.hn2,
-                  (void *)h.proj, (void *)h.vnl, (void *)h.partial, (void *)h.mom_a,
+                  (void *)h.hn3, (void *)h.proj, (void *)h.vnl, (void *)h.partial, (void *)h.mom_a,
                   (void *)h.mom_b, (void *)h.obs, (void *)h.mom_partial, (void *)h.proj_part})
     if (p) (void)hipFree(p);
   h.V = nullptr;
   h.kA = nullptr;
-  h.work = h.hn = h.hn2 = h.proj = h.vnl = nullptr;
+  h.work = h.hn = h.hn2 = h.hn3 = h.proj = h.vnl = nullptr;
   h.partial = nullptr;
   h.mom_a = h.mom_b = nullptr;
   h.obs = nullptr;
@@ -972,6 +1008,7 @@ static void create(handle &h, const inqamd_system_desc &d, hipStream_t stream) {
   h.work = (cplx *)dalloc(orb);
   h.hn = (cplx *)dalloc(orb);
   h.hn2 = (cplx *)dalloc(orb);
+  if (h.three_sweep) h.hn3 = (cplx *)dalloc(orb);
   const long nchunk = (h.npoint + EN_CHUNK - 1) / EN_CHUNK;
   h.npartial = nchunk * h.max_bands * 2;
   h.partial = (double *)dalloc(h.npartial * sizeof(double));

@@ -72,15 +72,22 @@ struct project_expand_args {
 };
 
 // psi_acc += c * (H psi) accumulations fused into the Hpsi epilogue (Taylor
-// sums); p == nullptr disables a slot.
+// sums); p == nullptr disables a slot, and p2 needs p1.
 struct taylor_acc {
   cplx *p1 = nullptr;
   long ld1 = 0;
   double c1re = 0.0, c1im = 0.0;
-  bool init1 = false;  // p1 = psi + c1 hpsi (p1's old values unused)
+  const cplx *src1 = nullptr;  // p1 = src1 + ... (nullptr: p1's old values)
+  long lds1 = 0;
   cplx *p2 = nullptr;
   long ld2 = 0;
   double c2re = 0.0, c2im = 0.0;
+  // three-sweep Hpsi only: earlier powers added before hpsi (leading dimension
+  // ldpend) with their coefficients in either sum
+  int npend = 0;
+  const cplx *pend[TAYLOR_PENDING] = {};
+  long ldpend = 0;
+  std::complex<double> pc1[TAYLOR_PENDING], pc2[TAYLOR_PENDING];
   // three-sweep Hpsi only: the forward transform of psi, band-major
   // [nst][kz][kx][ky] (nullptr: not written)
   cplx *gdump = nullptr;
@@ -113,6 +120,7 @@ struct inqamd_hamiltonian {
   inqamd::cplx *work = nullptr; // [N][max_bands] FFT intermediate
   inqamd::cplx *hn = nullptr;   // [N][max_bands] Taylor H^n psi
   inqamd::cplx *hn2 = nullptr;  // [N][max_bands] Taylor ping-pong
+  inqamd::cplx *hn3 = nullptr;  // [N][max_bands] third power of a Taylor chain (three-sweep)
   inqamd::cplx *proj = nullptr; // [nproj][max_nlm][max_bands]
   inqamd::cplx *vnl = nullptr;  // [nent][max_bands] V_nl psi per ownership entry
   double *partial = nullptr;    // reduction partials

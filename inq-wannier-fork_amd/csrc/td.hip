@@ -882,7 +882,7 @@ void replay_half(inqamd_td *td, cplx *cur, int nb, cplx *const *Y, cplx *next, i
     acc.ld1 = nb;
     acc.c1re = coeff.real();
     acc.c1im = coeff.imag();
-    acc.init1 = it == 1;
+    if (it == 1) acc.src1 = Y[0], acc.lds1 = nb;
     if (td->fused) acc.gdump = Y[order + it - 1];  // transform of Y_{it-1}
     cplx *out = it < order ? Y[it] : td->hk[0];
     hamiltonian_apply(h, Y[it - 1], nb, out, nb, nb, slot, &acc);
@@ -917,7 +917,7 @@ void adjoint_half_fused(inqamd_td *td, int nb, cplx *const *Y, int slot, double 
       taylor_acc acc;
       acc.p1 = td->lam_in;
       acc.ld1 = nb;
-      acc.init1 = k == 1;
+      if (k == 1) acc.src1 = td->lam, acc.lds1 = nb;
       acc.c1re = ck.real();
       acc.c1im = ck.imag();
       acc.gdump = td->Ah[k - 1];
