@@ -443,13 +443,13 @@ void batch_build(inqamd_batch *b, const void *const *psi, void *const *hpsi, con
   b->coefficients = true;
   for (int s = 0; s < nsys; s++) {
     const handle &h = *b->hs[s];
-    if (h.three_sweep && batch_supported_length(h.n[0]) && h.pt.nproj > 0 &&
+    if (h.three_sweep && !h.rect && batch_supported_length(h.n[0]) && h.pt.nproj > 0 &&
         h.pt.nunique > 0 && !vnl_from_coefficients(h))
       b->coefficients = false;
   }
   for (int s = 0; s < nsys; s++) {
     handle &h = *b->hs[s];
-    if (!h.three_sweep || !batch_supported_length(h.n[0])) {
+    if (!h.three_sweep || h.rect || !batch_supported_length(h.n[0])) {
       b->fallback.push_back(s);
       continue;
     }
@@ -763,7 +763,7 @@ int inqamd_batch_create(inqamd_hamiltonian_t const *handles, int nsys, void *str
     INQAMD_HIP_CHECK(hipDeviceGetAttribute(&b->cus, hipDeviceAttributeMultiprocessorCount, dev));
     size_t zmax = 0, zbmax = 0, xymax = 0;
     for (auto *h : b->hs)
-      if (h->three_sweep) {
+      if (h->three_sweep && !h->rect) {
         zmax = std::max(zmax, (size_t)h->n[0] * Z_COLS * sizeof(cplx));
         zbmax = std::max(zbmax, z_bwd_lds(h->n[0]));
         xymax = std::max(xymax, (size_t)h->n[0] * (h->n[0] + 1) * sizeof(cplx));

@@ -83,7 +83,7 @@ bool fft_dense_launch(const fft_pass_args &a, int mode, hipStream_t stream);
 constexpr int TAYLOR_PENDING = 3;
 
 // Arguments of the three-sweep local Hamiltonian (fft3.hip) on a band chunk
-// of a cubic L^3 grid.
+// of a cubic L^3 grid (or an nx x ny x nz one: fft3_rect.hpp).
 struct fft3_args {
   const cplx *psi;   // chunk's first band, INQ layout, leading dimension ld
   long ld;
@@ -98,8 +98,11 @@ struct fft3_args {
   const double *V;   // [N]
   const double *kA;  // device covariant k + A
   double rlat[9];
-  const cplx *tw;    // W_L^k table
+  const cplx *tw;    // W_L^k table (of the z axis)
   double scale;      // 1/N
+  // nx x ny x nz grids (fft3_rect.hpp): extents and tables of the other axes
+  int nx, ny;
+  const cplx *twx, *twy;
   // projector apply fused into the last sweep (own == nullptr: not fused):
   // hpsi(p, b) += sum_{j < cnt} Qe[e0 + j][b] with own[p] = (e0 << OWN_COUNT_BITS) | cnt
   // (own[p] = -1 where no sphere reaches)
@@ -166,5 +169,13 @@ void fft3_prepare(int L);
 // three sweeps (sweep < 0) or only sweep 0 (z forward), 1 (x-y) or 2 (z back).
 void fft3_local_hamiltonian(const fft3_args &a, int L, hipStream_t stream, int sweep = -1,
                             bool fwd_next = false);
+
+// The same sweeps on an n[0] x n[1] x n[2] grid (fft3_rect.hip): true when every
+// length has a plan there and the plane and the z tile fit in max_lds.
+bool fft3_rect_supported(const int n[3], size_t max_lds);
+void fft3_rect_prepare(const int n[3]);
+void fft3_rect_local_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream, int sweep,
+                                 bool fwd_next);
+void fft3_rect_fourier_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream);
 
 }  // namespace inqamd

@@ -1,0 +1,301 @@
+// x-y sweeps of the nx x ny x nz three-sweep Hpsi, and its launches (see
+// fft3_rect.hpp).
+//
+// A workgroup transforms one (band, z) plane W[b][z][.][.] of nx x ny in LDS
+// (rows padded to an odd count of 16-byte elements), like the cubic planes, but
+// the number of columns of each axis's transform is a run-time value: butterfly w
+// is butterfly w / C of column w % C, by a float reciprocal (exact: w < 2^14).
+// Workgroups of 128 to 1024 threads by the size of the plane, so that a thread
+// holds at most about 12 elements between a stage's loads and its stores.
+
+#include "fft3_rect.hpp"
+
+namespace inqamd {
+
+// Most elements of a plane for a workgroup of NT threads
+constexpr int rect_elements(int NT) {
+  return NT == 128 ? 1280 : (NT == 256 ? 2560 : (NT == 512 ? 6144 : 10240));
+}
+
+// Most columns beside an axis of length L
+constexpr int rect_columns(int L, int NT) {
+  return rect_elements(NT) / L < RECT_MAX_LEN ? rect_elements(NT) / L : RECT_MAX_LEN;
+}
+
+template <int R, int L, int NT>
+struct rect_regs {
+  static constexpr int NBF = (L / R * rect_columns(L, NT) + NT - 1) / NT;
+  cplx v[NBF][R];
+};
+
+// Columns of one axis's transform
+struct rect_cols {
+  int C;
+  float inv;
+  __device__ void split(int w, int &j, int &c) const {
+    j = (int)(((float)w + 0.5f) * inv);
+    c = w - j * C;
+  }
+};
+
+// Calls f(q, j, c) for each butterfly of this thread
+template <int R, int L, int NT, class F>
+__device__ __forceinline__ void rect_each(const rect_cols &k, F f) {
+#pragma unroll
+  for (int q = 0; q < rect_regs<R, L, NT>::NBF; q++) {
+    const int w = threadIdx.x + q * NT;
+    int j, c;
+    k.split(w, j, c);
+    if (j < L / R) f(q, j, c);
+  }
+}
+
+template <int R, int L, int NT, class LD>
+__device__ __forceinline__ void rect_load(rect_regs<R, L, NT> &in, const rect_cols &k, LD ld) {
+  rect_each<R, L, NT>(k, [&](int q, int j, int c) {
+#pragma unroll
+    for (int r = 0; r < R; r++) in.v[q][r] = ld(j + r * (L / R), c);
+  });
+}
+
+template <int R, int NS, int L, int NT>
+__device__ __forceinline__ void rect_compute(rect_regs<R, L, NT> &in, const rect_cols &k,
+                                             const cplx *__restrict__ tw, int sign) {
+  rect_each<R, L, NT>(k, [&](int q, int j, int) {
+    if constexpr (NS > 1) {
+      const int kk = j % NS;
+#pragma unroll
+      for (int r = 1; r < R; r++)
+        in.v[q][r] = cmul(in.v[q][r], twiddle(tw, r * kk * (L / (NS * R)), sign));
+    }
+    dft<R>(in.v[q], sign);
+  });
+}
+
+template <int R, int NS, int L, int NT, class ST>
+__device__ __forceinline__ void rect_store(rect_regs<R, L, NT> &in, const rect_cols &k, ST st) {
+  rect_each<R, L, NT>(k, [&](int q, int j, int c) {
+    const int base = (j / NS) * NS * R + j % NS;
+#pragma unroll
+    for (int r = 0; r < R; r++) st(base + r * NS, c, in.v[q][r]);
+  });
+}
+
+// One in-place LDS stage (between barriers)
+template <int R, int NS, int L, int NT, class LD, class ST>
+__device__ __forceinline__ void rect_stage(const rect_cols &k, const cplx *tw, int sign, LD ld,
+                                           ST st) {
+  rect_regs<R, L, NT> in;
+  rect_load<R, L, NT>(in, k, ld);
+  rect_compute<R, NS, L, NT>(in, k, tw, sign);
+  __syncthreads();
+  rect_store<R, NS, L, NT>(in, k, st);
+  __syncthreads();
+}
+
+// The stages of an axis from `first` (global or LDS) to `last` (LDS or global)
+// through ld / st in LDS; FROM_LDS, TO_LDS: whether the ends share the array
+template <int R0, int R1, int R2, int NT, bool FROM_LDS, bool TO_LDS, class FL, class LD, class ST,
+          class LS>
+__device__ __forceinline__ void rect_axis(const rect_cols &k, const cplx *tw, int sign, FL first,
+                                          LD ld, ST st, LS last) {
+  constexpr int L = R0 * R1 * R2;
+  static_assert(R1 > 1, "at least two stages");
+  {
+    rect_regs<R0, L, NT> in;
+    rect_load<R0, L, NT>(in, k, first);
+    rect_compute<R0, 1, L, NT>(in, k, tw, sign);
+    if (FROM_LDS) __syncthreads();
+    rect_store<R0, 1, L, NT>(in, k, st);
+    __syncthreads();
+  }
+  if constexpr (R2 > 1) rect_stage<R1, R0, L, NT>(k, tw, sign, ld, st);
+  constexpr int RL = R2 > 1 ? R2 : R1, NSL = L / RL;
+  rect_regs<RL, L, NT> in;
+  rect_load<RL, L, NT>(in, k, ld);
+  rect_compute<RL, NSL, L, NT>(in, k, tw, sign);
+  if (TO_LDS) __syncthreads();
+  rect_store<RL, NSL, L, NT>(in, k, last);
+  if (TO_LDS) __syncthreads();
+}
+
+// The y axis of the kinetic plane: forward, x 1/2 |G+k+A|^2 (and the copy of the
+// transform before it), inverse.  The forward's last stage holds in butterfly j
+// the outputs j + r L/RL, the inputs of the first stage of the inverse run with
+// the radices in reverse order, so that stage starts from the registers.
+template <int R0, int R1, int R2, int NT, class LD, class ST, class KIN>
+__device__ __forceinline__ void rect_y_kinetic(const rect_cols &k, const cplx *tw, LD ld, ST st,
+                                               KIN kin) {
+  constexpr int L = R0 * R1 * R2;
+  constexpr int RL = R2 > 1 ? R2 : R1, NSL = L / RL;
+  rect_stage<R0, 1, L, NT>(k, tw, -1, ld, st);
+  if constexpr (R2 > 1) rect_stage<R1, R0, L, NT>(k, tw, -1, ld, st);
+  {
+    rect_regs<RL, L, NT> in;
+    rect_load<RL, L, NT>(in, k, ld);
+    rect_compute<RL, NSL, L, NT>(in, k, tw, -1);
+    rect_each<RL, L, NT>(k, [&](int q, int j, int c) {
+#pragma unroll
+      for (int r = 0; r < RL; r++) in.v[q][r] = kin(j + r * NSL, c, in.v[q][r]);
+    });
+    rect_compute<RL, 1, L, NT>(in, k, tw, +1);
+    __syncthreads();
+    rect_store<RL, 1, L, NT>(in, k, st);
+    __syncthreads();
+  }
+  if constexpr (R2 > 1) rect_stage<R1, RL, L, NT>(k, tw, +1, ld, st);
+  rect_stage<R0, L / R0, L, NT>(k, tw, +1, ld, st);
+}
+
+// FWD: only the forward transforms, in place in W (G-space Hpsi)
+template <int NT, bool FWD>
+__global__ __launch_bounds__(NT) void rect_xy_kernel(const fft3_args a, int nz) {
+  extern __shared__ cplx lds[];
+  const int nx = a.nx, ny = a.ny, pad = ny | 1;
+  const long plane = blockIdx.x;  // band * nz + z
+  const int z = (int)(plane % nz);
+  cplx *W = a.W + plane * nx * ny;
+  const rect_cols kx = {ny, 1.0f / (float)ny}, ky = {nx, 1.0f / (float)nx};
+
+  // x axis: element (i = x, c = y); y axis: (i = y, c = x)
+  auto gx = [&](int i, int c) -> cplx { return W[i * ny + c]; };
+  auto wx = [&](int i, int c, cplx v) { W[i * ny + c] = v; };
+  auto lx = [&](int i, int c) -> cplx { return lds[i * pad + c]; };
+  auto sx = [&](int i, int c, cplx v) { lds[i * pad + c] = v; };
+  auto ly = [&](int i, int c) -> cplx { return lds[c * pad + i]; };
+  auto sy = [&](int i, int c, cplx v) { lds[c * pad + i] = v; };
+
+  switch (nx) {
+#define INQAMD_RECT_CASE(L, R0, R1, R2)                                                   \
+  case L:                                                                                \
+    rect_axis<R0, R1, R2, NT, false, true>(kx, a.twx, -1, gx, lx, sx, sx);               \
+    break;
+    INQAMD_RECT_XY(INQAMD_RECT_CASE)
+#undef INQAMD_RECT_CASE
+  }
+  if constexpr (FWD) {
+    auto wy = [&](int i, int c, cplx v) { W[c * ny + i] = v; };
+    switch (ny) {
+#define INQAMD_RECT_CASE(L, R0, R1, R2)                                                   \
+  case L:                                                                                \
+    rect_axis<R0, R1, R2, NT, true, false>(ky, a.twy, -1, ly, ly, sy, wy);               \
+    break;
+      INQAMD_RECT_XY(INQAMD_RECT_CASE)
+#undef INQAMD_RECT_CASE
+    }
+  } else {
+    // 1/2 |G + k + A|^2 with G = m_x b0 + m_y b1 + m_z b2 (cartesian)
+    double kc[3], gz[3], b0[3], b1[3];
+    xy_kc(a, kc);
+    const int mz = symmetric_index(z, nz);
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      gz[d] = mz * a.rlat[2 * 3 + d] + kc[d];
+      b0[d] = a.rlat[0 * 3 + d];
+      b1[d] = a.rlat[1 * 3 + d];
+    }
+    cplx *G = a.gdump ? a.gdump + plane * nx * ny : nullptr;
+    auto kin = [&](int i, int c, cplx v) -> cplx {
+      if (G) G[c * ny + i] = v;
+      const int my = symmetric_index(i, ny), mx = symmetric_index(c, nx);
+      const double q0 = mx * b0[0] + my * b1[0] + gz[0];
+      const double q1 = mx * b0[1] + my * b1[1] + gz[1];
+      const double q2 = mx * b0[2] + my * b1[2] + gz[2];
+      return cscale(0.5 * (q0 * q0 + q1 * q1 + q2 * q2), v);
+    };
+    switch (ny) {
+#define INQAMD_RECT_CASE(L, R0, R1, R2)                                                   \
+  case L: rect_y_kinetic<R0, R1, R2, NT>(ky, a.twy, ly, sy, kin); break;
+      INQAMD_RECT_XY(INQAMD_RECT_CASE)
+#undef INQAMD_RECT_CASE
+    }
+    switch (nx) {
+#define INQAMD_RECT_CASE(L, R0, R1, R2)                                                   \
+  case L:                                                                                \
+    rect_axis<R0, R1, R2, NT, true, false>(kx, a.twx, +1, lx, lx, sx, wx);               \
+    break;
+      INQAMD_RECT_XY(INQAMD_RECT_CASE)
+#undef INQAMD_RECT_CASE
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// host
+// ---------------------------------------------------------------------------
+static size_t rect_xy_lds(const int n[3]) { return (size_t)n[0] * (n[1] | 1) * sizeof(cplx); }
+
+template <int NT>
+static void rect_xy_prepare(size_t lds) {
+  if (lds <= 65536) return;
+  INQAMD_HIP_CHECK(hipFuncSetAttribute((const void *)rect_xy_kernel<NT, false>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
+  INQAMD_HIP_CHECK(hipFuncSetAttribute((const void *)rect_xy_kernel<NT, true>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
+}
+
+template <bool FWD>
+static void rect_xy_launch(const fft3_args &a, const int n[3], hipStream_t stream) {
+  const unsigned planes = (unsigned)((long)a.nb * n[2]);
+  const size_t lds = rect_xy_lds(n);
+  const int el = n[0] * n[1];
+  if (el <= rect_elements(128))
+    hipLaunchKernelGGL((rect_xy_kernel<128, FWD>), dim3(planes), dim3(128), lds, stream, a, n[2]);
+  else if (el <= rect_elements(256))
+    hipLaunchKernelGGL((rect_xy_kernel<256, FWD>), dim3(planes), dim3(256), lds, stream, a, n[2]);
+  else if (el <= rect_elements(512))
+    hipLaunchKernelGGL((rect_xy_kernel<512, FWD>), dim3(planes), dim3(512), lds, stream, a, n[2]);
+  else
+    hipLaunchKernelGGL((rect_xy_kernel<1024, FWD>), dim3(planes), dim3(1024), lds, stream, a,
+                       n[2]);
+  INQAMD_HIP_CHECK(hipGetLastError());
+}
+
+static bool rect_length(int L) {
+  switch (L) {
+#define INQAMD_RECT_CASE(LL, R0, R1, R2) case LL:
+    INQAMD_RECT_XY(INQAMD_RECT_CASE)
+#undef INQAMD_RECT_CASE
+      return true;
+    default: return false;
+  }
+}
+
+bool fft3_rect_supported(const int n[3], size_t max_lds) {
+  return rect_length(n[0]) && rect_length(n[1]) && rect_length(n[2]) &&
+         n[0] * n[1] <= rect_elements(1024) && rect_xy_lds(n) <= max_lds &&
+         z_bwd_lds(n[2]) <= max_lds;
+}
+
+static void rect_z(const fft3_args &a, int nz, rect_z_kernel k, hipStream_t stream) {
+  if (rect_z_launch_a(a, nz, k, stream) || rect_z_launch_b(a, nz, k, stream) ||
+      rect_z_launch_c(a, nz, k, stream))
+    return;
+  throw error{ERR_UNSUPPORTED, "three-sweep Hpsi: unsupported z length"};
+}
+
+void fft3_rect_prepare(const int n[3]) {
+  const size_t lds = rect_xy_lds(n);
+  rect_xy_prepare<512>(lds);
+  rect_xy_prepare<1024>(lds);
+  rect_z(fft3_args{}, n[2], RECT_Z_PREPARE, nullptr);
+}
+
+void fft3_rect_local_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream, int sweep,
+                                 bool fwd_next) {
+  if (sweep < 0 || sweep == 0) rect_z(a, n[2], RECT_Z_FWD, stream);
+  if (sweep < 0 || sweep == 1) rect_xy_launch<false>(a, n, stream);
+  if (sweep < 0 || sweep == 2)
+    rect_z(a, n[2],
+           a.acc1 ? (fwd_next ? RECT_Z_BWD_ACC_FWD : RECT_Z_BWD_ACC)
+                  : (fwd_next ? RECT_Z_BWD_FWD : RECT_Z_BWD),
+           stream);
+}
+
+void fft3_rect_fourier_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream) {
+  rect_z(a, n[2], RECT_Z_POT, stream);
+  rect_xy_launch<true>(a, n, stream);
+  rect_z(a, n[2], RECT_Z_KIN, stream);
+}
+
+}  // namespace inqamd

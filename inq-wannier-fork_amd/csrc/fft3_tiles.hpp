@@ -1,6 +1,7 @@
 // Tile bodies of the three-sweep local Hpsi (T + V) for cubic grids L^3,
 // shared by the one-system kernels (fft3.hip) and the uneven-batch
-// work-queue kernels (batch.hip).
+// work-queue kernels (batch.hip); the z tiles also for nx x ny x L grids (RECT,
+// fft3_rect.hpp: the x and y extents from the arguments).
 //
 //   z_fwd_tile     psi [x][y][z][band] (INQ layout) -> W[band][z][x][y]
 //                  tile: one x, TY y, TB = 64/TY bands, all z.  The first
@@ -55,14 +56,16 @@ constexpr int plane_threads(int L) {
 // ---------------------------------------------------------------------------
 // POT: the tile transforms V psi + V_nl psi (ownership entries Qe) instead
 // of psi, formed as the first stage loads psi.
-template <int R0, int R1, int R2, int Z_TY, int NT = Z_NT, bool POT = false>
+template <int R0, int R1, int R2, int Z_TY, int NT = Z_NT, bool POT = false,
+          bool RECT = false>
 __device__ __forceinline__ void z_fwd_tile(const fft3_args &a, long t, cplx *lds) {
   using P = plan3<R0, R1, R2>;
   constexpr int L = P::LEN;
   constexpr int Z_TB = Z_COLS / Z_TY;
+  const int NX = RECT ? a.nx : L, NY = RECT ? a.ny : L;
   // lds: [L][Z_COLS], column = b * Z_TY + y
 
-  const int nyt = (L + Z_TY - 1) / Z_TY;
+  const int nyt = (NY + Z_TY - 1) / Z_TY;
   const int nbt = (a.nb + Z_TB - 1) / Z_TB;
   const int bt = (int)(t % nbt);
   t /= nbt;
@@ -76,8 +79,8 @@ __device__ __forceinline__ void z_fwd_tile(const fft3_args &a, long t, cplx *lds
   // of TB * 16 contiguous bytes, each used whole.
   auto gl = [&](int i, int c) -> cplx {
     const int b = c / Z_TY, y = c % Z_TY;
-    if (!(y0 + y < L && cb0 + b < a.nb)) return mk(0.0, 0.0);
-    const long p = ((long)x * L + y0 + y) * L + i;
+    if (!(y0 + y < NY && cb0 + b < a.nb)) return mk(0.0, 0.0);
+    const long p = ((long)x * NY + y0 + y) * L + i;
     cplx v = a.psi[p * a.ld + gb0 + b];
     if constexpr (POT) {
       const double vp = a.V[p];
@@ -95,8 +98,8 @@ __device__ __forceinline__ void z_fwd_tile(const fft3_args &a, long t, cplx *lds
   auto ls = [&](int i, int c, cplx v, int, int) { lds[i * Z_COLS + zswz(c)] = v; };
   auto gs = [&](int i, int c, cplx v, int, int) {
     const int b = c / Z_TY, y = c % Z_TY;
-    if (y0 + y < L && cb0 + b < a.nb)
-      a.W[(((long)(cb0 + b) * L + i) * L + x) * L + y0 + y] = v;
+    if (y0 + y < NY && cb0 + b < a.nb)
+      a.W[(((long)(cb0 + b) * L + i) * NX + x) * NY + y0 + y] = v;
   };
   run_plan<P, R0, R1, R2, Z_COLS, NT>(a.tw, -1, false, gl, ll, ls, gs, false);
 }
@@ -503,19 +506,20 @@ __device__ __forceinline__ void vnl_expand_wave(const fft3_args &a, int gb0, con
 
 // ZC: columns of the tile (TY y values x ZC / TY bands), 64 or 32
 template <int R0, int R1, int R2, int Z_TY, int NT = Z_NT, bool ACC = false, bool GS = false,
-          bool FWD = false, int ZC = Z_COLS>
+          bool FWD = false, int ZC = Z_COLS, bool RECT = false>
 __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx *lds) {
   using P = plan3<R0, R1, R2>;
   constexpr int L = P::LEN;
   constexpr int Z_COLS = ZC;  // (shadows the namespace constant in this tile)
   constexpr int Z_TB = Z_COLS / Z_TY;
+  const int NX = RECT ? a.nx : L, NY = RECT ? a.ny : L;
   constexpr int RPI = 64 / Z_COLS;  // tile rows one wave's 16-byte DMA fills
   static_assert(L % RPI == 0, "whole rows per DMA instruction");
   auto zswz = [](int c) { return zswz_n<ZC>(c); };
   static_assert(NT % Z_TB == 0, "thread -> band mapping of the epilogue");
   constexpr int NE = (L * Z_COLS + NT - 1) / NT;  // output elements per thread
 
-  const int nyt = (L + Z_TY - 1) / Z_TY;
+  const int nyt = (NY + Z_TY - 1) / Z_TY;
   const int nbt = (a.nb + Z_TB - 1) / Z_TB;
   const int bt = (int)(t % nbt);
   t /= nbt;
@@ -537,9 +541,9 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lr = lane / Z_COLS, c = zswz(lane % Z_COLS);
     const int b = c / Z_TY, y = c % Z_TY;
-    const bool ok = y0 + y < L && cb0 + b < a.nb;
-    const long col = ok ? (((long)(cb0 + b) * L) * L + x) * L + y0 + y : 0;
-    const long row = ok ? (long)L * L : 0;
+    const bool ok = y0 + y < NY && cb0 + b < a.nb;
+    const long col = ok ? (((long)(cb0 + b) * L) * NX + x) * NY + y0 + y : 0;
+    const long row = ok ? (long)NX * NY : 0;
     for (int i = wave * RPI; i < L; i += (NT / 64) * RPI)
       __builtin_amdgcn_global_load_lds(a.W + col + (i + lr) * row, lds + i * Z_COLS, 16, 0, 0);
     if (64 * wave < L && 64 * wave + lane < L)
@@ -561,14 +565,14 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
   for (int k = 0; k < NE; k++) {
     const int e = threadIdx.x + k * NT;
     const int b = e % Z_TB, y = (e / Z_TB) % Z_TY, z = e / Z_COLS;
-    vk[k] = e < L * Z_COLS && y0 + y < L && cb0 + b < a.nb;
-    pk[k] = vk[k] ? (x * L + y0 + y) * L + z : 0;
+    vk[k] = e < L * Z_COLS && y0 + y < NY && cb0 + b < a.nb;
+    pk[k] = vk[k] ? (x * NY + y0 + y) * L + z : 0;
     bk[k] = gb0 + (vk[k] ? b : 0);
   }
   if constexpr (GS) {
     double kc[3], gx[3];
     xy_kc(a, kc);
-    const int mx = symmetric_index(x, L);
+    const int mx = symmetric_index(x, NX);
 #pragma unroll
     for (int d = 0; d < 3; d++) gx[d] = mx * a.rlat[0 * 3 + d] + kc[d];
     cplx kin[NE];
@@ -578,7 +582,7 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
     for (int k = 0; k < NE; k++) {
       const int e = threadIdx.x + k * NT;
       const int y = (e / Z_TB) % Z_TY, z = e / Z_COLS;
-      const int my = symmetric_index(y0 + y, L), mz = symmetric_index(z, L);
+      const int my = symmetric_index(y0 + y, NY), mz = symmetric_index(z, L);
       const double q0 = gx[0] + my * a.rlat[3] + mz * a.rlat[6];
       const double q1 = gx[1] + my * a.rlat[4] + mz * a.rlat[7];
       const double q2 = gx[2] + my * a.rlat[5] + mz * a.rlat[8];
@@ -618,7 +622,7 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
 
   auto gl = [&](int i, int c) -> cplx {
     const int b = c / Z_TY, y = c % Z_TY;
-    return (y0 + y < L && cb0 + b < a.nb) ? a.W[(((long)(cb0 + b) * L + i) * L + x) * L + y0 + y]
+    return (y0 + y < NY && cb0 + b < a.nb) ? a.W[(((long)(cb0 + b) * L + i) * NX + x) * NY + y0 + y]
                                           : mk(0.0, 0.0);
   };
   auto ll = [&](int i, int c) -> cplx { return lds[i * Z_COLS + zswz(c)]; };
@@ -651,8 +655,8 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
       for (int k = 0; k < NE; k++) {
         const int e = threadIdx.x + k * NT;
         const int b = e % Z_TB, y = (e / Z_TB) % Z_TY, z = e / Z_COLS;
-        own[k] = e < L * Z_COLS && y0 + y < L && cb0 + b < a.nb
-                     ? a.own[((long)x * L + y0 + y) * L + z]
+        own[k] = e < L * Z_COLS && y0 + y < NY && cb0 + b < a.nb
+                     ? a.own[((long)x * NY + y0 + y) * L + z]
                      : -1;
       }
       cplx q[NE];
@@ -689,9 +693,9 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
     for (int k = 0; k < NE; k++) {
       const int e = threadIdx.x + k * NT;
       const int b = e % Z_TB, y = (e / Z_TB) % Z_TY, z = e / Z_COLS;
-      if (e < L * Z_COLS && y0 + y < L && cb0 + b < a.nb) {
+      if (e < L * Z_COLS && y0 + y < NY && cb0 + b < a.nb) {
         const cplx v = result(k, b, y, z);
-        if (!a.skip_store) a.hpsi[(((long)x * L + y0 + y) * L + z) * a.hld + gb0 + b] = v;
+        if (!a.skip_store) a.hpsi[(((long)x * NY + y0 + y) * L + z) * a.hld + gb0 + b] = v;
         if constexpr (FWD) lds[z * Z_COLS + zswz(b * Z_TY + y)] = v;
       }
     }
@@ -714,8 +718,8 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
       for (int g = 0; g < G; g++) {
         const int e = threadIdx.x + (k0 + g) * NT;
         const int b = e % Z_TB, y = (e / Z_TB) % Z_TY, z = e / Z_COLS;
-        ok[g] = k0 + g < NE && e < L * Z_COLS && y0 + y < L && cb0 + b < a.nb;
-        pp[g] = ok[g] ? ((long)x * L + y0 + y) * L + z : 0;
+        ok[g] = k0 + g < NE && e < L * Z_COLS && y0 + y < NY && cb0 + b < a.nb;
+        pp[g] = ok[g] ? ((long)x * NY + y0 + y) * L + z : 0;
         cbk[g] = gb0 + (ok[g] ? b : 0);
       }
 #pragma unroll
@@ -788,8 +792,8 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
     __syncthreads();
     auto gs = [&](int i, int c, cplx v, int, int) {
       const int b = c / Z_TY, y = c % Z_TY;
-      if (y0 + y < L && cb0 + b < a.nb)
-        a.W[(((long)(cb0 + b) * L + i) * L + x) * L + y0 + y] = v;
+      if (y0 + y < NY && cb0 + b < a.nb)
+        a.W[(((long)(cb0 + b) * L + i) * NX + x) * NY + y0 + y] = v;
     };
     run_plan<P, R0, R1, R2, Z_COLS, NT>(ltw, -1, true, ll, ll, ls, gs, false);
   }
@@ -825,7 +829,7 @@ constexpr int z_bwd_min_waves(int L) { return L == 72 ? 1 : 4; }
 // outputs per thread) and so held a CU alone with 8 waves, while at 768 it
 // takes 124 and 12 waves share the CU (z_bwd_epi 0.58 vs 0.66 ms at
 // 72^3 x 128).
-constexpr int z_threads(int L) { return L >= 80 ? 1024 : (L == 72 ? 768 : Z_NT); }
+constexpr int z_threads(int L) { return L >= 80 ? 1024 : (L >= 70 ? 768 : Z_NT); }
 constexpr int z_bwd_waves(int L) { return L == 72 ? 4 : z_bwd_min_waves(L); }
 
 // Columns and threads of the one-system z_bwd_epi tiles: 32 columns of 512
@@ -836,9 +840,9 @@ constexpr int z_bwd_waves(int L) { return L == 72 ? 4 : z_bwd_min_waves(L); }
 // form that transforms its output forward writes W in 64-byte runs of 4 y)
 // and 103.4 -> 104.3 ms with only the last order's form at 32.
 // taylor: a form that adds to Taylor sums or transforms its output forward
-constexpr int z_bwd_cols(int L, bool taylor) { return L == 96 && !taylor ? 32 : Z_COLS; }
+constexpr int z_bwd_cols(int L, bool taylor) { return L >= 84 && !taylor ? 32 : Z_COLS; }
 constexpr int z_bwd_threads(int L, bool taylor) {
-  return L == 96 && !taylor ? Z_NT : z_threads(L);
+  return z_bwd_cols(L, taylor) == 32 ? Z_NT : z_threads(L);
 }
 
 // Grid lengths with three-sweep kernels: (L, radices of the plan)

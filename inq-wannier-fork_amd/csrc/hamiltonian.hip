@@ -350,7 +350,11 @@ static void local_passes(handle &h, const cplx *psi, long ld, cplx *hpsi, long h
     a.V = h.V;
     a.kA = h.kA + 3 * slot;
     for (int d = 0; d < 9; d++) a.rlat[d] = h.rlat[d];
-    a.tw = h.axis[0].tw;
+    a.tw = h.axis[2].tw;
+    a.nx = h.n[0];
+    a.ny = h.n[1];
+    a.twx = h.axis[0].tw;
+    a.twy = h.axis[1].tw;
     a.scale = 1.0 / (double)h.npoint;
     const projector_tables &t = h.pt;
     if (vnl_from_coefficients(h)) {
@@ -397,7 +401,10 @@ static void local_passes(handle &h, const cplx *psi, long ld, cplx *hpsi, long h
     a.skip_store = skip_store ? 1 : 0;
     a.z_ty = h.tune_z_ty;
     a.xy_wide = h.tune_xy_wide;
-    fft3_local_hamiltonian(a, h.n[0], stream ? stream : h.stream, sweep, fwd_next);
+    if (h.rect)
+      fft3_rect_local_hamiltonian(a, h.n, stream ? stream : h.stream, sweep, fwd_next);
+    else
+      fft3_local_hamiltonian(a, h.n[0], stream ? stream : h.stream, sweep, fwd_next);
     return;
   }
   cplx *w = h.work;
@@ -586,7 +593,11 @@ void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi,
     a.V = h.V;
     a.kA = h.kA + 3 * KA_CURRENT;
     for (int d = 0; d < 9; d++) a.rlat[d] = h.rlat[d];
-    a.tw = h.axis[0].tw;
+    a.tw = h.axis[2].tw;
+    a.nx = h.n[0];
+    a.ny = h.n[1];
+    a.twx = h.axis[0].tw;
+    a.twy = h.axis[1].tw;
     a.scale = 1.0;
     const projector_tables &t = h.pt;
     if (t.nproj > 0 && t.nunique > 0) {
@@ -596,7 +607,10 @@ void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi,
     }
     a.kin_in = phi + b0;
     a.kin_ld = ld;
-    fft3_fourier_hamiltonian(a, h.n[0], h.stream);
+    if (h.rect)
+      fft3_rect_fourier_hamiltonian(a, h.n, h.stream);
+    else
+      fft3_fourier_hamiltonian(a, h.n[0], h.stream);
   }
 }
 
@@ -983,11 +997,15 @@ static void create(handle &h, const inqamd_system_desc &d, hipStream_t stream) {
     h.max_lds = (size_t)lds;
     const char *path = getenv("INQAMD_HPSI_PATH");
     const bool pencil_forced = path && std::string(path) == "pencil";
-    h.three_sweep = !pencil_forced && h.n[0] == h.n[1] && h.n[1] == h.n[2] &&
-                    fft3_supported(h.n[0], h.max_lds);
+    const bool cubic = h.n[0] == h.n[1] && h.n[1] == h.n[2] && fft3_supported(h.n[0], h.max_lds);
+    h.rect = !pencil_forced && !cubic && fft3_rect_supported(h.n, h.max_lds);
+    h.three_sweep = h.rect || (!pencil_forced && cubic);
     // kernel attributes are set now so that no later call (or capture) has to
     if (h.three_sweep) {
-      fft3_prepare(h.n[0]);
+      if (h.rect)
+        fft3_rect_prepare(h.n);
+      else
+        fft3_prepare(h.n[0]);
       INQAMD_HIP_CHECK(hipStreamCreateWithFlags(&h.aux, hipStreamNonBlocking));
       INQAMD_HIP_CHECK(hipEventCreateWithFlags(&h.ev_fork, hipEventDisableTiming));
       INQAMD_HIP_CHECK(hipEventCreateWithFlags(&h.ev_join, hipEventDisableTiming));
@@ -1370,7 +1388,7 @@ int inqamd_hamiltonian_profile(inqamd_hamiltonian_t h, const void *psi, void *hp
     check_orbital(*h, hpsi, "hpsi");
     check_bands(*h, nst, ld, true);
     INQAMD_REQUIRE(ms && launches, "outputs are null");
-    if (!h->three_sweep)
+    if (!h->three_sweep || h->rect)
       throw error{ERR_UNSUPPORTED, "per-sweep timing needs the three-sweep Hpsi (cubic grid)"};
     const band_chunks plan = chunk_plan(*h, nst, ld, true);
     const int nchunk = plan.n;

@@ -110,7 +110,8 @@ struct inqamd_hamiltonian {
 
   inqamd::fft_axis_plan axis[3];
   size_t max_lds = 65536;       // opt-in LDS per workgroup on this device
-  bool three_sweep = false;     // cubic grid with fft3 kernels available
+  bool three_sweep = false;     // grid with three-sweep kernels (fft3 or fft3_rect)
+  bool rect = false;            // ... those of fft3_rect (the cubic ones where they exist)
 
   double *V = nullptr;          // [N]
   double *kA = nullptr;         // [KA_NSLOTS][3]

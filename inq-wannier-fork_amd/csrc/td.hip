@@ -505,8 +505,8 @@ __global__ __launch_bounds__(256) void vgrad_multi_kernel(const vgrad_multi_args
 struct gpair_args {
   const cplx *A[TD_MAXM];  // band-major [b][kz][kx][ky] forward transforms
   const cplx *Y[TD_MAXM];
-  int L;
-  long total;  // nb * L^3
+  int n[3];
+  long total;  // nb * N
   double bd[3], kad;
 };
 
@@ -516,14 +516,14 @@ template <int MM>
 __global__ __launch_bounds__(256) void gpair_kernel(const gpair_args a, const coef_matrix E,
                                                     double *partial) {
   __shared__ double red[256];
-  const int L = a.L;
-  const long L2 = (long)L * L, L3 = L2 * L;
+  const int nx = a.n[0], ny = a.n[1], nz = a.n[2];
+  const long L2 = (long)nx * ny, L3 = L2 * nz;
   double s = 0.0;
   for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < a.total; e += (long)gridDim.x * 256) {
     const long r = e % L3;
-    const int kz = (int)(r / L2), kx = (int)((r / L) % L), ky = (int)(r % L);
-    const double w = sym_index(kx, L) * a.bd[0] + sym_index(ky, L) * a.bd[1] +
-                     sym_index(kz, L) * a.bd[2] + a.kad;
+    const int kz = (int)(r / L2), kx = (int)((r / ny) % nx), ky = (int)(r % ny);
+    const double w = sym_index(kx, nx) * a.bd[0] + sym_index(ky, ny) * a.bd[1] +
+                     sym_index(kz, nz) * a.bd[2] + a.kad;
     cplx y[MM], x[MM];
 #pragma unroll
     for (int j = 0; j < MM; j++) y[j] = a.Y[j][e];
@@ -972,7 +972,7 @@ void adjoint_half_fused(inqamd_td *td, int nb, cplx *const *Y, int slot, double 
       a.A[k] = td->Ah[k];
       a.Y[k] = Y[M + k];
     }
-    a.L = h.n[0];
+    for (int d = 0; d < 3; d++) a.n[d] = h.n[d];
     a.total = h.npoint * nb;
     for (int e = 0; e < 3; e++) a.bd[e] = w.bd[e];
     a.kad = w.kad;
