@@ -145,6 +145,9 @@ struct fft3_args {
   // hpsi not written at all (the last term of a Taylor chain: only the
   // accumulators need it)
   int skip_store;
+  // deal z tiles per XCD also in the sweeps that run them in natural order
+  // (rows that start off a 128-byte line: neighbouring band tiles share lines)
+  int xcd;
   // launch shapes (0: the process default): z tiles of z_ty y values, x-y
   // planes with plane_threads(L) (xy_wide 1) or twice as many (2)
   int z_ty, xy_wide;

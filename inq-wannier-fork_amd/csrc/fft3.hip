@@ -22,7 +22,9 @@ namespace inqamd {
 template <int R0, int R1, int R2, int TY>
 __global__ __launch_bounds__(z_threads(R0 * R1 * R2)) void z_fwd_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
-  z_fwd_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2)>(a, blockIdx.x, lds);
+  constexpr int TB = Z_COLS / TY;
+  const long t = a.xcd ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
+  z_fwd_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2)>(a, t, lds);
 }
 
 constexpr int wide_threads(int L) {
@@ -53,7 +55,8 @@ void z_bwd_epi_kernel(const fft3_args a) {
   // dealt per XCD)
   constexpr bool T = ACC || FWD;
   constexpr int TB = z_bwd_cols(L, T) / z_bwd_ty(L, T, TY);
-  const long t = T ? (long)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB);
+  const long t =
+      T && !a.xcd ? (long)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB);
   z_bwd_epi_tile<R0, R1, R2, z_bwd_ty(L, T, TY), z_bwd_threads(L, T), ACC, false, FWD,
                  z_bwd_cols(L, T)>(a, t, lds);
 }
@@ -88,7 +91,9 @@ __global__ __launch_bounds__(z_threads(R0 * R1 * R2))
 __attribute__((amdgpu_waves_per_eu(z_bwd_waves(R0 * R1 * R2))))
 void z_kin_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
-  z_bwd_epi_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2), false, true>(a, blockIdx.x, lds);
+  constexpr int TB = Z_COLS / TY;
+  const long t = a.xcd ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
+  z_bwd_epi_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2), false, true>(a, t, lds);
 }
 
 static int z_ty_choice() {

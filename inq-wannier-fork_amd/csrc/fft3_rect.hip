@@ -6,7 +6,10 @@
 // the number of columns of each axis's transform is a run-time value: butterfly w
 // is butterfly w / C of column w % C, by a float reciprocal (exact: w < 2^14).
 // Workgroups of 128 to 1024 threads by the size of the plane, so that a thread
-// holds at most about 12 elements between a stage's loads and its stores.
+// holds at most 12 elements between a stage's loads and its stores and, at the
+// 16 waves that 128 registers leave a CU, as many planes are in flight as its
+// LDS holds: the sweep is bound by the barriers between the stages, which other
+// planes fill.
 
 #include "fft3_rect.hpp"
 
@@ -14,7 +17,7 @@ namespace inqamd {
 
 // Most elements of a plane for a workgroup of NT threads
 constexpr int rect_elements(int NT) {
-  return NT == 128 ? 1280 : (NT == 256 ? 2560 : (NT == 512 ? 6144 : 10240));
+  return NT == 128 ? 1280 : (NT == 256 ? 3072 : (NT == 512 ? 5120 : 10240));
 }
 
 // Most columns beside an axis of length L

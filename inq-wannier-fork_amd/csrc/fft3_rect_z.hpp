@@ -12,7 +12,7 @@ __global__ __launch_bounds__(z_threads(R0 * R1 * R2)) void rect_z_fwd_kernel(con
   extern __shared__ cplx lds[];
   constexpr int TB = Z_COLS / RECT_TY;
   // (the potential form shares V and the ownership words over a pair's band tiles)
-  const long t = POT ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
+  const long t = POT || a.xcd ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
   z_fwd_tile<R0, R1, R2, RECT_TY, z_threads(R0 * R1 * R2), POT, true>(a, t, lds);
 }
 
@@ -24,7 +24,8 @@ void rect_z_bwd_kernel(const fft3_args a) {
   constexpr int L = R0 * R1 * R2;
   constexpr bool T = ACC || FWD;
   constexpr int ZC = z_bwd_cols(L, T), TY = ZC == Z_COLS ? RECT_TY : RECT_TY / 2, TB = ZC / TY;
-  const long t = T ? (long)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB);
+  const long t =
+      T && !a.xcd ? (long)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB);
   z_bwd_epi_tile<R0, R1, R2, TY, z_bwd_threads(L, T), ACC, false, FWD, ZC, true>(a, t, lds);
 }
 
@@ -33,8 +34,10 @@ __global__ __launch_bounds__(z_threads(R0 * R1 * R2))
 __attribute__((amdgpu_waves_per_eu(z_bwd_waves(R0 * R1 * R2))))
 void rect_z_kin_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
+  constexpr int TB = Z_COLS / RECT_TY;
+  const long t = a.xcd ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
   z_bwd_epi_tile<R0, R1, R2, RECT_TY, z_threads(R0 * R1 * R2), false, true, false, Z_COLS, true>(
-      a, blockIdx.x, lds);
+      a, t, lds);
 }
 
 template <typename K>

@@ -399,6 +399,12 @@ static void local_passes(handle &h, const cplx *psi, long ld, cplx *hpsi, long h
       a.gdump = acc->gdump + (size_t)b0 * h.npoint;
     }
     a.skip_store = skip_store ? 1 : 0;
+    // Rows of a whole number of 128-byte lines keep the natural order where it
+    // is the faster one; others are dealt per XCD everywhere: each band tile of
+    // such a row shares its first and last line with its neighbours, and the
+    // eight L2s would each fetch and write them (ETRS step at 72^3 x 101 bands
+    // 10.26 -> 9.61 ms, 64^3 x 101 6.91 -> 6.60, 48 x 60 x 72 x 101 6.16 -> 5.89)
+    a.xcd = ld % 8 != 0;
     a.z_ty = h.tune_z_ty;
     a.xy_wide = h.tune_xy_wide;
     if (h.rect)
@@ -457,6 +463,12 @@ struct band_chunks {
   }
 };
 
+// Whether two chunks can be in flight: both have a slot of the intermediate.
+// (The last of two contiguous chunks needs only its own bands.)
+static bool two_slots(const handle &h, const band_chunks &p) {
+  return p.n > 1 && (2 * p.chunk <= h.max_bands || (p.n == 2 && !p.gskip));
+}
+
 static band_chunks chunk_plan(const handle &h, int nst, long ld, bool groups) {
   static const bool enabled = [] {
     const char *e = getenv("INQAMD_BAND_GROUPS");
@@ -505,7 +517,7 @@ void hamiltonian_apply(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld
     const char *e = getenv("INQAMD_PIPELINE");
     return !(e && atoi(e) == 0);
   }();
-  const bool two = pipeline && h.three_sweep && h.aux && chunk < nst && 2 * chunk <= h.max_bands;
+  const bool two = pipeline && h.three_sweep && h.aux && two_slots(h, plan);
   bool overlap = false;
   if (two) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -605,6 +617,7 @@ void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi,
       a.Qe = h.vnl + b0;
       a.ldQ = nst;
     }
+    a.xcd = nst % 8 != 0;
     a.kin_in = phi + b0;
     a.kin_ld = ld;
     if (h.rect)
@@ -682,7 +695,7 @@ void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int s
     const char *e = getenv("INQAMD_PIPELINE");
     return !(e && atoi(e) == 0);
   }();
-  const bool two = pipeline && h.aux && plan.chunk < nst && 2 * plan.chunk <= h.max_bands;
+  const bool two = pipeline && h.aux && two_slots(h, plan);
   const bool proj = h.pt.nproj > 0 && h.pt.nunique > 0;
   projector_phases(h, slot);
   if (two) {
