@@ -209,7 +209,8 @@ int inqamd_preconditioner(inqamd_hamiltonian_t h, void *phi, int nst, int ld);
 /* operations::orthogonalize (orthogonalize.hpp:25-32): Cholesky of
  * S = dV Phi^H Phi and Phi <- Phi R^-H (Gram-Schmidt in band order), in
  * place; dV of real space (fourier = 0) or G space (fourier != 0).
- * Synchronises the handle's stream (the factorisation runs on the host). */
+ * Synchronises the handle's stream (it refuses an overlap without a factor,
+ * leaving phi as it is). */
 int inqamd_orthogonalize(inqamd_hamiltonian_t h, void *phi, int nst, int ld, int fourier);
 /* eigensolvers::steepest_descent (steepest_descent.hpp:23-88) on fourier_space
  * orbitals with ks_hamiltonian's G-space operator (ks_hamiltonian.hpp:156-176)

@@ -16,7 +16,7 @@
 //   pass 4  <r|r>, <phi|r>, <r|Hr>, <phi|Hr> and the step lambda per band
 //   pass 5  phi += lambda r, hphi += lambda Hr (with the next step's pass-1 sums)
 // orthogonalize forms S = dV Phi^H Phi (a split-K strided-batched ZGEMM),
-// factors it on the host (S = R R^H, R lower) and applies Phi <- Phi R^-H
+// factors it (S = R R^H, R lower: cholesky.hip) and applies Phi <- Phi R^-H
 // with ZGEMM; the subspace diagonalisation diagonalises dV Phi^H H Phi with
 // rocSOLVER ZHEEVD.
 
@@ -45,10 +45,11 @@ struct gs_state {
   double *band = nullptr;   // [max_bands][16] per-band results
   rocblas_handle blas = nullptr;
   cplx *S = nullptr;        // [max_bands]^2 device overlap / rotation
+  cplx *T = nullptr;        // [max_bands]^2 rotation of orthogonalize
+  cplx *chol = nullptr;     // scratch of the Cholesky factorisation
   double *eig = nullptr;    // [2 max_bands] eigenvalues + tridiagonal work
   cplx *ip_part = nullptr;  // [IP_BATCHES + 1][max_bands]^2 split-K inner-product partials
   rocblas_int *info = nullptr;
-  std::vector<std::complex<double>> hostS;
 };
 
 #define GS_BLAS_CHECK(expr)                                                              \
@@ -96,6 +97,8 @@ void ensure_blas(handle &h) {
   gs_state &g = state(h);
   if (!g.blas) GS_BLAS_CHECK(rocblas_create_handle(&g.blas));
   if (!g.S) g.S = (cplx *)dalloc((size_t)h.max_bands * h.max_bands * sizeof(cplx));
+  if (!g.T) g.T = (cplx *)dalloc((size_t)h.max_bands * h.max_bands * sizeof(cplx));
+  if (!g.chol) g.chol = (cplx *)dalloc((size_t)cholesky_scratch(h.max_bands) * sizeof(cplx));
   if (!g.eig) g.eig = (double *)dalloc((size_t)2 * h.max_bands * sizeof(double));
   if (!g.info) g.info = (rocblas_int *)dalloc(sizeof(rocblas_int));
   if (!g.ip_part)
@@ -527,51 +530,24 @@ void orthogonalize(handle &h, cplx *phi, long ld, int nst, double dV) {
   gs_state &g = state(h);
   // S[i][j] = dV sum_p conj(phi_pi) phi_pj, row-major
   inner_products(h, phi, ld, phi, ld, nst, dV, g.S);
-  g.hostS.resize((size_t)nst * nst);
-  INQAMD_HIP_CHECK(hipMemcpyAsync(g.hostS.data(), g.S, (size_t)nst * nst * sizeof(cplx),
-                                  hipMemcpyDeviceToHost, h.stream));
+  cholesky_rotation(g.S, nst, g.chol, g.T, g.info, h.stream);
+  // phi stays as it is where S has no factor
+  rocblas_int band = -1;
+  INQAMD_HIP_CHECK(
+      hipMemcpyAsync(&band, g.info, sizeof(band), hipMemcpyDeviceToHost, h.stream));
   INQAMD_HIP_CHECK(hipStreamSynchronize(h.stream));
-  using C = std::complex<double>;
-  const std::vector<C> &S = g.hostS;
-  std::vector<C> R((size_t)nst * nst, 0.0);
-  for (int j = 0; j < nst; j++) {
-    double d = std::real(S[(size_t)j * nst + j]);
-    for (int k = 0; k < j; k++) d -= std::norm(R[(size_t)j * nst + k]);
-    if (!(d > 0.0)) throw error{ERR_ARGUMENT, "orthogonalize: overlap matrix is not positive definite (band " + std::to_string(j) + ")"};
-    const double rjj = std::sqrt(d);
-    R[(size_t)j * nst + j] = rjj;
-    for (int i = j + 1; i < nst; i++) {
-      C v = S[(size_t)i * nst + j];
-      for (int k = 0; k < j; k++) v -= R[(size_t)i * nst + k] * std::conj(R[(size_t)j * nst + k]);
-      R[(size_t)i * nst + j] = v / rjj;
-    }
-  }
-  // R^-1 by forward substitution, then T = (R^-1)^H, upper triangular
-  std::vector<C> Ri((size_t)nst * nst, 0.0);
-  for (int c = 0; c < nst; c++) {
-    Ri[(size_t)c * nst + c] = 1.0 / std::real(R[(size_t)c * nst + c]);
-    for (int i = c + 1; i < nst; i++) {
-      C v = 0.0;
-      for (int k = c; k < i; k++) v -= R[(size_t)i * nst + k] * Ri[(size_t)k * nst + c];
-      Ri[(size_t)i * nst + c] = v / std::real(R[(size_t)i * nst + i]);
-    }
-  }
-  std::vector<C> &T = g.hostS;
-  for (int i = 0; i < nst; i++)
-    for (int j = 0; j < nst; j++) T[(size_t)i * nst + j] = std::conj(Ri[(size_t)j * nst + i]);
-  INQAMD_HIP_CHECK(hipMemcpyAsync(g.S, T.data(), (size_t)nst * nst * sizeof(cplx),
-                                  hipMemcpyHostToDevice, h.stream));
+  if (band >= 0)
+    throw error{ERR_ARGUMENT, "orthogonalize: overlap matrix is not positive definite (band " +
+                                  std::to_string(band) + ")"};
   // out[p][j] = sum_i phi[p][i] T[i][j]: column-major out^T = T_cm * Phi^T
   // with T_cm (ld nst) the row-major T read column-major
   const rocblas_double_complex one = {1.0, 0.0}, zero = {0.0, 0.0};
   GS_BLAS_CHECK(rocblas_zgemm(g.blas, rocblas_operation_none, rocblas_operation_none, nst,
                               (rocblas_int)h.npoint, nst, &one,
-                              reinterpret_cast<const rocblas_double_complex *>(g.S), nst,
+                              reinterpret_cast<const rocblas_double_complex *>(g.T), nst,
                               reinterpret_cast<const rocblas_double_complex *>(phi), (int)ld,
                               &zero, reinterpret_cast<rocblas_double_complex *>(h.hn), nst));
   copy(h, h.hn, nst, phi, ld, nst);
-  // the host buffer is reused by the next call only after this copy ran
-  INQAMD_HIP_CHECK(hipStreamSynchronize(h.stream));
 }
 
 // eigensolvers::steepest_descent (steepest_descent.hpp:23-88) on
@@ -659,7 +635,7 @@ void gs_release(handle &h) {
   if (!h.gs) return;
   gs_state *g = static_cast<gs_state *>(h.gs);
   for (void *p : {(void *)g->hphi, (void *)g->res, (void *)g->hres, (void *)g->part,
-                  (void *)g->band, (void *)g->S, (void *)g->eig, (void *)g->info,
+                  (void *)g->band, (void *)g->S, (void *)g->T, (void *)g->chol, (void *)g->eig, (void *)g->info,
                   (void *)g->ip_part})
     if (p) (void)hipFree(p);
   if (g->blas) (void)rocblas_destroy_handle(g->blas);

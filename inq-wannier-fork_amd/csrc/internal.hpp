@@ -205,6 +205,9 @@ void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int s
                   std::complex<double> z2, cplx *const *outs, cplx *const *dumps);
 void exponential_in_place(handle &h, std::complex<double> z, int order, cplx *psi, long ld,
                           int nst, int slot);
+// cholesky.hip
+long cholesky_scratch(int n);
+void cholesky_rotation(cplx *S, int n, cplx *scratch, cplx *T, int *info, hipStream_t stream);
 // gs.hip
 void hamiltonian_fourier(handle &h, const cplx *phi, long ld, cplx *hphi, long hld, int nst);
 void gs_release(handle &h);
