@@ -34,9 +34,15 @@
 namespace inqamd {
 namespace {
 
-constexpr int GS_BT = 64;       // bands per reduction block
-constexpr int GS_LANES = 4;     // point lanes per band
-constexpr long GS_CHUNK = 512;  // grid points per partial sum
+// The per-band reductions run in blocks of 256 threads over a chunk of points and
+// BT = 64 or 16 bands, 256 / BT lanes of points per band: 16 where 64 would leave
+// a quarter of the lanes or more without a band (the descent at 40^3 x 48 bands
+// 2.54 -> 1.90 ms together with the shorter chunks).  Chunks of up to
+// GS_CHUNK points, shorter where that would leave fewer than GS_BLOCKS blocks
+// (125 for 40^3 x 48, on 256 CUs).
+constexpr long GS_CHUNK = 512;
+constexpr long GS_CHUNK_MIN = 64;
+constexpr long GS_BLOCKS = 2048;
 constexpr int IP_BATCHES = 64;  // point chunks of the split-K inner products
 
 struct gs_state {
@@ -60,7 +66,32 @@ struct gs_state {
                                                    rocblas_status_to_string(_s)};        \
   } while (0)
 
-long nchunks(const handle &h) { return (h.npoint + GS_CHUNK - 1) / GS_CHUNK; }
+// Launch shape of the per-band reductions over nst bands
+struct gs_shape {
+  int bt;       // bands per block
+  long groups;  // blocks of bands
+  long chunk;   // points per partial sum
+  long nchunk;
+};
+
+gs_shape shape(const handle &h, int nst) {
+  gs_shape g;
+  g.bt = nst % 64 == 0 || nst % 64 > 48 ? 64 : 16;
+  g.groups = (nst + g.bt - 1) / g.bt;
+  g.chunk = (h.npoint * g.groups + GS_BLOCKS - 1) / GS_BLOCKS;
+  g.chunk = g.chunk < GS_CHUNK_MIN ? GS_CHUNK_MIN : (g.chunk > GS_CHUNK ? GS_CHUNK : g.chunk);
+  g.nchunk = (h.npoint + g.chunk - 1) / g.chunk;
+  return g;
+}
+
+// Most partial sums (chunks x bands) of any nst <= max_bands: chunks of
+// GS_CHUNK, or GS_BLOCKS blocks of at most 64 bands (and a chunk cut short in
+// each band group)
+long most_partials(const handle &h) {
+  const long full = (h.npoint + GS_CHUNK - 1) / GS_CHUNK * h.max_bands;
+  const long split = (GS_BLOCKS + h.max_bands / 16 + 1) * 64;
+  return full > split ? full : split;
+}
 
 gs_state &state(handle &h) {
   if (!h.gs) h.gs = new gs_state();
@@ -77,7 +108,7 @@ void *dalloc(size_t bytes) {
 void ensure_reductions(handle &h) {
   gs_state &g = state(h);
   if (!g.part) {
-    g.part = (double *)dalloc((size_t)nchunks(h) * h.max_bands * 8 * sizeof(double));
+    g.part = (double *)dalloc((size_t)most_partials(h) * 8 * sizeof(double));
     g.band = (double *)dalloc((size_t)h.max_bands * 16 * sizeof(double));
   }
 }
@@ -112,10 +143,11 @@ void ensure_blas(handle &h) {
 struct gspace {
   int n0, n1, n2;
   double b[9];
-  __device__ void m_of(long p, int &m0, int &m1, int &m2) const {
-    const int iz = (int)(p % n2);
-    const long t = p / n2;
-    const int iy = (int)(t % n1), ix = (int)(t / n1);
+  __device__ void m_of(long point, int &m0, int &m1, int &m2) const {
+    const unsigned p = (unsigned)point;  // (grids have fewer than 2^31 points)
+    const unsigned t = p / (unsigned)n2;
+    const int iz = (int)(p - t * (unsigned)n2);
+    const int iy = (int)(t % (unsigned)n1), ix = (int)(t / (unsigned)n1);
     m0 = ix >= (n0 + 1) / 2 ? ix - n0 : ix;
     m1 = iy >= (n1 + 1) / 2 ? iy - n1 : iy;
     m2 = iz >= (n2 + 1) / 2 ? iz - n2 : iz;
@@ -167,39 +199,49 @@ __global__ __launch_bounds__(256) void laplacian_add_kernel(gspace geo, const cp
 }
 
 // ---------------------------------------------------------------------------
-// per-band reductions: block (chunk, 64-band group); thread = band x lane
+// per-band reductions: block (chunk, band group); thread = band x lane
 // ---------------------------------------------------------------------------
-template <int NV, class F>
-__device__ __forceinline__ void band_partials(long npoint, int nst, double *part, F term) {
-  __shared__ double red[GS_LANES][GS_BT][NV];
-  const int bb = threadIdx.x % GS_BT;
-  const int lane = threadIdx.x / GS_BT;
-  const int b = blockIdx.y * GS_BT + bb;
-  const long p0 = (long)blockIdx.x * GS_CHUNK;
-  const long p1 = p0 + GS_CHUNK < npoint ? p0 + GS_CHUNK : npoint;
+template <int NV, int BT, class F>
+__device__ __forceinline__ void band_partials(long npoint, long chunk, int nst, double *part,
+                                              F term) {
+  constexpr int LANES = 256 / BT;
+  __shared__ double red[4][BT][NV];
+  const int bb = threadIdx.x % BT;
+  const int lane = threadIdx.x / BT;
+  const int b = blockIdx.y * BT + bb;
+  const long p0 = (long)blockIdx.x * chunk;
+  const long p1 = p0 + chunk < npoint ? p0 + chunk : npoint;
   double acc[NV];
 #pragma unroll
   for (int v = 0; v < NV; v++) acc[v] = 0.0;
   if (b < nst)
-    for (long p = p0 + lane; p < p1; p += GS_LANES) term(p, b, acc);
+    for (long p = p0 + lane; p < p1; p += LANES) term(p, b, acc);
+  // the lanes of a band within each wave by a butterfly, the waves in order
 #pragma unroll
-  for (int v = 0; v < NV; v++) red[lane][bb][v] = acc[v];
+  for (int w = BT; w < 64; w <<= 1)
+#pragma unroll
+    for (int v = 0; v < NV; v++) acc[v] += __shfl_xor(acc[v], w, 64);
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) < BT)
+#pragma unroll
+    for (int v = 0; v < NV; v++) red[wave][bb][v] = acc[v];
   __syncthreads();
-  if (lane == 0 && b < nst) {
+  if (threadIdx.x < BT && b < nst) {
 #pragma unroll
     for (int v = 0; v < NV; v++) {
       double s = red[0][bb][v];
-      for (int l = 1; l < GS_LANES; l++) s += red[l][bb][v];
+      for (int l = 1; l < 4; l++) s += red[l][bb][v];
       part[((long)blockIdx.x * nst + b) * 8 + v] = s;
     }
   }
 }
 
 // pass 1: eig = sum conj(hphi) phi, norm = sum |phi|^2
+template <int BT>
 __global__ __launch_bounds__(256) void eig_norm_partial(const cplx *__restrict__ hphi, long hld,
                                                         const cplx *__restrict__ phi, long ld,
-                                                        int nst, long npoint, double *part) {
-  band_partials<3>(npoint, nst, part, [&](long p, int b, double *a) {
+                                                        int nst, long npoint, long chunk, double *part) {
+  band_partials<3, BT>(npoint, chunk, nst, part, [&](long p, int b, double *a) {
     const cplx h = hphi[p * hld + b], f = phi[p * ld + b];
     a[0] += h.x * f.x + h.y * f.y;
     a[1] += h.x * f.y - h.y * f.x;
@@ -209,12 +251,13 @@ __global__ __launch_bounds__(256) void eig_norm_partial(const cplx *__restrict__
 
 // pass 2: residual = hphi - evn phi (shift.hpp:19-31 with factor -1), and
 // the preconditioner's sums 1/2|G|^2 |r|^2, |r|^2 (preconditioner.hpp:42)
+template <int BT>
 __global__ __launch_bounds__(256) void residual_partial(gspace geo, const cplx *__restrict__ hphi,
                                                         long hld, const cplx *__restrict__ phi,
                                                         long ld, cplx *__restrict__ res, long rld,
                                                         const double *__restrict__ band, int nst,
-                                                        long npoint, double *part) {
-  band_partials<2>(npoint, nst, part, [&](long p, int b, double *a) {
+                                                        long npoint, long chunk, double *part) {
+  band_partials<2, BT>(npoint, chunk, nst, part, [&](long p, int b, double *a) {
     const double er = band[b * 16 + 3], ei = band[b * 16 + 4];  // evn
     const cplx h = hphi[p * hld + b], f = phi[p * ld + b];
     cplx r;
@@ -231,11 +274,12 @@ __global__ __launch_bounds__(256) void residual_partial(gspace geo, const cplx *
 }
 
 // pass 4: m0 = <r|r>, m1 = <phi|r>, m2 = <r|Hr>, m3 = <phi|Hr>
+template <int BT>
 __global__ __launch_bounds__(256) void mm_partial(const cplx *__restrict__ phi, long ld,
                                                   const cplx *__restrict__ res,
                                                   const cplx *__restrict__ hres, long rld, int nst,
-                                                  long npoint, double *part) {
-  band_partials<8>(npoint, nst, part, [&](long p, int b, double *a) {
+                                                  long npoint, long chunk, double *part) {
+  band_partials<8, BT>(npoint, chunk, nst, part, [&](long p, int b, double *a) {
     const cplx f = phi[p * ld + b], r = res[p * rld + b], hr = hres[p * rld + b];
     a[0] += r.x * r.x + r.y * r.y;
     a[1] += r.x * r.y - r.y * r.x;
@@ -365,19 +409,20 @@ __global__ __launch_bounds__(256) void precondition_kernel(gspace geo, cplx *__r
 
 // pass 5 (steepest_descent.hpp:70-77) of the last step, which leaves hphi:
 // phi += lambda r over the grid of the partial-sum passes (point chunk x
-// 64-band block; the lanes of a point chunk stride its points)
+// band group; the lanes of a point chunk stride its points)
+template <int BT>
 __global__ __launch_bounds__(256) void sd_update_phi(cplx *__restrict__ phi, long ld,
                                                      const cplx *__restrict__ res, long rld,
-                                                     int nst, long npoint,
+                                                     int nst, long npoint, long chunk,
                                                      const double *__restrict__ band) {
-  const int bb = threadIdx.x % GS_BT;
-  const int lane = threadIdx.x / GS_BT;
-  const int b = blockIdx.y * GS_BT + bb;
+  const int bb = threadIdx.x % BT;
+  const int lane = threadIdx.x / BT;
+  const int b = blockIdx.y * BT + bb;
   if (b >= nst) return;
-  const long p0 = (long)blockIdx.x * GS_CHUNK;
-  const long p1 = p0 + GS_CHUNK < npoint ? p0 + GS_CHUNK : npoint;
+  const long p0 = (long)blockIdx.x * chunk;
+  const long p1 = p0 + chunk < npoint ? p0 + chunk : npoint;
   const double lam = band[b * 16 + 6];
-  for (long p = p0 + lane; p < p1; p += GS_LANES) {
+  for (long p = p0 + lane; p < p1; p += 256 / BT) {
     cplx f = phi[p * ld + b];
     const cplx r = res[p * rld + b];
     f.x += lam * r.x;
@@ -389,14 +434,15 @@ __global__ __launch_bounds__(256) void sd_update_phi(cplx *__restrict__ phi, lon
 // pass 5 of a step fused with pass 1 of the next (the partial sums of
 // eig_norm_partial over the updated phi and hphi, in its order), for steps
 // that update hphi
+template <int BT>
 __global__ __launch_bounds__(256) void sd_update_eig_norm(cplx *__restrict__ phi, long ld,
                                                           const cplx *__restrict__ res,
                                                           cplx *__restrict__ hphi,
                                                           const cplx *__restrict__ hres, long rld,
                                                           int nst, long npoint,
                                                           const double *__restrict__ band,
-                                                          double *part) {
-  band_partials<3>(npoint, nst, part, [&](long p, int b, double *a) {
+                                                          long chunk, double *part) {
+  band_partials<3, BT>(npoint, chunk, nst, part, [&](long p, int b, double *a) {
     const double lam = band[b * 16 + 6];
     cplx f = phi[p * ld + b];
     const cplx r = res[p * rld + b];
@@ -414,9 +460,16 @@ __global__ __launch_bounds__(256) void sd_update_eig_norm(cplx *__restrict__ phi
   });
 }
 
-dim3 red_grid(const handle &h, int nst) {
-  return dim3((unsigned)nchunks(h), (unsigned)((nst + GS_BT - 1) / GS_BT));
-}
+// Launches a reduction kernel in the shape of nst bands
+#define GS_REDUCE(kernel, g, stream, ...)                                                  \
+  do {                                                                                     \
+    const dim3 grid_((unsigned)(g).nchunk, (unsigned)(g).groups);                          \
+    if ((g).bt == 64)                                                                      \
+      hipLaunchKernelGGL(kernel<64>, grid_, dim3(256), 0, stream, __VA_ARGS__);            \
+    else                                                                                   \
+      hipLaunchKernelGGL(kernel<16>, grid_, dim3(256), 0, stream, __VA_ARGS__);            \
+    check_launch();                                                                        \
+  } while (0)
 
 void check_launch() { INQAMD_HIP_CHECK(hipGetLastError()); }
 
@@ -472,7 +525,7 @@ void inner_products(handle &h, const cplx *A, long lda, const cplx *B, long ldb,
 void precondition_apply(handle &h, cplx *phi, long ld, int nst) {
   gs_state &g = state(h);
   hipLaunchKernelGGL(kinetic_final, dim3(nst), dim3(256), 0, h.stream,
-                     (const double *)g.part, nchunks(h), nst, g.band);
+                     (const double *)g.part, shape(h, nst).nchunk, nst, g.band);
   check_launch();
   const long waves = h.npoint < PRECOND_POINT_WAVES ? h.npoint : PRECOND_POINT_WAVES;
   hipLaunchKernelGGL(precondition_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
@@ -481,10 +534,11 @@ void precondition_apply(handle &h, cplx *phi, long ld, int nst) {
 }
 
 // kinetic sums of phi alone (preconditioner.hpp:42) into the partial buffer
+template <int BT>
 __global__ __launch_bounds__(256) void kinetic_partial(gspace geo, const cplx *__restrict__ phi,
                                                        long ld, int nst, long npoint,
-                                                       double *part) {
-  band_partials<2>(npoint, nst, part, [&](long p, int b, double *a) {
+                                                       long chunk, double *part) {
+  band_partials<2, BT>(npoint, chunk, nst, part, [&](long p, int b, double *a) {
     const cplx f = phi[p * ld + b];
     int m0, m1, m2;
     geo.m_of(p, m0, m1, m2);
@@ -516,9 +570,9 @@ void hamiltonian_fourier(handle &h, const cplx *phi, long ld, cplx *hphi, long h
 void preconditioner(handle &h, cplx *phi, long ld, int nst) {
   ensure_reductions(h);
   gs_state &g = state(h);
-  hipLaunchKernelGGL(kinetic_partial, red_grid(h, nst), dim3(256), 0, h.stream, geometry(h),
-                     (const cplx *)phi, ld, nst, h.npoint, g.part);
-  check_launch();
+  const gs_shape rs = shape(h, nst);
+  GS_REDUCE(kinetic_partial, rs, h.stream, geometry(h), (const cplx *)phi, ld, nst, h.npoint,
+            rs.chunk, g.part);
   precondition_apply(h, phi, ld, nst);
 }
 
@@ -556,42 +610,38 @@ void steepest_descent(handle &h, cplx *phi, long ld, int nst, bool precond) {
   ensure_workspace(h);
   gs_state &g = state(h);
   const long rl = nst;
-  const long nchunk = nchunks(h);
+  const gs_shape rs = shape(h, nst);
+  const long nchunk = rs.nchunk;
   // fourier_space::volume_element (fourier_space.hpp:41-44)
   const double dV = h.volume / ((double)h.npoint * (double)h.npoint);
-  const dim3 rg = red_grid(h, nst), fg(nst);
+  const dim3 fg(nst);
   hamiltonian_fourier(h, phi, ld, g.hphi, rl, nst);
   const int num_steps = 5;
   for (int istep = 0; istep < num_steps; istep++) {
     // pass 1 (after the first step, the previous step's update made its sums)
     if (istep == 0) {
-      hipLaunchKernelGGL(eig_norm_partial, rg, dim3(256), 0, h.stream, (const cplx *)g.hphi,
-                         rl, (const cplx *)phi, ld, nst, h.npoint, g.part);
-      check_launch();
+      GS_REDUCE(eig_norm_partial, rs, h.stream, (const cplx *)g.hphi, rl, (const cplx *)phi, ld,
+                nst, h.npoint, rs.chunk, g.part);
     }
     hipLaunchKernelGGL(eig_norm_final, fg, dim3(256), 0, h.stream, (const double *)g.part, nchunk,
                        nst, dV, g.band);
     check_launch();
-    hipLaunchKernelGGL(residual_partial, rg, dim3(256), 0, h.stream, geometry(h),
-                       (const cplx *)g.hphi, rl, (const cplx *)phi, ld, g.res, rl,
-                       (const double *)g.band, nst, h.npoint, g.part);
-    check_launch();
+    GS_REDUCE(residual_partial, rs, h.stream, geometry(h), (const cplx *)g.hphi, rl,
+              (const cplx *)phi, ld, g.res, rl, (const double *)g.band, nst, h.npoint, rs.chunk,
+              g.part);
     if (precond) precondition_apply(h, g.res, rl, nst);
     hamiltonian_fourier(h, g.res, rl, g.hres, rl, nst);
-    hipLaunchKernelGGL(mm_partial, rg, dim3(256), 0, h.stream, (const cplx *)phi, ld,
-                       (const cplx *)g.res, (const cplx *)g.hres, rl, nst, h.npoint, g.part);
-    check_launch();
+    GS_REDUCE(mm_partial, rs, h.stream, (const cplx *)phi, ld, (const cplx *)g.res,
+              (const cplx *)g.hres, rl, nst, h.npoint, rs.chunk, g.part);
     hipLaunchKernelGGL(lambda_final, fg, dim3(256), 0, h.stream, (const double *)g.part, nchunk,
                        nst, dV, g.band);
     check_launch();
     if (istep != num_steps - 1)
-      hipLaunchKernelGGL(sd_update_eig_norm, rg, dim3(256), 0, h.stream, phi, ld,
-                         (const cplx *)g.res, g.hphi, (const cplx *)g.hres, rl, nst, h.npoint,
-                         (const double *)g.band, g.part);
+      GS_REDUCE(sd_update_eig_norm, rs, h.stream, phi, ld, (const cplx *)g.res, g.hphi,
+                (const cplx *)g.hres, rl, nst, h.npoint, (const double *)g.band, rs.chunk, g.part);
     else
-      hipLaunchKernelGGL(sd_update_phi, rg, dim3(256), 0, h.stream, phi, ld,
-                         (const cplx *)g.res, rl, nst, h.npoint, (const double *)g.band);
-    check_launch();
+      GS_REDUCE(sd_update_phi, rs, h.stream, phi, ld, (const cplx *)g.res, rl, nst, h.npoint,
+                rs.chunk, (const double *)g.band);
   }
   orthogonalize(h, phi, ld, nst, dV);
 }
