@@ -82,6 +82,17 @@ bool fft_dense_launch(const fft_pass_args &a, int mode, hipStream_t stream);
 // Powers H^n psi that a Taylor chain keeps before one sweep adds them to its sums
 constexpr int TAYLOR_PENDING = 3;
 
+struct project_expand_args;  // internal.hpp
+
+// The projector phases e^{+-i(k+A).r} of a call, computed by extra workgroups of
+// its first sweep (pos == nullptr: none)
+struct phase_args {
+  const float *pos;
+  const int *uent;
+  int nsph, nent;
+  cplx *sph, *ent;
+};
+
 // Arguments of the three-sweep local Hamiltonian (fft3.hip) on a band chunk
 // of a cubic L^3 grid (or an nx x ny x nz one: fft3_rect.hpp).
 struct fft3_args {
@@ -145,6 +156,9 @@ struct fft3_args {
   // hpsi not written at all (the last term of a Taylor chain: only the
   // accumulators need it)
   int skip_store;
+  // the phases of the projector, in workgroups after the z forward tiles
+  phase_args phase;
+  int nproj;  // spheres of the projector that an x-y launch carries
   // deal z tiles per XCD also in the sweeps that run them in natural order
   // (rows that start off a 128-byte line: neighbouring band tiles share lines)
   int xcd;
@@ -170,15 +184,21 @@ bool fft3_supported(int L, size_t max_lds);
 void fft3_prepare(int L);
 // hpsi = IFFT(1/2|G+k+A|^2 FFT(psi)) / N + V psi for the chunk's bands: all
 // three sweeps (sweep < 0) or only sweep 0 (z forward), 1 (x-y) or 2 (z back).
+// proj: the chunk's projector coefficients, by workgroups of the x-y launch
+// (lengths and workgroup shapes of fft3_projector only).
 void fft3_local_hamiltonian(const fft3_args &a, int L, hipStream_t stream, int sweep = -1,
-                            bool fwd_next = false);
+                            bool fwd_next = false, const project_expand_args *proj = nullptr);
+// Whether the x-y launch of nb bands on an L^3 grid may carry the projector;
+// xy_wide as in fft3_args.
+bool fft3_projector(int L, int nb, int xy_wide);
 
 // The same sweeps on an n[0] x n[1] x n[2] grid (fft3_rect.hip): true when every
 // length has a plan there and the plane and the z tile fit in max_lds.
 bool fft3_rect_supported(const int n[3], size_t max_lds);
 void fft3_rect_prepare(const int n[3]);
 void fft3_rect_local_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream, int sweep,
-                                 bool fwd_next);
+                                 bool fwd_next, const project_expand_args *proj = nullptr);
+bool fft3_rect_projector(const int n[3], int nb);
 void fft3_rect_fourier_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream);
 
 }  // namespace inqamd

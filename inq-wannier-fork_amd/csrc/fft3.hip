@@ -9,6 +9,7 @@
 // so W stays resident in the Infinity Cache between sweeps.
 
 #include "fft3_tiles.hpp"
+#include "projector_dev.hpp"
 
 #include <cstdlib>
 
@@ -23,7 +24,12 @@ template <int R0, int R1, int R2, int TY>
 __global__ __launch_bounds__(z_threads(R0 * R1 * R2)) void z_fwd_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
   constexpr int TB = Z_COLS / TY;
-  const long t = a.xcd ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
+  const long tiles = z_tiles<TY>(R0 * R1 * R2, a.nb);
+  if (blockIdx.x >= tiles) {
+    phase_block(a, (int)(blockIdx.x - tiles));
+    return;
+  }
+  const long t = a.xcd ? xcd_tile(blockIdx.x, tiles, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
   z_fwd_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2)>(a, t, lds);
 }
 
@@ -36,6 +42,24 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(xy_kin_waves
 void xy_kin_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
   xy_kin_plane<R0, R1, R2, NT>(a, blockIdx.x, lds);
+}
+
+// The same planes after the workgroups of the projector (projector_beside_planes)
+constexpr int proj_plane_threads(int L) { return wide_threads(L) < P4_NT ? wide_threads(L) : P4_NT; }
+
+template <int R0, int R1, int R2>
+constexpr size_t xy_proj_lds() {
+  return xy_kin_lds<R0, R1, R2>() > P4_BLOCK_LDS ? xy_kin_lds<R0, R1, R2>() : P4_BLOCK_LDS;
+}
+
+template <int R0, int R1, int R2>
+__global__ __launch_bounds__(P4_NT) __attribute__((amdgpu_waves_per_eu(4)))
+void xy_proj_kernel(const fft3_args a, const project_expand_args pa, int ntile, int nproj) {
+  extern __shared__ cplx lds[];
+  if ((int)blockIdx.x < nproj)
+    p4_block(pa, blockIdx.x, ntile, lds);
+  else
+    xy_kin_plane<R0, R1, R2, proj_plane_threads(R0 * R1 * R2)>(a, blockIdx.x - nproj, lds);
 }
 
 // TY: y values of a 64-column tile (8 or 16); a 32-column tile takes TY / 2
@@ -130,6 +154,7 @@ static void prepare3() {
   ensure_lds(z_fwd_kernel<R0, R1, R2, 16>, zl);
   ensure_lds(xy_kin_kernel<R0, R1, R2, plane_threads(L)>, xy_kin_lds<R0, R1, R2>());
   ensure_lds(xy_kin_kernel<R0, R1, R2, wide_threads(L)>, xy_kin_lds<R0, R1, R2>());
+  if constexpr (L <= PROJ_MAX_LEN) ensure_lds(xy_proj_kernel<R0, R1, R2>, xy_proj_lds<R0, R1, R2>());
   ensure_lds(z_pot_kernel<R0, R1, R2, 8>, zl);
   ensure_lds(z_kin_kernel<R0, R1, R2, 8>, zl);
   ensure_lds(xy_fwd_kernel<R0, R1, R2, wide_threads(L)>, pl);
@@ -144,22 +169,35 @@ static void prepare3() {
   ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 16, true, true>, zba);
 }
 
+// proj: the launch of the x-y planes with the projector's workgroups
 // sweep: -1 all three, 0/1/2 one of them; fwd_next: the last sweep also
 // transforms its output forward in z into W (Taylor chains)
 template <int R0, int R1, int R2, int TY, int NT>
-static void launch3v(const fft3_args &a, hipStream_t stream, int sweep, bool fwd_next) {
+static void launch3v(const fft3_args &a, hipStream_t stream, int sweep, bool fwd_next,
+                     const project_expand_args *proj) {
   constexpr int L = R0 * R1 * R2;
   const long ztiles = z_tiles<TY>(L, a.nb);
   const size_t zlds = (size_t)L * Z_COLS * sizeof(cplx);
   const size_t plds = xy_kin_lds<R0, R1, R2>();
   if (sweep < 0 || sweep == 0) {
-    hipLaunchKernelGGL((z_fwd_kernel<R0, R1, R2, TY>), dim3((unsigned)ztiles), dim3(z_threads(L)), zlds,
-                       stream, a);
+    hipLaunchKernelGGL((z_fwd_kernel<R0, R1, R2, TY>),
+                       dim3((unsigned)(ztiles + phase_blocks(a, z_threads(L)))),
+                       dim3(z_threads(L)), zlds, stream, a);
     INQAMD_HIP_CHECK(hipGetLastError());
   }
   if (sweep < 0 || sweep == 1) {
-    hipLaunchKernelGGL((xy_kin_kernel<R0, R1, R2, NT>), dim3((unsigned)((long)a.nb * L)), dim3(NT),
-                       plds, stream, a);
+    if (proj) {
+      if constexpr (L <= PROJ_MAX_LEN) {
+        const int ntile = (proj->nbc + P4_BANDS - 1) / P4_BANDS, np = ntile * a.nproj;
+        hipLaunchKernelGGL((xy_proj_kernel<R0, R1, R2>), dim3((unsigned)((long)a.nb * L + np)),
+                           dim3(P4_NT), (xy_proj_lds<R0, R1, R2>()), stream, a, *proj, ntile, np);
+      } else {
+        throw error{ERR_UNSUPPORTED, "no plane kernel with the projector for this length"};
+      }
+    } else {
+      hipLaunchKernelGGL((xy_kin_kernel<R0, R1, R2, NT>), dim3((unsigned)((long)a.nb * L)),
+                         dim3(NT), plds, stream, a);
+    }
     INQAMD_HIP_CHECK(hipGetLastError());
   }
   if (sweep < 0 || sweep == 2) {
@@ -177,20 +215,21 @@ static void launch3v(const fft3_args &a, hipStream_t stream, int sweep, bool fwd
 }
 
 template <int R0, int R1, int R2>
-static void launch3(const fft3_args &a, hipStream_t stream, int sweep, bool fwd_next) {
+static void launch3(const fft3_args &a, hipStream_t stream, int sweep, bool fwd_next,
+                    const project_expand_args *proj) {
   constexpr int L = R0 * R1 * R2;
   const bool wide = a.xy_wide ? a.xy_wide == 2 : xy_wide_choice();
   const int ty = a.z_ty ? a.z_ty : z_ty_choice();
   if (ty == 16) {
     if (wide)
-      launch3v<R0, R1, R2, 16, wide_threads(L)>(a, stream, sweep, fwd_next);
+      launch3v<R0, R1, R2, 16, wide_threads(L)>(a, stream, sweep, fwd_next, proj);
     else
-      launch3v<R0, R1, R2, 16, plane_threads(L)>(a, stream, sweep, fwd_next);
+      launch3v<R0, R1, R2, 16, plane_threads(L)>(a, stream, sweep, fwd_next, proj);
   } else {
     if (wide)
-      launch3v<R0, R1, R2, 8, wide_threads(L)>(a, stream, sweep, fwd_next);
+      launch3v<R0, R1, R2, 8, wide_threads(L)>(a, stream, sweep, fwd_next, proj);
     else
-      launch3v<R0, R1, R2, 8, plane_threads(L)>(a, stream, sweep, fwd_next);
+      launch3v<R0, R1, R2, 8, plane_threads(L)>(a, stream, sweep, fwd_next, proj);
   }
 }
 
@@ -242,14 +281,22 @@ void fft3_prepare(int L) {
 }
 
 void fft3_local_hamiltonian(const fft3_args &a, int L, hipStream_t stream, int sweep,
-                            bool fwd_next) {
+                            bool fwd_next, const project_expand_args *proj) {
   switch (L) {
 #define INQAMD_FFT3_CASE(LL, R0, R1, R2) \
-  case LL: launch3<R0, R1, R2>(a, stream, sweep, fwd_next); return;
+  case LL: launch3<R0, R1, R2>(a, stream, sweep, fwd_next, proj); return;
     INQAMD_FFT3_TABLE(INQAMD_FFT3_CASE)
 #undef INQAMD_FFT3_CASE
     default: throw error{ERR_UNSUPPORTED, "three-sweep Hpsi: unsupported grid length"};
   }
+}
+
+// The planes then run in workgroups of P4_NT threads: at 48 to 64 they do so
+// anyway (384 to 512), below that only where the launch is too small for the
+// idle threads to matter.
+bool fft3_projector(int L, int nb, int xy_wide) {
+  if (xy_wide ? xy_wide != 2 : !xy_wide_choice()) return false;
+  return L <= PROJ_MAX_LEN && (L >= 48 || (long)nb * L <= PROJ_FEW_PLANES);
 }
 
 }  // namespace inqamd

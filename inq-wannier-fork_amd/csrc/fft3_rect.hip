@@ -12,6 +12,7 @@
 // planes fill.
 
 #include "fft3_rect.hpp"
+#include "projector_dev.hpp"
 
 namespace inqamd {
 
@@ -150,12 +151,11 @@ __device__ __forceinline__ void rect_y_kinetic(const rect_cols &k, const cplx *t
   rect_stage<R0, L / R0, L, NT>(k, tw, +1, ld, st);
 }
 
-// FWD: only the forward transforms, in place in W (G-space Hpsi)
+// Plane `plane` = band * nz + z.  FWD: only the forward transforms, in place in W
+// (G-space Hpsi)
 template <int NT, bool FWD>
-__global__ __launch_bounds__(NT) void rect_xy_kernel(const fft3_args a, int nz) {
-  extern __shared__ cplx lds[];
+__device__ __forceinline__ void rect_xy_plane(const fft3_args &a, int nz, long plane, cplx *lds) {
   const int nx = a.nx, ny = a.ny, pad = ny | 1;
-  const long plane = blockIdx.x;  // band * nz + z
   const int z = (int)(plane % nz);
   cplx *W = a.W + plane * nx * ny;
   const rect_cols kx = {ny, 1.0f / (float)ny}, ky = {nx, 1.0f / (float)nx};
@@ -223,6 +223,24 @@ __global__ __launch_bounds__(NT) void rect_xy_kernel(const fft3_args a, int nz) 
   }
 }
 
+template <int NT, bool FWD>
+__global__ __launch_bounds__(NT) void rect_xy_kernel(const fft3_args a, int nz) {
+  extern __shared__ cplx lds[];
+  rect_xy_plane<NT, FWD>(a, nz, blockIdx.x, lds);
+}
+
+// The kinetic planes after the workgroups of the projector
+// (projector_beside_planes)
+__global__ __launch_bounds__(P4_NT) __attribute__((amdgpu_waves_per_eu(4)))
+void rect_xy_proj_kernel(const fft3_args a, int nz, const project_expand_args pa, int ntile,
+                         int nproj) {
+  extern __shared__ cplx lds[];
+  if ((int)blockIdx.x < nproj)
+    p4_block(pa, blockIdx.x, ntile, lds);
+  else
+    rect_xy_plane<P4_NT, false>(a, nz, blockIdx.x - nproj, lds);
+}
+
 // ---------------------------------------------------------------------------
 // host
 // ---------------------------------------------------------------------------
@@ -279,15 +297,33 @@ static void rect_z(const fft3_args &a, int nz, rect_z_kernel k, hipStream_t stre
 
 void fft3_rect_prepare(const int n[3]) {
   const size_t lds = rect_xy_lds(n);
+  if (lds > 65536)
+    INQAMD_HIP_CHECK(hipFuncSetAttribute((const void *)rect_xy_proj_kernel,
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
   rect_xy_prepare<512>(lds);
   rect_xy_prepare<1024>(lds);
   rect_z(fft3_args{}, n[2], RECT_Z_PREPARE, nullptr);
 }
 
+// As fft3_projector: planes of a 512-thread workgroup's size, or few of them
+bool fft3_rect_projector(const int n[3], int nb) {
+  const int el = n[0] * n[1];
+  return el <= rect_elements(P4_NT) &&
+         (el > rect_elements(P4_NT / 2) || (long)nb * n[2] <= PROJ_FEW_PLANES);
+}
+
 void fft3_rect_local_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream, int sweep,
-                                 bool fwd_next) {
+                                 bool fwd_next, const project_expand_args *proj) {
   if (sweep < 0 || sweep == 0) rect_z(a, n[2], RECT_Z_FWD, stream);
-  if (sweep < 0 || sweep == 1) rect_xy_launch<false>(a, n, stream);
+  if ((sweep < 0 || sweep == 1) && proj) {
+    const int ntile = (proj->nbc + P4_BANDS - 1) / P4_BANDS, np = ntile * a.nproj;
+    const size_t lds = rect_xy_lds(n) > P4_BLOCK_LDS ? rect_xy_lds(n) : P4_BLOCK_LDS;
+    hipLaunchKernelGGL(rect_xy_proj_kernel, dim3((unsigned)((long)a.nb * n[2] + np)), dim3(P4_NT),
+                       lds, stream, a, n[2], *proj, ntile, np);
+    INQAMD_HIP_CHECK(hipGetLastError());
+  } else if (sweep < 0 || sweep == 1) {
+    rect_xy_launch<false>(a, n, stream);
+  }
   if (sweep < 0 || sweep == 2)
     rect_z(a, n[2],
            a.acc1 ? (fwd_next ? RECT_Z_BWD_ACC_FWD : RECT_Z_BWD_ACC)

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "fft3_rect.hpp"
+#include "projector_dev.hpp"
 
 namespace inqamd {
 
@@ -12,7 +13,13 @@ __global__ __launch_bounds__(z_threads(R0 * R1 * R2)) void rect_z_fwd_kernel(con
   extern __shared__ cplx lds[];
   constexpr int TB = Z_COLS / RECT_TY;
   // (the potential form shares V and the ownership words over a pair's band tiles)
-  const long t = POT || a.xcd ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
+  const int nbt = (a.nb + TB - 1) / TB;
+  const long tiles = (long)a.nx * ((a.ny + RECT_TY - 1) / RECT_TY) * nbt;
+  if (blockIdx.x >= tiles) {
+    phase_block(a, (int)(blockIdx.x - tiles));
+    return;
+  }
+  const long t = POT || a.xcd ? xcd_tile(blockIdx.x, tiles, nbt) : (long)blockIdx.x;
   z_fwd_tile<R0, R1, R2, RECT_TY, z_threads(R0 * R1 * R2), POT, true>(a, t, lds);
 }
 
@@ -77,7 +84,8 @@ static void rect_z_run(const fft3_args &a, rect_z_kernel k, hipStream_t stream) 
   if (prep || k == RECT_Z_BWD_FWD) rect_z_bwd<R0, R1, R2, false, true>(a, stream, prep);
   if (prep || k == RECT_Z_BWD_ACC_FWD) rect_z_bwd<R0, R1, R2, true, true>(a, stream, prep);
   if (k == RECT_Z_FWD)
-    hipLaunchKernelGGL((rect_z_fwd_kernel<R0, R1, R2, false>), dim3((unsigned)tiles),
+    hipLaunchKernelGGL((rect_z_fwd_kernel<R0, R1, R2, false>),
+                       dim3((unsigned)(tiles + phase_blocks(a, z_threads(L)))),
                        dim3(z_threads(L)), zl, stream, a);
   if (k == RECT_Z_POT)
     hipLaunchKernelGGL((rect_z_fwd_kernel<R0, R1, R2, true>), dim3((unsigned)tiles),

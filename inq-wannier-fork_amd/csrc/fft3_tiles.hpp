@@ -23,6 +23,18 @@
 
 namespace inqamd {
 
+// Longest planes whose launch may carry the projector, and the planes of a launch
+// up to which shorter ones do (a few per CU)
+constexpr int PROJ_MAX_LEN = 64;
+constexpr long PROJ_FEW_PLANES = 2048;
+
+// Extra workgroups of a z forward launch for the phases of the call
+inline unsigned phase_blocks(const fft3_args &a, int threads) {
+  if (!a.phase.pos) return 0;
+  const int n = a.phase.nsph > a.phase.nent ? a.phase.nsph : a.phase.nent;
+  return (unsigned)((n + threads - 1) / threads);
+}
+
 constexpr int Z_COLS = 64;  // FFT columns per z tile: TY y values x TB bands
 constexpr int Z_NT = 512;
 
@@ -861,7 +873,7 @@ constexpr int z_bwd_threads(int L, bool taylor) {
 
 // Work items of a band chunk of nb bands (tiles of ZC columns)
 template <int Z_TY, int ZC = Z_COLS>
-inline long z_tiles(int L, int nb) {
+__host__ __device__ inline long z_tiles(int L, int nb) {
   constexpr int Z_TB = ZC / Z_TY;
   return (long)L * ((L + Z_TY - 1) / Z_TY) * ((nb + Z_TB - 1) / Z_TB);
 }

@@ -332,11 +332,14 @@ static void hpsi_projector(handle &h, const cplx *psi, long ld, int nst) {
 // The local part T + V on the bands [b0, b0 + nb) of psi (pointers already
 // offset to b0).  The three-sweep path also adds the projector apply and the
 // Taylor accumulations `acc` (offset to b0) in its last sweep; the pencil
-// path leaves both to the caller.
+// path leaves both to the caller.  Three-sweep only: `pa`, the chunk's projector
+// coefficients beside the x-y planes, and `phases`, the call's phases beside the
+// z forward tiles.
 static void local_passes(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld, int nb,
                          int slot, int b0, long ldP, const taylor_acc *acc, int sweep = -1,
                          hipStream_t stream = nullptr, cplx *W = nullptr, int gskip = 0,
-                         int glog = 0, bool fwd_next = false, bool skip_store = false) {
+                         int glog = 0, bool fwd_next = false, bool skip_store = false,
+                         const project_expand_args *pa = nullptr, bool phases = false) {
   if (h.three_sweep) {
     fft3_args a{};
     a.gskip = gskip;
@@ -399,6 +402,9 @@ static void local_passes(handle &h, const cplx *psi, long ld, cplx *hpsi, long h
       a.gdump = acc->gdump + (size_t)b0 * h.npoint;
     }
     a.skip_store = skip_store ? 1 : 0;
+    a.nproj = t.nproj;
+    if (phases)
+      a.phase = {t.pos, t.uent, t.nproj * t.max_sphere, t.nent, t.phase_sph, t.phase_ent};
     // Rows of a whole number of 128-byte lines keep the natural order where it
     // is the faster one; others are dealt per XCD everywhere: each band tile of
     // such a row shares its first and last line with its neighbours, and the
@@ -408,9 +414,9 @@ static void local_passes(handle &h, const cplx *psi, long ld, cplx *hpsi, long h
     a.z_ty = h.tune_z_ty;
     a.xy_wide = h.tune_xy_wide;
     if (h.rect)
-      fft3_rect_local_hamiltonian(a, h.n, stream ? stream : h.stream, sweep, fwd_next);
+      fft3_rect_local_hamiltonian(a, h.n, stream ? stream : h.stream, sweep, fwd_next, pa);
     else
-      fft3_local_hamiltonian(a, h.n[0], stream ? stream : h.stream, sweep, fwd_next);
+      fft3_local_hamiltonian(a, h.n[0], stream ? stream : h.stream, sweep, fwd_next, pa);
     return;
   }
   cplx *w = h.work;
@@ -518,6 +524,32 @@ void hamiltonian_apply(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld
     return !(e && atoi(e) == 0);
   }();
   const bool two = pipeline && h.three_sweep && h.aux && two_slots(h, plan);
+  const int gs = plan.gskip;  // 0 unless three-sweep
+  if (h.three_sweep && projector_beside_planes(h, nst)) {
+    // each chunk's coefficients ride with its x-y planes; the phases with the z
+    // forward tiles when there is one chunk
+    const bool ph = plan.n == 1;
+    if (!ph) projector_phases(h, slot);
+    if (two) {
+      INQAMD_HIP_CHECK(hipEventRecord(h.ev_fork, h.stream));
+      INQAMD_HIP_CHECK(hipStreamWaitEvent(h.aux, h.ev_fork, 0));
+    }
+    for (int c = 0; c < plan.n; c++) {
+      const int b0 = plan.b0(c), nb = plan.nb(c);
+      hipStream_t s = two && (c & 1) ? h.aux : h.stream;
+      cplx *W = two ? h.work + (size_t)(c & 1) * chunk * h.npoint : h.work;
+      const project_expand_args pa =
+          projector_chunk_args(h, psi + b0, ld, nst, b0, nb, gs, plan.glog);
+      for (int sweep = 0; sweep < 3; sweep++)
+        local_passes(h, psi + b0, ld, hpsi + b0, hld, nb, slot, b0, nst, acc, sweep, s, W, gs,
+                     plan.glog, false, false, sweep == 1 ? &pa : nullptr, ph && sweep == 0);
+    }
+    if (two) {
+      INQAMD_HIP_CHECK(hipEventRecord(h.ev_join, h.aux));
+      INQAMD_HIP_CHECK(hipStreamWaitEvent(h.stream, h.ev_join, 0));
+    }
+    return;
+  }
   bool overlap = false;
   if (two) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -541,7 +573,6 @@ void hamiltonian_apply(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld
     projector_project_expand(h, psi, ld, nst, nullptr, 0, true);
   if (overlap) INQAMD_HIP_CHECK(hipEventRecord(h.ev_proj, h.stream));
   if (two && !overlap) fork();
-  const int gs = plan.gskip;  // 0 unless three-sweep
   bool waited[3] = {true, false, false};  // the main stream runs after the projector
   for (int c = 0; c < plan.n; c++) {
     const int b0 = plan.b0(c), nb = plan.nb(c);
@@ -646,7 +677,8 @@ void copy(handle &h, const cplx *x, long xld, cplx *y, long yld, int nst) {
 // n = 1..order, H^n in = H (H^{n-1} in) with p1 += c1_n H^n in (p1 = in + c1_1
 // H in when init1) and p2 += c2_n H^n in, c_n = z^n / n!.  Run
 // band chunk by band chunk with every order of a chunk on one stream: the
-// projector takes the chunk's bands of H^{n-1} in, and each order's last
+// projector takes the chunk's bands of H^{n-1} in (beside its x-y planes where
+// projector_beside_planes), and each order's last
 // sweep also transforms its output forward in z into W for the next order,
 // so no z_fwd sweep reads H^n in back (16 B per point and band per order).
 // Chunks alternate between two streams.
@@ -697,7 +729,9 @@ void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int s
   }();
   const bool two = pipeline && h.aux && two_slots(h, plan);
   const bool proj = h.pt.nproj > 0 && h.pt.nunique > 0;
-  projector_phases(h, slot);
+  const bool beside = proj && projector_beside_planes(h, nst);
+  const bool ph = beside && plan.n == 1;  // the phases with the first z forward tiles
+  if (!ph) projector_phases(h, slot);
   if (two) {
     INQAMD_HIP_CHECK(hipEventRecord(h.ev_fork, h.stream));
     INQAMD_HIP_CHECK(hipStreamWaitEvent(h.aux, h.ev_fork, 0));
@@ -718,7 +752,10 @@ void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int s
       auto power = [&](int m) { return outs && outs[m - 1] ? outs[m - 1] : buf[(m - 1) % 3]; };
       cplx *dst = power(n) + b0;
       const bool keep = n < order || (outs && outs[n - 1]);
-      if (proj)
+      project_expand_args pa;
+      if (beside)
+        pa = projector_chunk_args(h, src, sld, nst, b0, nb, plan.gskip, plan.glog);
+      else if (proj)
         projector_project_p4_chunk(h, src, sld, nst, b0, nb, plan.gskip, plan.glog, s,
                                    two ? (c & 1) : 0);
       taylor_acc acc;
@@ -743,8 +780,9 @@ void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int s
       acc.gdump = dumps ? dumps[n - 1] : nullptr;
       if (n == 1)
         local_passes(h, src, sld, dst, nst, nb, slot, b0, nst, &acc, 0, s, W, plan.gskip,
-                     plan.glog);
-      local_passes(h, src, sld, dst, nst, nb, slot, b0, nst, &acc, 1, s, W, plan.gskip, plan.glog);
+                     plan.glog, false, false, nullptr, ph);
+      local_passes(h, src, sld, dst, nst, nb, slot, b0, nst, &acc, 1, s, W, plan.gskip, plan.glog,
+                   false, false, beside ? &pa : nullptr);
       local_passes(h, src, sld, dst, nst, nb, slot, b0, nst, &acc, 2, s, W, plan.gskip, plan.glog,
                    n < order, !keep);
       src = dst;

@@ -179,6 +179,13 @@ void projector_project_p4(handle &h, const cplx *psi, long ld, int nst);
 // its point-chunked form uses; concurrent calls take different slots)
 void projector_project_p4_chunk(handle &h, const cplx *psi, long ld, int nst, int b0, int nb,
                                 int gskip, int glog, hipStream_t stream, int part_slot);
+// The arguments of that call, for a sweep that computes the coefficients itself
+project_expand_args projector_chunk_args(const handle &h, const cplx *psi, long ld, int nst, int b0,
+                                         int nb, int gskip, int glog);
+// 16-band tiles of all spheres below which the coefficients are split over
+// points, or computed beside the x-y planes (projector_beside_planes)
+constexpr long PROJ_FEW_TILES = 512;
+bool projector_beside_planes(const handle &h, int nst);
 void mfma4_selftest(double *out_device, hipStream_t stream);
 
 // hamiltonian.hip

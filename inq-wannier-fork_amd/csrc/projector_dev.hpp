@@ -27,6 +27,12 @@ __device__ __forceinline__ void phase_item(const float *pos, const int *uent, in
   }
 }
 
+// Workgroup `block` of the phases that a sweep's launch carries
+__device__ __forceinline__ void phase_block(const fft3_args &a, int block) {
+  phase_item(a.phase.pos, a.phase.uent, a.phase.nsph, a.phase.nent, a.kA, a.phase.sph,
+             a.phase.ent, block * (int)blockDim.x + (int)threadIdx.x);
+}
+
 // Nonlocal projector on the FP64 matrix cores (v_mfma_f64_16x16x4f64).
 //
 // One workgroup per (sphere p, tile of 8 bands = 16 real columns):
@@ -362,6 +368,21 @@ __device__ __forceinline__ void p4_store(const project_expand_args &a, int p, in
       a.P[((long)p * a.max_nlm + lm) * a.nst + b] = mk(d * sum[2 * t], d * sum[2 * t + 1]);
     }
   }
+}
+
+// The coefficients of sphere and 16-band tile `block` (sphere block / ntile) by
+// one workgroup of P4_NT threads, in the LDS that its kernel lends
+// (P4_BLOCK_LDS bytes)
+constexpr size_t P4_BLOCK_LDS = (P4_WAVES * 128 + 128) * sizeof(double);
+
+__device__ __forceinline__ void p4_block(const project_expand_args &a, int block, int ntile,
+                                         void *lds) {
+  auto *red = reinterpret_cast<double(*)[1][64][2]>(lds);
+  double *sum = reinterpret_cast<double *>(lds) + P4_WAVES * 128;
+  const int p = block / ntile, b0 = (block - p * ntile) * P4_BANDS;
+  gemm1_p4_points<1>(a, p, b0, 0, a.size[p], red, sum);
+  __syncthreads();
+  p4_store<1>(a, p, b0, sum);
 }
 
 }  // namespace inqamd

@@ -142,10 +142,9 @@ void projector_project_p4(handle &h, const cplx *psi, long ld, int nst) {
   projector_project_p4_chunk(h, psi, ld, nst, 0, nst, 0, 0, h.stream, 0);
 }
 
-void projector_project_p4_chunk(handle &h, const cplx *psi, long ld, int nst, int b0, int nb,
-                                int gskip, int glog, hipStream_t stream, int part_slot) {
+project_expand_args projector_chunk_args(const handle &h, const cplx *psi, long ld, int nst, int b0,
+                                         int nb, int gskip, int glog) {
   const projector_tables &t = h.pt;
-  if (t.nproj == 0) return;
   project_expand_args a{};
   a.psi = psi;
   a.ld = ld;
@@ -164,6 +163,31 @@ void projector_project_p4_chunk(handle &h, const cplx *psi, long ld, int nst, in
   a.gskip = gskip;
   a.glog = glog;
   a.pband0 = b0;
+  return a;
+}
+
+// Few (sphere, band tile) pairs leave the projector's launch nearly empty and
+// bound by its chain of gathers (9 us for 8 spheres x 16 bands, 3 more for the
+// sum of its point chunks), so it runs in workgroups ahead of the x-y planes of
+// the same launch, which need nothing from it and which it needs nothing from.
+// One workgroup then takes all the points of its sphere (no partial tiles).
+// Decided by all nst bands, so that a band's coefficients are the same bits
+// whichever chunk and path computes them.  With the phases beside the z forward
+// tiles, Hpsi of 32^3 x 16 bands takes three launches instead of six: 37.6 -> 30.0
+// us; 24^3 x 8 29.4 -> 22.5, 48^3 x 64 190 -> 177, 25 x 45 x 27 x 45 64 -> 54; ETRS
+// step of 30^3 x 14 296 -> 240, adjoint of 10 steps at 32^3 x 16 11.3 -> 9.7 ms.
+bool projector_beside_planes(const handle &h, int nst) {
+  if (!vnl_from_coefficients(h)) return false;
+  const long tiles = (long)((nst + P4_BANDS - 1) / P4_BANDS) * h.pt.nproj;
+  if (tiles >= PROJ_FEW_TILES) return false;
+  return h.rect ? fft3_rect_projector(h.n, nst) : fft3_projector(h.n[0], nst, h.tune_xy_wide);
+}
+
+void projector_project_p4_chunk(handle &h, const cplx *psi, long ld, int nst, int b0, int nb,
+                                int gskip, int glog, hipStream_t stream, int part_slot) {
+  const projector_tables &t = h.pt;
+  if (t.nproj == 0) return;
+  const project_expand_args a = projector_chunk_args(h, psi, ld, nst, b0, nb, gskip, glog);
   INQAMD_REQUIRE(t.max_nlm <= 4, "the 4x4x4 projector needs max_nlm <= 4");
   INQAMD_REQUIRE(part_slot >= 0 && part_slot < PROJ_PART_SLOTS, "projector partial slot");
   const long slot_doubles = PROJ_PART_TILES * 256 / PROJ_PART_SLOTS;
@@ -189,7 +213,7 @@ static void project_p4_launch(handle &h, const project_expand_args &a, int nst, 
   const int nbt = (nst + P4_BANDS - 1) / P4_BANDS;
   const long tiles = (long)((nst_all + P4_BANDS - 1) / P4_BANDS) * t.nproj;
   int nc = 1;
-  if (tiles < 512 && part) {
+  if (tiles < PROJ_FEW_TILES && part) {
     nc = (int)((1024 + tiles - 1) / tiles);
     const int by_points = t.max_sphere / 256 > 1 ? t.max_sphere / 256 : 1;
     if (nc > by_points) nc = by_points;
