@@ -1,6 +1,7 @@
 // Hamiltonian handle, Hpsi, transforms, reductions and the Taylor/ETRS
 // propagator, exported through the C ABI of include/inq_amd.h.
 
+#include "fields.hpp"
 #include "internal.hpp"
 #include "inq_amd.h"
 
@@ -314,6 +315,14 @@ void fft3d(handle &h, const cplx *in, long in_ld, cplx *out, long out_ld, int ns
   fft_launch_pass(pass_args(h, 0, in, in_ld, out, out_ld, nst, sign, 1.0), FFT_PLAIN, h.stream);
   fft_launch_pass(pass_args(h, 1, out, out_ld, out, out_ld, nst, sign, 1.0), FFT_PLAIN, h.stream);
   fft_launch_pass(pass_args(h, 2, out, out_ld, out, out_ld, nst, sign, scale), FFT_PLAIN, h.stream);
+}
+
+// The y transforms of nf consecutive [x][y][z] fields, in place: one pass over nf
+// times the x rows
+void fft_y_pass(handle &h, cplx *c, int nf, int sign) {
+  fft_pass_args a = pass_args(h, 1, c, 1, c, 1, 1, sign, 1.0);
+  a.c2 *= nf;
+  fft_launch_pass(a, FFT_PLAIN, h.stream);
 }
 
 // The projector step of the three-sweep Hpsi (after projector_phases).  Where

@@ -13,8 +13,10 @@
 #include <complex>
 #include <vector>
 
+#include "fields.hpp"
 #include "internal.hpp"
 #include "inq_amd.h"
+#include "xc_point.hpp"
 
 namespace inqamd {
 
@@ -31,7 +33,9 @@ struct td_state {
   double *rho = nullptr, *rho_old = nullptr, *vh = nullptr, *vxc = nullptr;  // [N]
   double *occ = nullptr;       // [max_bands]
   double *red = nullptr;       // [TD_RED_BLOCKS][4] partial sums + [4] totals
-  cplx *cf = nullptr;          // [N] complex Poisson work
+  cplx *cf = nullptr;          // [N] complex work: a field's transforms
+  cplx *cg = nullptr;          // [N] more of it
+  double *fred = nullptr;      // [2][field_partials] sums of the fused passes + [FIELD_SUMS]
   cplx *save = nullptr;        // [N][max_bands] the ETRS half step
   cplx *g3 = nullptr;          // [N][3] density gradient / GGA flux (spectral)
 };
@@ -59,6 +63,10 @@ void ensure_fields(handle &h) {
   t.occ = (double *)dalloc((size_t)h.max_bands * sizeof(double));
   t.red = (double *)dalloc((size_t)(TD_RED_BLOCKS + 1) * 4 * sizeof(double));
   t.cf = (cplx *)dalloc((size_t)h.npoint * sizeof(cplx));
+  if (fields_supported(h)) {
+    t.cg = (cplx *)dalloc((size_t)h.npoint * sizeof(cplx));
+    t.fred = (double *)dalloc((size_t)(2 * field_partials(h) + FIELD_SUMS) * sizeof(double));
+  }
 }
 
 void ensure_gga(handle &h) {
@@ -163,52 +171,6 @@ __device__ void lda_point(double n, double &e, double &v) {
   v = vx + vc;
 }
 
-// PBE (Perdew, Burke, Ernzerhof 1996), one spin component: energy per
-// particle e, vn = d(n e)/dn and vs = d(n e)/dsigma (sigma = |grad n|^2);
-// the uniform-gas correlation is Perdew-Wang 1992 with libxc's LDA_C_PW_MOD
-// parameters, as GGA_C_PBE uses it.
-__device__ void pbe_exchange(double n, double sigma, double &e, double &vn, double &vs) {
-  const double kappa = 0.8040, mu = 0.2195149727645171;
-  const double ax = -0.75 * cbrt(3.0 / M_PI);
-  const double n13 = cbrt(n);
-  const double n83 = n13 * n13 * n * n;                                // n^(8/3)
-  const double c = 4.0 * pow(3.0 * M_PI * M_PI, 2.0 / 3.0);
-  const double x = sigma / (c * n83);                                  // s^2
-  const double den = 1.0 + mu * x / kappa;
-  const double F = 1.0 + kappa - kappa / den, dF = mu / (den * den);
-  e = ax * n13 * F;
-  vn = ax * n13 * ((4.0 / 3.0) * F - (8.0 / 3.0) * x * dF);
-  vs = ax * n13 * n * dF / (c * n83);
-}
-
-__device__ void pbe_correlation(double n, double sigma, double &e, double &vn, double &vs) {
-  const double beta = 0.06672455060314922, gamma = (1.0 - M_LN2) / (M_PI * M_PI);
-  const double A0 = 0.0310907, a1 = 0.21370, b1 = 7.5957, b2 = 3.5876, b3 = 1.6382,
-               b4 = 0.49294;
-  const double rs = cbrt(3.0 / (4.0 * M_PI * n)), sq = sqrt(rs);
-  const double q0 = -2.0 * A0 * (1.0 + a1 * rs);
-  const double q1 = 2.0 * A0 * (b1 * sq + b2 * rs + b3 * rs * sq + b4 * rs * rs);
-  const double q1p = A0 * (b1 / sq + 2.0 * b2 + 3.0 * b3 * sq + 4.0 * b4 * rs);
-  const double lg = log(1.0 + 1.0 / q1);
-  const double ec = q0 * lg;
-  const double dec = (-2.0 * A0 * a1 * lg - q0 * q1p / (q1 * q1 + q1)) * (-rs / (3.0 * n));
-  const double kf = cbrt(3.0 * M_PI * M_PI * n);
-  const double ty = M_PI / (16.0 * kf * n * n);  // t^2 / sigma
-  const double y = sigma * ty;
-  const double ex = exp(-ec / gamma);
-  const double A = (beta / gamma) / (ex - 1.0);
-  const double dA = (beta / (gamma * gamma)) * ex / ((ex - 1.0) * (ex - 1.0));
-  const double P = 1.0 + A * y, D = 1.0 + A * y + A * A * y * y;
-  const double N = (beta / gamma) * y * P / D;
-  const double H = gamma * log(1.0 + N);
-  const double dNy = (beta / gamma) * ((P + A * y) * D - y * P * (A + 2.0 * A * A * y)) / (D * D);
-  const double dNA = (beta / gamma) * y * (y * D - P * (y + 2.0 * A * y * y)) / (D * D);
-  const double g = gamma / (1.0 + N);
-  e = ec + H;
-  vn = e + n * (dec + g * dNA * dA * dec - g * dNy * (7.0 / 3.0) * y / n);
-  vs = n * g * dNy * ty;
-}
-
 // i G_d f(G) / N into g3[p][d] (operations::gradient in Fourier space)
 __global__ __launch_bounds__(256) void grad_spec_kernel(const cplx *__restrict__ f, int n0, int n1,
                                                         int n2, double b0, double b1, double b2,
@@ -309,18 +271,8 @@ __global__ __launch_bounds__(256) void gga_point_kernel(const double *__restrict
     const double n = r < 0.0 ? 0.0 : r;
     const double gx = g3[p * 3].x, gy = g3[p * 3 + 1].x, gz = g3[p * 3 + 2].x;
     const double sigma = gx * gx + gy * gy + gz * gz;
-    double e = 0.0, vn = 0.0, vs = 0.0;
-    if (n >= 1e-15) {
-      double e1, v1, s1;
-      if (which & 1) {
-        pbe_exchange(n, sigma, e1, v1, s1);
-        e += e1, vn += v1, vs += s1;
-      }
-      if (which & 2) {
-        pbe_correlation(n, sigma, e1, v1, s1);
-        e += e1, vn += v1, vs += s1;
-      }
-    }
+    double e, vn, vs;
+    gga_point(n, sigma, which, e, vn, vs);
     vxc[p] = vn;
     g3[p * 3] = mk(-2.0 * vs * gx, 0.0);
     g3[p * 3 + 1] = mk(-2.0 * vs * gy, 0.0);
@@ -407,17 +359,45 @@ unsigned red_blocks(long n) {
   return (unsigned)(b > TD_RED_BLOCKS ? TD_RED_BLOCKS : b);
 }
 
+// a block_sums4 kernel into the partial sums; returns its blocks
+template <typename K, typename... A>
+unsigned launch_sums4(handle &h, long n, K kernel, A... args) {
+  const unsigned nb = red_blocks(n);
+  hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, h.stream, args..., state(h).red);
+  check_launch();
+  return nb;
+}
+
 // run a block_sums4 kernel, then its fixed-order total; copy the 4 totals to host
 template <typename K, typename... A>
 void reduce4(handle &h, long n, double out[4], K kernel, A... args) {
   td_state &t = state(h);
-  const unsigned nb = red_blocks(n);
-  hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, h.stream, args..., t.red);
-  check_launch();
+  const unsigned nb = launch_sums4(h, n, kernel, args...);
   hipLaunchKernelGGL(final_sums4, dim3(1), dim3(256), 0, h.stream, t.red, (int)nb);
   check_launch();
   INQAMD_HIP_CHECK(hipMemcpyAsync(out, t.red + (long)TD_RED_BLOCKS * 4, 4 * sizeof(double),
                                   hipMemcpyDeviceToHost, h.stream));
+  INQAMD_HIP_CHECK(hipStreamSynchronize(h.stream));
+}
+
+// Totals of the fused passes' sums, and of the first two of a block_sums4
+// kernel's nb4 blocks, in one copy: {e n, rho vxc, value 0, value 1}
+void field_totals_to_host(handle &h, bool gga, unsigned nb4, double out[FIELD_SUMS]) {
+  td_state &t = state(h);
+  const long nf = field_partials(h);
+  double *tot = t.fred + 2 * nf;
+  field_sum_rows r{};
+  for (int k = 0; k < 2; k++) {
+    r.part[k] = t.fred + k * nf;
+    r.n[k] = gga ? (int)nf : 0;
+    r.stride[k] = 1;
+    r.part[2 + k] = t.red + k;
+    r.n[2 + k] = (int)nb4;
+    r.stride[2 + k] = 4;
+  }
+  field_sums(h, r, FIELD_SUMS, tot);
+  INQAMD_HIP_CHECK(hipMemcpyAsync(out, tot, FIELD_SUMS * sizeof(double), hipMemcpyDeviceToHost,
+                                  h.stream));
   INQAMD_HIP_CHECK(hipStreamSynchronize(h.stream));
 }
 
@@ -432,6 +412,11 @@ void density(handle &h, const cplx *psi, long ld, int nst, const double *occ_dev
 void poisson(handle &h, const double *rho, double *vh) {
   ensure_fields(h);
   td_state &t = state(h);
+  if (fields_supported(h)) {
+    field_forward_xy(h, rho, t.cf);
+    field_hartree(h, t.cf, t.cg, vh);
+    return;
+  }
   hipLaunchKernelGGL(real_to_complex, dim3(grid1(h.npoint)), dim3(256), 0, h.stream, rho,
                      h.npoint, t.cf);
   check_launch();
@@ -474,6 +459,15 @@ void gga_xc(handle &h, const double *rho, int which, double *vxc, double *exc, d
   td_state &t = state(h);
   const double dV = h.volume / (double)h.npoint, inv_n = 1.0 / (double)h.npoint;
   const double *b = h.rlat;
+  if (fields_supported(h)) {
+    field_forward_xy(h, rho, t.cf);
+    field_gga(h, t.cf, t.g3, t.cg, rho, which, vxc, t.fred, t.fred + field_partials(h));
+    double s[FIELD_SUMS];
+    field_totals_to_host(h, true, 0, s);
+    *exc = dV * s[0];
+    *nvxc = dV * s[1];
+    return;
+  }
   hipLaunchKernelGGL(real_to_complex, dim3(grid1(h.npoint)), dim3(256), 0, h.stream, rho,
                      h.npoint, t.cf);
   check_launch();
@@ -523,6 +517,28 @@ void ks_potential(handle &h, const double *vion, const double *rho, bool hartree
   td_state &t = state(h);
   const double dV = h.volume / (double)h.npoint;
   energies[2] = energies[3] = 0.0;
+  if (fields_supported(h) && xc != 1) {
+    // one forward transform of the density for both, one copy for all sums
+    if (hartree || xc) field_forward_xy(h, rho, t.cf);
+    if (hartree) field_hartree(h, t.cf, t.cg, t.vh);
+    if (xc) {
+      ensure_gga(h);
+      field_gga(h, t.cf, t.g3, t.cg, rho, 3, t.vxc, t.fred, t.fred + field_partials(h));
+    }
+    const unsigned nb =
+        launch_sums4(h, h.npoint, ks_kernel, vion, rho, hartree ? (const double *)t.vh : nullptr,
+                     xc ? (const double *)t.vxc : nullptr, h.npoint, h.V);
+    double s[FIELD_SUMS];
+    field_totals_to_host(h, xc != 0, nb, s);
+    h.generation++;
+    energies[0] = dV * s[2];
+    energies[1] = hartree ? 0.5 * dV * s[3] : 0.0;
+    if (xc) {
+      energies[2] = dV * s[0];
+      energies[3] = dV * s[1];
+    }
+    return;
+  }
   if (hartree) poisson(h, rho, t.vh);
   if (xc) xc_functional(h, rho, xc == 2 ? 5 : 2, t.vxc, &energies[2], &energies[3]);
   double s[4];
@@ -590,7 +606,7 @@ void td_release(handle &h) {
   td_state *t = static_cast<td_state *>(h.tddft);
   for (void *p : {(void *)t->rho, (void *)t->rho_old, (void *)t->vh, (void *)t->vxc,
                   (void *)t->occ, (void *)t->red, (void *)t->cf, (void *)t->save,
-                  (void *)t->g3})
+                  (void *)t->g3, (void *)t->cg, (void *)t->fred})
     if (p) (void)hipFree(p);
   delete t;
   h.tddft = nullptr;
