@@ -245,24 +245,25 @@ __global__ __launch_bounds__(64) void nl_pair_kernel(const cplx *mX, const cplx 
   if (threadIdx.x < 18) partial[(long)row * 18 + threadIdx.x] = red[threadIdx.x][0];
 }
 
-// out[k] = sum over rows of partial[row][k] (k < width), one 256-thread
-// block: thread t adds rows t, t + 256, ..., then a tree over the threads, a
-// fixed order.
+// out[k] = sum over rows of partial[row][k], k = blockIdx.x < width: thread t adds
+// rows t, t + 256, ..., then a butterfly per wave and the waves in order, a fixed
+// order.  (One workgroup for all columns in turn took 13.7 us for 1024 rows of 8
+// and for 112 of 18, all of it the latency of its barriers: density, dipole,
+// energies and current of 36 x 36 x 90 x 48 bands 563 -> 539 us.)
 constexpr int SUM_ROWS_NT = 256;
 __global__ __launch_bounds__(SUM_ROWS_NT) void sum_rows_kernel(const double *partial, int nrows,
                                                                int width, double *out) {
-  __shared__ double red[SUM_ROWS_NT];
-  for (int k = 0; k < width; k++) {
-    double s = 0.0;
-    for (int r = threadIdx.x; r < nrows; r += SUM_ROWS_NT) s += partial[(long)r * width + k];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = SUM_ROWS_NT / 2; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[k] = red[0];
-    __syncthreads();
+  __shared__ double red[SUM_ROWS_NT / 64];
+  const int k = blockIdx.x;
+  double s = 0.0;
+  for (int r = threadIdx.x; r < nrows; r += SUM_ROWS_NT) s += partial[(long)r * width + k];
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) s += __shfl_xor(s, w, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < SUM_ROWS_NT / 64; w++) s += red[w];
+    out[k] = s;
   }
 }
 
@@ -681,7 +682,7 @@ static void gspace_record(handle &h, const cplx *Xh, const cplx *Yh, long ld, in
   hipLaunchKernelGGL(gspace_moments_kernel, dim3(OBS_GS_BLOCKS), dim3(256), 0, h.stream, Xh, Yh,
                      ld, nb, h.n[0], h.n[1], h.n[2], part);
   INQAMD_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(SUM_ROWS_NT), 0, h.stream,
+  hipLaunchKernelGGL(sum_rows_kernel, dim3(8), dim3(SUM_ROWS_NT), 0, h.stream,
                      (const double *)part, OBS_GS_BLOCKS, 8, rec);
   INQAMD_HIP_CHECK(hipGetLastError());
 }
@@ -698,7 +699,7 @@ static void nl_record(handle &h, const cplx *mX, const cplx *mY, int nb, double 
                        coeff, t.max_nlm, nb, part);
     INQAMD_HIP_CHECK(hipGetLastError());
   }
-  hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(SUM_ROWS_NT), 0, h.stream,
+  hipLaunchKernelGGL(sum_rows_kernel, dim3(18), dim3(SUM_ROWS_NT), 0, h.stream,
                      (const double *)part, nrows, 18, rec + 8);
   INQAMD_HIP_CHECK(hipGetLastError());
 }
@@ -989,14 +990,14 @@ void adjoint_half_fused(inqamd_td *td, int nb, cplx *const *Y, int slot, double 
     }
     INQAMD_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(SUM_ROWS_NT), 0, h.stream,
-                       (const double *)part, OBS_GS_BLOCKS, 1, rec);
+                     (const double *)part, OBS_GS_BLOCKS, 1, rec);
     INQAMD_HIP_CHECK(hipGetLastError());
   }
   // projector part of dL/ds from sphere moments of A_k and Y_j
   const projector_tables &t = h.pt;
   const int nrows = t.nproj * t.max_nlm;
   if (nrows > 0) {
-    projector_phases(h, slot);
+    // (the phases of this slot are those of the H applications above)
     double L[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     lattice_dot(h, td->d.direction, L);
     sphere_moments_multi(h, A, M, nb, nb, L, false, td->momA, td->mom_stride);
@@ -1006,7 +1007,7 @@ void adjoint_half_fused(inqamd_td *td, int nb, cplx *const *Y, int slot, double 
                        (const double *)t.coeff, nb, E, part);
     INQAMD_HIP_CHECK(hipGetLastError());
   }
-  hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(SUM_ROWS_NT), 0, h.stream,
+  hipLaunchKernelGGL(sum_rows_kernel, dim3(2), dim3(SUM_ROWS_NT), 0, h.stream,
                      (const double *)part, nrows, 2, rec + 1);
   INQAMD_HIP_CHECK(hipGetLastError());
   grad_fused_args ga;
