@@ -177,14 +177,19 @@ __device__ __forceinline__ void rect_xy_plane(const fft3_args &a, int nz, long p
 #undef INQAMD_RECT_CASE
   }
   if constexpr (FWD) {
-    auto wy = [&](int i, int c, cplx v) { W[c * ny + i] = v; };
+    // (back into LDS and out in order, as in the cubic planes)
     switch (ny) {
 #define INQAMD_RECT_CASE(L, R0, R1, R2)                                                   \
   case L:                                                                                \
-    rect_axis<R0, R1, R2, NT, true, false>(ky, a.twy, -1, ly, ly, sy, wy);               \
+    rect_axis<R0, R1, R2, NT, true, true>(ky, a.twy, -1, ly, ly, sy, sy);                \
     break;
       INQAMD_RECT_XY(INQAMD_RECT_CASE)
 #undef INQAMD_RECT_CASE
+    }
+    for (int e = threadIdx.x; e < nx * ny; e += NT) {
+      int x, y;
+      kx.split(e, x, y);
+      W[e] = lds[x * pad + y];
     }
   } else {
     // 1/2 |G + k + A|^2 with G = m_x b0 + m_y b1 + m_z b2 (cartesian)

@@ -392,9 +392,12 @@ __device__ __forceinline__ void xy_fwd_plane(const fft3_args &a, long plane, cpl
   auto sx = [&](int i, int c, cplx v, int, int) { lds[i * PAD + c] = v; };
   auto ly = [&](int i, int c) -> cplx { return lds[c * PAD + i]; };    // (i = y, c = x)
   auto sy = [&](int i, int c, cplx v, int, int) { lds[c * PAD + i] = v; };
-  auto wy = [&](int i, int c, cplx v, int, int) { W[c * L + i] = v; };
   run_plan<P, X0, X1, X2, L, NT>(a.tw, -1, false, gx, lx, sx, sx, true);  // x forward
-  run_plan<P, X0, X1, X2, L, NT>(a.tw, -1, true, ly, ly, sy, wy, false);  // y forward
+  // y forward back into LDS and out in order: from the last stage's registers a
+  // wave would write 16 bytes into each of 64 rows (the steepest descent at 64^3
+  // x 256 and its diagonalisation 59.9 ms so, 57.0 in order)
+  run_plan<P, X0, X1, X2, L, NT>(a.tw, -1, true, ly, ly, sy, sy, true);
+  for (int e = threadIdx.x; e < L * L; e += NT) W[e] = lds[e / L * PAD + e % L];
 }
 
 // ---------------------------------------------------------------------------
