@@ -169,7 +169,30 @@ struct fft3_args {
   // last sweep adds (fft3_fourier_hamiltonian)
   const cplx *kin_in;
   long kin_ld;
+  // and the partial sums of the line search over them (mm_phi == nullptr: none):
+  // for each (x, y rows) of the grid and band mm_band0 + b, the eight of
+  // line_sums over phi, kin_in and hpsi into mm_part[row][mm_nst][8]
+  const cplx *mm_phi;
+  long mm_ld;
+  double *mm_part;
+  int mm_nst, mm_band0;
 };
+
+// <r|r>, <f|r>, <r|h>, <f|h> (real, imaginary) of one element
+// (steepest_descent.hpp:47-51)
+__device__ __forceinline__ void line_sums(double *a, cplx f, cplx r, cplx h) {
+  a[0] += r.x * r.x + r.y * r.y;
+  a[1] += r.x * r.y - r.y * r.x;
+  a[2] += f.x * r.x + f.y * r.y;
+  a[3] += f.x * r.y - f.y * r.x;
+  a[4] += r.x * h.x + r.y * h.y;
+  a[5] += r.x * h.y - r.y * h.x;
+  a[6] += f.x * h.x + f.y * h.y;
+  a[7] += f.x * h.y - f.y * h.x;
+}
+
+// Rows of those partial sums
+inline long line_sum_rows(int nx, int ny) { return (long)nx * ((ny + 7) / 8); }
 
 // G-space Hpsi on the chunk's bands from psi = IFFT(phi) (INQ layout, `psi`)
 // and phi itself (`kin_in`): hpsi = FFT(V psi + V_nl psi) + 1/2 |G+k+A|^2 phi,

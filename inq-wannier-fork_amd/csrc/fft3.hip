@@ -110,14 +110,15 @@ __global__ __launch_bounds__(NT) void xy_fwd_kernel(const fft3_args a) {
   xy_fwd_plane<R0, R1, R2, NT>(a, blockIdx.x, lds);
 }
 
-template <int R0, int R1, int R2, int TY>
+template <int R0, int R1, int R2, int TY, bool MM>
 __global__ __launch_bounds__(z_threads(R0 * R1 * R2))
 __attribute__((amdgpu_waves_per_eu(z_bwd_waves(R0 * R1 * R2))))
 void z_kin_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
   constexpr int TB = Z_COLS / TY;
   const long t = a.xcd ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
-  z_bwd_epi_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2), false, true>(a, t, lds);
+  z_bwd_epi_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2), false, true, false, Z_COLS, false, MM>(
+      a, t, lds);
 }
 
 static int z_ty_choice() {
@@ -156,7 +157,8 @@ static void prepare3() {
   ensure_lds(xy_kin_kernel<R0, R1, R2, wide_threads(L)>, xy_kin_lds<R0, R1, R2>());
   if constexpr (L <= PROJ_MAX_LEN) ensure_lds(xy_proj_kernel<R0, R1, R2>, xy_proj_lds<R0, R1, R2>());
   ensure_lds(z_pot_kernel<R0, R1, R2, 8>, zl);
-  ensure_lds(z_kin_kernel<R0, R1, R2, 8>, zl);
+  ensure_lds(z_kin_kernel<R0, R1, R2, 8, false>, zl);
+  ensure_lds(z_kin_kernel<R0, R1, R2, 8, true>, zl);
   ensure_lds(xy_fwd_kernel<R0, R1, R2, wide_threads(L)>, pl);
   const size_t zbp = z_bwd_lds(L, z_bwd_cols(L, false)), zba = z_bwd_lds(L, z_bwd_cols(L, true));
   ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 8, false, false>, zbp);
@@ -245,8 +247,12 @@ static void launch_fourier(const fft3_args &a, hipStream_t stream) {
   hipLaunchKernelGGL((xy_fwd_kernel<R0, R1, R2, wide_threads(L)>), dim3((unsigned)((long)a.nb * L)),
                      dim3(wide_threads(L)), plds, stream, a);
   INQAMD_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL((z_kin_kernel<R0, R1, R2, 8>), dim3((unsigned)ztiles), dim3(z_threads(L)), zlds,
-                     stream, a);
+  if (a.mm_phi)
+    hipLaunchKernelGGL((z_kin_kernel<R0, R1, R2, 8, true>), dim3((unsigned)ztiles),
+                       dim3(z_threads(L)), zlds, stream, a);
+  else
+    hipLaunchKernelGGL((z_kin_kernel<R0, R1, R2, 8, false>), dim3((unsigned)ztiles),
+                       dim3(z_threads(L)), zlds, stream, a);
   INQAMD_HIP_CHECK(hipGetLastError());
 }
 

@@ -36,14 +36,14 @@ void rect_z_bwd_kernel(const fft3_args a) {
   z_bwd_epi_tile<R0, R1, R2, TY, z_bwd_threads(L, T), ACC, false, FWD, ZC, true>(a, t, lds);
 }
 
-template <int R0, int R1, int R2>
+template <int R0, int R1, int R2, bool MM>
 __global__ __launch_bounds__(z_threads(R0 * R1 * R2))
 __attribute__((amdgpu_waves_per_eu(z_bwd_waves(R0 * R1 * R2))))
 void rect_z_kin_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
   constexpr int TB = Z_COLS / RECT_TY;
   const long t = a.xcd ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
-  z_bwd_epi_tile<R0, R1, R2, RECT_TY, z_threads(R0 * R1 * R2), false, true, false, Z_COLS, true>(
+  z_bwd_epi_tile<R0, R1, R2, RECT_TY, z_threads(R0 * R1 * R2), false, true, false, Z_COLS, true, MM>(
       a, t, lds);
 }
 
@@ -77,7 +77,8 @@ static void rect_z_run(const fft3_args &a, rect_z_kernel k, hipStream_t stream) 
   if (prep) {
     rect_lds(rect_z_fwd_kernel<R0, R1, R2, false>, zl);
     rect_lds(rect_z_fwd_kernel<R0, R1, R2, true>, zl);
-    rect_lds(rect_z_kin_kernel<R0, R1, R2>, zl);
+    rect_lds(rect_z_kin_kernel<R0, R1, R2, false>, zl);
+    rect_lds(rect_z_kin_kernel<R0, R1, R2, true>, zl);
   }
   if (prep || k == RECT_Z_BWD) rect_z_bwd<R0, R1, R2, false, false>(a, stream, prep);
   if (prep || k == RECT_Z_BWD_ACC) rect_z_bwd<R0, R1, R2, true, false>(a, stream, prep);
@@ -90,8 +91,11 @@ static void rect_z_run(const fft3_args &a, rect_z_kernel k, hipStream_t stream) 
   if (k == RECT_Z_POT)
     hipLaunchKernelGGL((rect_z_fwd_kernel<R0, R1, R2, true>), dim3((unsigned)tiles),
                        dim3(z_threads(L)), zl, stream, a);
-  if (k == RECT_Z_KIN)
-    hipLaunchKernelGGL((rect_z_kin_kernel<R0, R1, R2>), dim3((unsigned)tiles),
+  if (k == RECT_Z_KIN && a.mm_phi)
+    hipLaunchKernelGGL((rect_z_kin_kernel<R0, R1, R2, true>), dim3((unsigned)tiles),
+                       dim3(z_threads(L)), zl, stream, a);
+  if (k == RECT_Z_KIN && !a.mm_phi)
+    hipLaunchKernelGGL((rect_z_kin_kernel<R0, R1, R2, false>), dim3((unsigned)tiles),
                        dim3(z_threads(L)), zl, stream, a);
   INQAMD_HIP_CHECK(hipGetLastError());
 }

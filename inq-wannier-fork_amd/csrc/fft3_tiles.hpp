@@ -520,8 +520,13 @@ __device__ __forceinline__ void vnl_expand_wave(const fft3_args &a, int gb0, con
 }
 
 // ZC: columns of the tile (TY y values x ZC / TY bands), 64 or 32
+// MM (G-space Hpsi): also the line search's partial sums of the tile, in place of
+// a pass over phi, the residual and H residual that read 48 bytes per point and
+// band (here phi alone is read again from memory, the residual from cache):
+// steepest descent at 40^3 x 48 bands 1869 -> 1824 us, at 64^3 x 256 (with the
+// diagonalisation) 57.1 -> 55.4 ms
 template <int R0, int R1, int R2, int Z_TY, int NT = Z_NT, bool ACC = false, bool GS = false,
-          bool FWD = false, int ZC = Z_COLS, bool RECT = false>
+          bool FWD = false, int ZC = Z_COLS, bool RECT = false, bool MM = false>
 __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx *lds) {
   using P = plan3<R0, R1, R2>;
   constexpr int L = P::LEN;
@@ -703,6 +708,53 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
     v.y += pre[k].y;
     return v;
   };
+  if constexpr (MM) {
+    static_assert(GS && Z_TY == 8 && ZC == 64, "the G-space write's tiles");
+    // hpsi and the sums over it: the residual (again: the prefetch was scaled)
+    // and phi of G outputs loaded together
+    constexpr int G = 4;
+    double s8[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k0 = 0; k0 < NE; k0 += G) {
+      cplx f[G], r[G];
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        const int k = k0 + g < NE ? k0 + g : NE - 1;
+        f[g] = a.mm_phi[(long)pk[k] * a.mm_ld + bk[k]];
+        r[g] = a.kin_in[(long)pk[k] * a.kin_ld + bk[k]];
+      }
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        const int k = k0 + g;
+        if (k < NE && vk[k < NE ? k : 0]) {
+          const int e = threadIdx.x + k * NT;
+          const cplx v = result(k, e % Z_TB, (e / Z_TB) % Z_TY, e / Z_COLS);
+          a.hpsi[(long)pk[k] * a.hld + bk[k]] = v;
+          line_sums(s8, f[g], r[g], v);
+        }
+      }
+    }
+    // a thread's outputs are all of band thread % 8: the lanes of a band by a
+    // butterfly, the waves in order through the tile's LDS
+    __syncthreads();
+    double *red = reinterpret_cast<double *>(lds);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int v = 0; v < 8; v++) {
+#pragma unroll
+      for (int w = Z_TB; w < 64; w <<= 1) s8[v] += __shfl_xor(s8[v], w, 64);
+      if (lane < Z_TB) red[(wave * Z_TB + lane) * 8 + v] = s8[v];
+    }
+    __syncthreads();
+    if (threadIdx.x < Z_TB * 8) {
+      const int b = threadIdx.x / 8, v = threadIdx.x % 8;
+      double t8 = red[threadIdx.x];
+      for (int w = 1; w < NT / 64; w++) t8 += red[w * Z_TB * 8 + threadIdx.x];
+      if (cb0 + b < a.nb)
+        a.mm_part[((long)(x * nyt + yt) * a.mm_nst + a.mm_band0 + gb0 + b) * 8 + v] = t8;
+    }
+    return;
+  }
   if constexpr (!ACC) {
 #pragma unroll
     for (int k = 0; k < NE; k++) {

@@ -13,7 +13,8 @@
 //           of the preconditioner sum 1/2|G|^2 |r|^2 and sum |r|^2
 //   pass 3  residual *= K(1/2|G|^2 / kinetic)
 //   H residual (G-space Hpsi)
-//   pass 4  <r|r>, <phi|r>, <r|Hr>, <phi|Hr> and the step lambda per band
+//   pass 4  <r|r>, <phi|r>, <r|Hr>, <phi|Hr> and the step lambda per band (on
+//           three-sweep grids in the sweep that writes H residual)
 //   pass 5  phi += lambda r, hphi += lambda Hr (with the next step's pass-1 sums)
 // orthogonalize forms S = dV Phi^H Phi (a split-K strided-batched ZGEMM),
 // factors it (S = R R^H, R lower: cholesky.hip) and applies Phi <- Phi R^-H
@@ -23,6 +24,7 @@
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
 
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstdlib>
@@ -86,11 +88,12 @@ gs_shape shape(const handle &h, int nst) {
 
 // Most partial sums (chunks x bands) of any nst <= max_bands: chunks of
 // GS_CHUNK, or GS_BLOCKS blocks of at most 64 bands (and a chunk cut short in
-// each band group)
+// each band group), or the rows of the line sums
 long most_partials(const handle &h) {
   const long full = (h.npoint + GS_CHUNK - 1) / GS_CHUNK * h.max_bands;
   const long split = (GS_BLOCKS + h.max_bands / 16 + 1) * 64;
-  return full > split ? full : split;
+  const long line = h.three_sweep ? line_sum_rows(h.n[0], h.n[1]) * h.max_bands : 0;
+  return std::max(full, std::max(split, line));
 }
 
 gs_state &state(handle &h) {
@@ -280,15 +283,7 @@ __global__ __launch_bounds__(256) void mm_partial(const cplx *__restrict__ phi, 
                                                   const cplx *__restrict__ hres, long rld, int nst,
                                                   long npoint, long chunk, double *part) {
   band_partials<8, BT>(npoint, chunk, nst, part, [&](long p, int b, double *a) {
-    const cplx f = phi[p * ld + b], r = res[p * rld + b], hr = hres[p * rld + b];
-    a[0] += r.x * r.x + r.y * r.y;
-    a[1] += r.x * r.y - r.y * r.x;
-    a[2] += f.x * r.x + f.y * r.y;
-    a[3] += f.x * r.y - f.y * r.x;
-    a[4] += r.x * hr.x + r.y * hr.y;
-    a[5] += r.x * hr.y - r.y * hr.x;
-    a[6] += f.x * hr.x + f.y * hr.y;
-    a[7] += f.x * hr.y - f.y * hr.x;
+    line_sums(a, phi[p * ld + b], res[p * rld + b], hres[p * rld + b]);
   });
 }
 
@@ -551,14 +546,18 @@ __global__ __launch_bounds__(256) void kinetic_partial(gspace geo, const cplx *_
 
 }  // namespace
 
-// ks_hamiltonian::operator() on fourier_space orbitals (ks_hamiltonian.hpp:
-// 156-176): to_real, the real-space operator, to_fourier.  Uses hn and hn2.
-void hamiltonian_fourier(handle &h, const cplx *phi, long ld, cplx *hphi, long hld, int nst) {
+static bool gspace_sweeps(const handle &h) {
   static const bool sweeps = [] {
     const char *e = getenv("INQAMD_GSPACE_SWEEPS");
     return !(e && atoi(e) == 0);
   }();
-  if (h.three_sweep && sweeps) {
+  return h.three_sweep && sweeps;
+}
+
+// ks_hamiltonian::operator() on fourier_space orbitals (ks_hamiltonian.hpp:
+// 156-176): to_real, the real-space operator, to_fourier.  Uses hn and hn2.
+void hamiltonian_fourier(handle &h, const cplx *phi, long ld, cplx *hphi, long hld, int nst) {
+  if (gspace_sweeps(h)) {
     hamiltonian_fourier_sweeps(h, phi, ld, hphi, hld, nst);
     return;
   }
@@ -630,10 +629,17 @@ void steepest_descent(handle &h, cplx *phi, long ld, int nst, bool precond) {
               (const cplx *)phi, ld, g.res, rl, (const double *)g.band, nst, h.npoint, rs.chunk,
               g.part);
     if (precond) precondition_apply(h, g.res, rl, nst);
-    hamiltonian_fourier(h, g.res, rl, g.hres, rl, nst);
-    GS_REDUCE(mm_partial, rs, h.stream, (const cplx *)phi, ld, (const cplx *)g.res,
-              (const cplx *)g.hres, rl, nst, h.npoint, rs.chunk, g.part);
-    hipLaunchKernelGGL(lambda_final, fg, dim3(256), 0, h.stream, (const double *)g.part, nchunk,
+    // H residual and pass 4, in one where the sweeps make H residual
+    long mm_rows = nchunk;
+    if (gspace_sweeps(h)) {
+      hamiltonian_fourier_sweeps(h, g.res, rl, g.hres, rl, nst, phi, ld, g.part);
+      mm_rows = line_sum_rows(h.n[0], h.n[1]);
+    } else {
+      hamiltonian_fourier(h, g.res, rl, g.hres, rl, nst);
+      GS_REDUCE(mm_partial, rs, h.stream, (const cplx *)phi, ld, (const cplx *)g.res,
+                (const cplx *)g.hres, rl, nst, h.npoint, rs.chunk, g.part);
+    }
+    hipLaunchKernelGGL(lambda_final, fg, dim3(256), 0, h.stream, (const double *)g.part, mm_rows,
                        nst, dV, g.band);
     check_launch();
     if (istep != num_steps - 1)

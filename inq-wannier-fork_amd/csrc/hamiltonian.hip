@@ -626,7 +626,7 @@ void hamiltonian_apply(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld
 // term).  The kinetic term acts on phi directly: the real-space
 // Hpsi followed by to_fourier would transform psi forward and back again.
 void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi, long hld,
-                                int nst) {
+                                int nst, const cplx *line, long line_ld, double *part) {
   fft3d(h, phi, ld, h.hn, nst, nst, +1, 1.0 / (double)h.npoint);
   projector_phases(h, KA_CURRENT);
   projector_project_expand(h, h.hn, nst, nst, h.vnl, nst, false);
@@ -660,6 +660,13 @@ void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi,
     a.xcd = nst % 8 != 0;
     a.kin_in = phi + b0;
     a.kin_ld = ld;
+    if (line) {
+      a.mm_phi = line + b0;
+      a.mm_ld = line_ld;
+      a.mm_part = part;
+      a.mm_nst = nst;
+      a.mm_band0 = b0;
+    }
     if (h.rect)
       fft3_rect_fourier_hamiltonian(a, h.n, h.stream);
     else
