@@ -169,6 +169,13 @@ struct fft3_args {
   // last sweep adds (fft3_fourier_hamiltonian)
   const cplx *kin_in;
   long kin_ld;
+  // its planes: the owned points of plane z are rows [zoff[z], zoff[z + 1]) of
+  // zxy (x << 16 | y), zown (ownership words) and S (zoff == nullptr: none);
+  // psi at the owned points goes to S [row][ldS], V_nl psi comes from Qe, both
+  // with the chunk's band cb at column cb
+  const int *zoff, *zxy, *zown;
+  cplx *S;
+  long ldS;
   // and the partial sums of the line search over them (mm_phi == nullptr: none):
   // for each (x, y rows) of the grid and band mm_band0 + b, the eight of
   // line_sums over phi, kin_in and hpsi into mm_part[row][mm_nst][8]
@@ -194,12 +201,14 @@ __device__ __forceinline__ void line_sums(double *a, cplx f, cplx r, cplx h) {
 // Rows of those partial sums
 inline long line_sum_rows(int nx, int ny) { return (long)nx * ((ny + 7) / 8); }
 
-// G-space Hpsi on the chunk's bands from psi = IFFT(phi) (INQ layout, `psi`)
-// and phi itself (`kin_in`): hpsi = FFT(V psi + V_nl psi) + 1/2 |G+k+A|^2 phi,
-// V_nl psi from the ownership entries Qe, in three sweeps (z forward of the
-// potential terms, x-y forward, a transposing write that adds the kinetic
-// term).
-void fft3_fourier_hamiltonian(const fft3_args &a, int L, hipStream_t stream);
+// G-space Hpsi on the chunk's bands from phi (`psi` and `kin_in`): hpsi =
+// FFT(V psi + V_nl psi) + 1/2 |G+k+A|^2 phi with psi = IFFT(phi).
+// G_INVERSE: z inverse into W and, with owned points, psi there into S (for
+// the projector, which leaves V_nl psi in Qe).  G_FORWARD: the planes (x and y
+// inverse, potential terms, x and y forward) and the z forward write with the
+// kinetic term.
+enum fourier_half : int { G_INVERSE, G_FORWARD };
+void fft3_fourier_hamiltonian(const fft3_args &a, int L, hipStream_t stream, fourier_half half);
 
 // True when the three-sweep kernels exist for length L and fit in max_lds.
 bool fft3_supported(int L, size_t max_lds);
@@ -222,6 +231,7 @@ void fft3_rect_prepare(const int n[3]);
 void fft3_rect_local_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream, int sweep,
                                  bool fwd_next, const project_expand_args *proj = nullptr);
 bool fft3_rect_projector(const int n[3], int nb);
-void fft3_rect_fourier_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream);
+void fft3_rect_fourier_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream,
+                                   fourier_half half);
 
 }  // namespace inqamd

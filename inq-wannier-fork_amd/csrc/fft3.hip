@@ -95,19 +95,17 @@ static void z_bwd_launch(const fft3_args &a, hipStream_t stream) {
 
 // G-space Hpsi sweeps
 template <int R0, int R1, int R2, int TY>
-__global__ __launch_bounds__(z_threads(R0 * R1 * R2)) void z_pot_kernel(const fft3_args a) {
+__global__ __launch_bounds__(z_threads(R0 * R1 * R2)) void z_inv_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
-  // tiles dealt per XCD: one (x, y rows) pair's band tiles share V and the
-  // ownership words through one L2
   constexpr int TB = Z_COLS / TY;
-  z_fwd_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2), true>(
-      a, xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB), lds);
+  const long t = a.xcd ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
+  z_fwd_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2), +1>(a, t, lds);
 }
 
-template <int R0, int R1, int R2, int NT>
-__global__ __launch_bounds__(NT) void xy_fwd_kernel(const fft3_args a) {
+template <int R0, int R1, int R2, int NT, bool GATHER>
+__global__ __launch_bounds__(NT) void xy_real_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
-  xy_fwd_plane<R0, R1, R2, NT>(a, blockIdx.x, lds);
+  xy_real_plane<R0, R1, R2, NT, GATHER>(a, xcd_tile(blockIdx.x, gridDim.x, a.nb), lds);
 }
 
 template <int R0, int R1, int R2, int TY, bool MM>
@@ -156,10 +154,11 @@ static void prepare3() {
   ensure_lds(xy_kin_kernel<R0, R1, R2, plane_threads(L)>, xy_kin_lds<R0, R1, R2>());
   ensure_lds(xy_kin_kernel<R0, R1, R2, wide_threads(L)>, xy_kin_lds<R0, R1, R2>());
   if constexpr (L <= PROJ_MAX_LEN) ensure_lds(xy_proj_kernel<R0, R1, R2>, xy_proj_lds<R0, R1, R2>());
-  ensure_lds(z_pot_kernel<R0, R1, R2, 8>, zl);
-  ensure_lds(z_kin_kernel<R0, R1, R2, 8, false>, zl);
-  ensure_lds(z_kin_kernel<R0, R1, R2, 8, true>, zl);
-  ensure_lds(xy_fwd_kernel<R0, R1, R2, wide_threads(L)>, pl);
+  ensure_lds(z_inv_kernel<R0, R1, R2, 8>, zl);
+  ensure_lds(z_kin_kernel<R0, R1, R2, 8, false>, z_bwd_lds(L));
+  ensure_lds(z_kin_kernel<R0, R1, R2, 8, true>, z_bwd_lds(L));
+  ensure_lds(xy_real_kernel<R0, R1, R2, wide_threads(L), true>, pl);
+  ensure_lds(xy_real_kernel<R0, R1, R2, wide_threads(L), false>, pl);
   const size_t zbp = z_bwd_lds(L, z_bwd_cols(L, false)), zba = z_bwd_lds(L, z_bwd_cols(L, true));
   ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 8, false, false>, zbp);
   ensure_lds(z_bwd_epi_kernel<R0, R1, R2, 16, false, false>, zbp);
@@ -236,30 +235,36 @@ static void launch3(const fft3_args &a, hipStream_t stream, int sweep, bool fwd_
 }
 
 template <int R0, int R1, int R2>
-static void launch_fourier(const fft3_args &a, hipStream_t stream) {
-  constexpr int L = R0 * R1 * R2;
-  const long ztiles = z_tiles<8>(L, a.nb);
-  const size_t zlds = (size_t)L * Z_COLS * sizeof(cplx);
+static void launch_fourier(const fft3_args &a, hipStream_t stream, fourier_half half) {
+  constexpr int L = R0 * R1 * R2, NT = wide_threads(L);
+  const dim3 tiles((unsigned)z_tiles<8>(L, a.nb)), planes((unsigned)((long)a.nb * L));
   const size_t plds = (size_t)L * (L + 1) * sizeof(cplx);
-  hipLaunchKernelGGL((z_pot_kernel<R0, R1, R2, 8>), dim3((unsigned)ztiles), dim3(z_threads(L)), zlds,
-                     stream, a);
+  if (half == G_INVERSE) {
+    hipLaunchKernelGGL((z_inv_kernel<R0, R1, R2, 8>), tiles, dim3(z_threads(L)),
+                       (size_t)L * Z_COLS * sizeof(cplx), stream, a);
+    INQAMD_HIP_CHECK(hipGetLastError());
+    if (a.zoff)
+      hipLaunchKernelGGL((xy_real_kernel<R0, R1, R2, NT, true>), planes, dim3(NT), plds, stream, a);
+    INQAMD_HIP_CHECK(hipGetLastError());
+    return;
+  }
+  hipLaunchKernelGGL((xy_real_kernel<R0, R1, R2, NT, false>), planes, dim3(NT), plds, stream, a);
   INQAMD_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL((xy_fwd_kernel<R0, R1, R2, wide_threads(L)>), dim3((unsigned)((long)a.nb * L)),
-                     dim3(wide_threads(L)), plds, stream, a);
-  INQAMD_HIP_CHECK(hipGetLastError());
+  fft3_args k = a;
+  k.scale = 1.0;  // (the planes took 1/N)
   if (a.mm_phi)
-    hipLaunchKernelGGL((z_kin_kernel<R0, R1, R2, 8, true>), dim3((unsigned)ztiles),
-                       dim3(z_threads(L)), zlds, stream, a);
+    hipLaunchKernelGGL((z_kin_kernel<R0, R1, R2, 8, true>), tiles, dim3(z_threads(L)),
+                       z_bwd_lds(L), stream, k);
   else
-    hipLaunchKernelGGL((z_kin_kernel<R0, R1, R2, 8, false>), dim3((unsigned)ztiles),
-                       dim3(z_threads(L)), zlds, stream, a);
+    hipLaunchKernelGGL((z_kin_kernel<R0, R1, R2, 8, false>), tiles, dim3(z_threads(L)),
+                       z_bwd_lds(L), stream, k);
   INQAMD_HIP_CHECK(hipGetLastError());
 }
 
-void fft3_fourier_hamiltonian(const fft3_args &a, int L, hipStream_t stream) {
+void fft3_fourier_hamiltonian(const fft3_args &a, int L, hipStream_t stream, fourier_half half) {
   switch (L) {
 #define INQAMD_FFT3_CASE(LL, R0, R1, R2) \
-  case LL: launch_fourier<R0, R1, R2>(a, stream); return;
+  case LL: launch_fourier<R0, R1, R2>(a, stream, half); return;
     INQAMD_FFT3_TABLE(INQAMD_FFT3_CASE)
 #undef INQAMD_FFT3_CASE
     default: throw error{ERR_UNSUPPORTED, "G-space three-sweep Hpsi: unsupported grid length"};

@@ -151,9 +151,8 @@ __device__ __forceinline__ void rect_y_kinetic(const rect_cols &k, const cplx *t
   rect_stage<R0, L / R0, L, NT>(k, tw, +1, ld, st);
 }
 
-// Plane `plane` = band * nz + z.  FWD: only the forward transforms, in place in W
-// (G-space Hpsi)
-template <int NT, bool FWD>
+// Plane `plane` = band * nz + z
+template <int NT>
 __device__ __forceinline__ void rect_xy_plane(const fft3_args &a, int nz, long plane, cplx *lds) {
   const int nx = a.nx, ny = a.ny, pad = ny | 1;
   const int z = (int)(plane % nz);
@@ -176,62 +175,122 @@ __device__ __forceinline__ void rect_xy_plane(const fft3_args &a, int nz, long p
     INQAMD_RECT_XY(INQAMD_RECT_CASE)
 #undef INQAMD_RECT_CASE
   }
-  if constexpr (FWD) {
-    // (back into LDS and out in order, as in the cubic planes)
-    switch (ny) {
-#define INQAMD_RECT_CASE(L, R0, R1, R2)                                                   \
-  case L:                                                                                \
-    rect_axis<R0, R1, R2, NT, true, true>(ky, a.twy, -1, ly, ly, sy, sy);                \
-    break;
-      INQAMD_RECT_XY(INQAMD_RECT_CASE)
-#undef INQAMD_RECT_CASE
-    }
-    for (int e = threadIdx.x; e < nx * ny; e += NT) {
-      int x, y;
-      kx.split(e, x, y);
-      W[e] = lds[x * pad + y];
-    }
-  } else {
-    // 1/2 |G + k + A|^2 with G = m_x b0 + m_y b1 + m_z b2 (cartesian)
-    double kc[3], gz[3], b0[3], b1[3];
-    xy_kc(a, kc);
-    const int mz = symmetric_index(z, nz);
+  // 1/2 |G + k + A|^2 with G = m_x b0 + m_y b1 + m_z b2 (cartesian)
+  double kc[3], gz[3], b0[3], b1[3];
+  xy_kc(a, kc);
+  const int mz = symmetric_index(z, nz);
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-      gz[d] = mz * a.rlat[2 * 3 + d] + kc[d];
-      b0[d] = a.rlat[0 * 3 + d];
-      b1[d] = a.rlat[1 * 3 + d];
-    }
-    cplx *G = a.gdump ? a.gdump + plane * nx * ny : nullptr;
-    auto kin = [&](int i, int c, cplx v) -> cplx {
-      if (G) G[c * ny + i] = v;
-      const int my = symmetric_index(i, ny), mx = symmetric_index(c, nx);
-      const double q0 = mx * b0[0] + my * b1[0] + gz[0];
-      const double q1 = mx * b0[1] + my * b1[1] + gz[1];
-      const double q2 = mx * b0[2] + my * b1[2] + gz[2];
-      return cscale(0.5 * (q0 * q0 + q1 * q1 + q2 * q2), v);
-    };
-    switch (ny) {
+  for (int d = 0; d < 3; d++) {
+    gz[d] = mz * a.rlat[2 * 3 + d] + kc[d];
+    b0[d] = a.rlat[0 * 3 + d];
+    b1[d] = a.rlat[1 * 3 + d];
+  }
+  cplx *G = a.gdump ? a.gdump + plane * nx * ny : nullptr;
+  auto kin = [&](int i, int c, cplx v) -> cplx {
+    if (G) G[c * ny + i] = v;
+    const int my = symmetric_index(i, ny), mx = symmetric_index(c, nx);
+    const double q0 = mx * b0[0] + my * b1[0] + gz[0];
+    const double q1 = mx * b0[1] + my * b1[1] + gz[1];
+    const double q2 = mx * b0[2] + my * b1[2] + gz[2];
+    return cscale(0.5 * (q0 * q0 + q1 * q1 + q2 * q2), v);
+  };
+  switch (ny) {
 #define INQAMD_RECT_CASE(L, R0, R1, R2)                                                   \
-  case L: rect_y_kinetic<R0, R1, R2, NT>(ky, a.twy, ly, sy, kin); break;
+case L: rect_y_kinetic<R0, R1, R2, NT>(ky, a.twy, ly, sy, kin); break;
+    INQAMD_RECT_XY(INQAMD_RECT_CASE)
+#undef INQAMD_RECT_CASE
+  }
+  switch (nx) {
+#define INQAMD_RECT_CASE(L, R0, R1, R2)                                                   \
+case L:                                                                                \
+  rect_axis<R0, R1, R2, NT, true, false>(kx, a.twx, +1, lx, lx, sx, wx);               \
+  break;
+    INQAMD_RECT_XY(INQAMD_RECT_CASE)
+#undef INQAMD_RECT_CASE
+  }
+}
+
+// The planes of the G-space Hpsi (xy_real_plane of the cubic grids)
+template <int NT, bool GATHER>
+__device__ __forceinline__ void rect_real_plane(const fft3_args &a, int nz, long t, cplx *lds) {
+  const int nx = a.nx, ny = a.ny, pad = ny | 1;
+  const int z = (int)(t / a.nb), b = (int)(t - (long)z * a.nb);
+  const int zo = a.zoff ? a.zoff[z] : 0, zn = a.zoff ? a.zoff[z + 1] - zo : 0;
+  if constexpr (GATHER) {
+    if (zn == 0) return;
+  }
+  cplx *W = a.W + ((long)b * nz + z) * nx * ny;
+  const rect_cols kx = {ny, 1.0f / (float)ny}, ky = {nx, 1.0f / (float)nx};
+  auto gx = [&](int i, int c) -> cplx { return W[i * ny + c]; };  // (i = x, c = y)
+  auto wx = [&](int i, int c, cplx v) { W[i * ny + c] = v; };
+  auto lx = [&](int i, int c) -> cplx { return lds[i * pad + c]; };
+  auto sx = [&](int i, int c, cplx v) { lds[i * pad + c] = v; };
+  auto ly = [&](int i, int c) -> cplx { return lds[c * pad + i]; };  // (i = y, c = x)
+  auto sy = [&](int i, int c, cplx v) { lds[c * pad + i] = v; };
+  const double *V = a.V + z;
+  auto sv = [&](int i, int c, cplx v) {
+    if constexpr (!GATHER) v = cscale(a.scale * V[((long)c * ny + i) * nz], v);
+    lds[c * pad + i] = v;
+  };
+  auto slot = [&](int k) {
+    const int xy = a.zxy[zo + k];
+    return (xy >> 16) * pad + (xy & 0xffff);
+  };
+  const int own0 = !GATHER && (int)threadIdx.x < zn ? a.zown[zo + threadIdx.x] : 0;
+  switch (nx) {
+#define INQAMD_RECT_CASE(L, R0, R1, R2) \
+  case L: rect_axis<R0, R1, R2, NT, false, true>(kx, a.twx, +1, gx, lx, sx, sx); break;
+    INQAMD_RECT_XY(INQAMD_RECT_CASE)
+#undef INQAMD_RECT_CASE
+  }
+  cplx first = mk(0.0, 0.0);
+  if (own0) first = a.Qe[(long)(own0 >> OWN_COUNT_BITS) * a.ldQ + b];
+  switch (ny) {
+#define INQAMD_RECT_CASE(L, R0, R1, R2) \
+  case L: rect_axis<R0, R1, R2, NT, true, true>(ky, a.twy, +1, ly, ly, sy, sv); break;
+    INQAMD_RECT_XY(INQAMD_RECT_CASE)
+#undef INQAMD_RECT_CASE
+  }
+  if constexpr (GATHER) {
+    for (int k = threadIdx.x; k < zn; k += NT)
+      a.S[(long)(zo + k) * a.ldS + b] = cscale(a.scale, lds[slot(k)]);
+  } else {
+    if (zn > 0) {
+      for (int k = threadIdx.x; k < zn; k += NT) {
+        const int own = k < NT ? own0 : a.zown[zo + k];
+        const int e0 = own >> OWN_COUNT_BITS, cnt = own & OWN_MAX_COUNT;
+        cplx v = k < NT ? first : a.Qe[(long)e0 * a.ldQ + b];
+        for (int j = 1; j < cnt; j++) v = cadd(v, a.Qe[(long)(e0 + j) * a.ldQ + b]);
+        const int e = slot(k);
+        lds[e] = cadd(lds[e], v);
+      }
+      __syncthreads();
+    }
+    switch (ny) {
+#define INQAMD_RECT_CASE(L, R0, R1, R2) \
+  case L: rect_axis<R0, R1, R2, NT, true, true>(ky, a.twy, -1, ly, ly, sy, sy); break;
       INQAMD_RECT_XY(INQAMD_RECT_CASE)
 #undef INQAMD_RECT_CASE
     }
     switch (nx) {
-#define INQAMD_RECT_CASE(L, R0, R1, R2)                                                   \
-  case L:                                                                                \
-    rect_axis<R0, R1, R2, NT, true, false>(kx, a.twx, +1, lx, lx, sx, wx);               \
-    break;
+#define INQAMD_RECT_CASE(L, R0, R1, R2) \
+  case L: rect_axis<R0, R1, R2, NT, true, false>(kx, a.twx, -1, lx, lx, sx, wx); break;
       INQAMD_RECT_XY(INQAMD_RECT_CASE)
 #undef INQAMD_RECT_CASE
     }
   }
 }
 
-template <int NT, bool FWD>
+// What an x-y launch runs
+enum rect_planes : int { RECT_KINETIC, RECT_GATHER, RECT_POTENTIAL };
+
+template <int NT, int MODE>
 __global__ __launch_bounds__(NT) void rect_xy_kernel(const fft3_args a, int nz) {
   extern __shared__ cplx lds[];
-  rect_xy_plane<NT, FWD>(a, nz, blockIdx.x, lds);
+  if constexpr (MODE == RECT_KINETIC)
+    rect_xy_plane<NT>(a, nz, blockIdx.x, lds);
+  else
+    rect_real_plane<NT, MODE == RECT_GATHER>(a, nz, xcd_tile(blockIdx.x, gridDim.x, a.nb), lds);
 }
 
 // The kinetic planes after the workgroups of the projector
@@ -243,7 +302,7 @@ void rect_xy_proj_kernel(const fft3_args a, int nz, const project_expand_args pa
   if ((int)blockIdx.x < nproj)
     p4_block(pa, blockIdx.x, ntile, lds);
   else
-    rect_xy_plane<P4_NT, false>(a, nz, blockIdx.x - nproj, lds);
+    rect_xy_plane<P4_NT>(a, nz, blockIdx.x - nproj, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -254,25 +313,25 @@ static size_t rect_xy_lds(const int n[3]) { return (size_t)n[0] * (n[1] | 1) * s
 template <int NT>
 static void rect_xy_prepare(size_t lds) {
   if (lds <= 65536) return;
-  INQAMD_HIP_CHECK(hipFuncSetAttribute((const void *)rect_xy_kernel<NT, false>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
-  INQAMD_HIP_CHECK(hipFuncSetAttribute((const void *)rect_xy_kernel<NT, true>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
+  for (const void *k : {(const void *)rect_xy_kernel<NT, RECT_KINETIC>,
+                        (const void *)rect_xy_kernel<NT, RECT_GATHER>,
+                        (const void *)rect_xy_kernel<NT, RECT_POTENTIAL>})
+    INQAMD_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
 }
 
-template <bool FWD>
+template <int MODE>
 static void rect_xy_launch(const fft3_args &a, const int n[3], hipStream_t stream) {
   const unsigned planes = (unsigned)((long)a.nb * n[2]);
   const size_t lds = rect_xy_lds(n);
   const int el = n[0] * n[1];
   if (el <= rect_elements(128))
-    hipLaunchKernelGGL((rect_xy_kernel<128, FWD>), dim3(planes), dim3(128), lds, stream, a, n[2]);
+    hipLaunchKernelGGL((rect_xy_kernel<128, MODE>), dim3(planes), dim3(128), lds, stream, a, n[2]);
   else if (el <= rect_elements(256))
-    hipLaunchKernelGGL((rect_xy_kernel<256, FWD>), dim3(planes), dim3(256), lds, stream, a, n[2]);
+    hipLaunchKernelGGL((rect_xy_kernel<256, MODE>), dim3(planes), dim3(256), lds, stream, a, n[2]);
   else if (el <= rect_elements(512))
-    hipLaunchKernelGGL((rect_xy_kernel<512, FWD>), dim3(planes), dim3(512), lds, stream, a, n[2]);
+    hipLaunchKernelGGL((rect_xy_kernel<512, MODE>), dim3(planes), dim3(512), lds, stream, a, n[2]);
   else
-    hipLaunchKernelGGL((rect_xy_kernel<1024, FWD>), dim3(planes), dim3(1024), lds, stream, a,
+    hipLaunchKernelGGL((rect_xy_kernel<1024, MODE>), dim3(planes), dim3(1024), lds, stream, a,
                        n[2]);
   INQAMD_HIP_CHECK(hipGetLastError());
 }
@@ -327,7 +386,7 @@ void fft3_rect_local_hamiltonian(const fft3_args &a, const int n[3], hipStream_t
                        lds, stream, a, n[2], *proj, ntile, np);
     INQAMD_HIP_CHECK(hipGetLastError());
   } else if (sweep < 0 || sweep == 1) {
-    rect_xy_launch<false>(a, n, stream);
+    rect_xy_launch<RECT_KINETIC>(a, n, stream);
   }
   if (sweep < 0 || sweep == 2)
     rect_z(a, n[2],
@@ -336,10 +395,17 @@ void fft3_rect_local_hamiltonian(const fft3_args &a, const int n[3], hipStream_t
            stream);
 }
 
-void fft3_rect_fourier_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream) {
-  rect_z(a, n[2], RECT_Z_POT, stream);
-  rect_xy_launch<true>(a, n, stream);
-  rect_z(a, n[2], RECT_Z_KIN, stream);
+void fft3_rect_fourier_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream,
+                                   fourier_half half) {
+  if (half == G_INVERSE) {
+    rect_z(a, n[2], RECT_Z_INV, stream);
+    if (a.zoff) rect_xy_launch<RECT_GATHER>(a, n, stream);
+    return;
+  }
+  rect_xy_launch<RECT_POTENTIAL>(a, n, stream);
+  fft3_args k = a;
+  k.scale = 1.0;  // (the planes took 1/N)
+  rect_z(k, n[2], RECT_Z_KIN, stream);
 }
 
 }  // namespace inqamd

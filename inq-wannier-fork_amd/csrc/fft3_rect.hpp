@@ -25,8 +25,8 @@ enum rect_z_kernel : int {
   RECT_Z_BWD_ACC,      // ... and the Taylor sums
   RECT_Z_BWD_FWD,      // ... transforming its output forward
   RECT_Z_BWD_ACC_FWD,  // ... both
-  RECT_Z_POT,          // z forward of V psi + V_nl psi (G-space Hpsi)
-  RECT_Z_KIN,          // transposing write with the kinetic term (G-space Hpsi)
+  RECT_Z_INV,          // z inverse (G-space Hpsi)
+  RECT_Z_KIN,          // z forward with the kinetic term (G-space Hpsi)
   RECT_Z_PREPARE       // LDS attributes of them all
 };
 

@@ -66,10 +66,8 @@ constexpr int plane_threads(int L) {
 // ---------------------------------------------------------------------------
 // sweep 1: z forward, INQ layout -> band-major W
 // ---------------------------------------------------------------------------
-// POT: the tile transforms V psi + V_nl psi (ownership entries Qe) instead
-// of psi, formed as the first stage loads psi.
-template <int R0, int R1, int R2, int Z_TY, int NT = Z_NT, bool POT = false,
-          bool RECT = false>
+// SIGN +1: the inverse transform (the first sweep of the G-space Hpsi)
+template <int R0, int R1, int R2, int Z_TY, int NT = Z_NT, int SIGN = -1, bool RECT = false>
 __device__ __forceinline__ void z_fwd_tile(const fft3_args &a, long t, cplx *lds) {
   using P = plan3<R0, R1, R2>;
   constexpr int L = P::LEN;
@@ -93,18 +91,7 @@ __device__ __forceinline__ void z_fwd_tile(const fft3_args &a, long t, cplx *lds
     const int b = c / Z_TY, y = c % Z_TY;
     if (!(y0 + y < NY && cb0 + b < a.nb)) return mk(0.0, 0.0);
     const long p = ((long)x * NY + y0 + y) * L + i;
-    cplx v = a.psi[p * a.ld + gb0 + b];
-    if constexpr (POT) {
-      const double vp = a.V[p];
-      v = mk(vp * v.x, vp * v.y);
-      // own[p] = -1 outside every sphere
-      const int w = a.own ? a.own[p] : -1;
-      if (w >= 0) {
-        const int e0 = w >> OWN_COUNT_BITS, cnt = w & OWN_MAX_COUNT;
-        for (int j = 0; j < cnt; j++) v = cadd(v, a.Qe[(long)(e0 + j) * a.ldQ + gb0 + b]);
-      }
-    }
-    return v;
+    return a.psi[p * a.ld + gb0 + b];
   };
   auto ll = [&](int i, int c) -> cplx { return lds[i * Z_COLS + zswz(c)]; };
   auto ls = [&](int i, int c, cplx v, int, int) { lds[i * Z_COLS + zswz(c)] = v; };
@@ -113,7 +100,7 @@ __device__ __forceinline__ void z_fwd_tile(const fft3_args &a, long t, cplx *lds
     if (y0 + y < NY && cb0 + b < a.nb)
       a.W[(((long)(cb0 + b) * L + i) * NX + x) * NY + y0 + y] = v;
   };
-  run_plan<P, R0, R1, R2, Z_COLS, NT>(a.tw, -1, false, gl, ll, ls, gs, false);
+  run_plan<P, R0, R1, R2, Z_COLS, NT>(a.tw, SIGN, false, gl, ll, ls, gs, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -378,26 +365,81 @@ __device__ __forceinline__ void xy_kin_plane(const fft3_args &a, long plane, cpl
   xy_kin_plane_from<R0, R1, R2, NT>(a, plane, lds, in, tw, kc);
 }
 
-// The forward x-y transform of one plane (G-space Hpsi), in place in W
-template <int R0, int R1, int R2, int NT = plane_threads(R0 * R1 * R2)>
-__device__ __forceinline__ void xy_fwd_plane(const fft3_args &a, long plane, cplx *lds) {
+// The planes of the G-space Hpsi, where W holds phi transformed to real space in z.
+// Plane t = (z, band), band fastest: the workgroups of one z share its V and
+// ownership rows.
+// GATHER: psi of the plane's owned points (x 1/N, projector_tables::zxy) into the
+// rows of S, whole planes without any skipped; W stays as it is.
+// Otherwise x and y to real space, x V / N and + V_nl psi of the owned points, back
+// in x and y, in place in W.
+template <int R0, int R1, int R2, int NT, bool GATHER>
+__device__ __forceinline__ void xy_real_plane(const fft3_args &a, long t, cplx *lds) {
   using XP = xy_plan<R0, R1, R2>;
   using P = typename XP::P;
   constexpr int X0 = XP::X0, X1 = XP::X1, X2 = XP::X2;
   constexpr int L = P::LEN;
   constexpr int PAD = L + 1;
-  cplx *W = a.W + plane * L * L;
+  constexpr int RL = P::NSTAGE == 2 ? X1 : X2;  // last radix
+  constexpr int NBL = L / RL;
+  constexpr int NBF = (NBL * L + NT - 1) / NT;
+  const int z = (int)(t / a.nb), b = (int)(t - (long)z * a.nb);
+  const int zo = a.zoff ? a.zoff[z] : 0, zn = a.zoff ? a.zoff[z + 1] - zo : 0;
+  if constexpr (GATHER) {
+    if (zn == 0) return;
+  }
+  cplx *W = a.W + ((long)b * L + z) * L * L;
   auto gx = [&](int i, int c) -> cplx { return W[i * L + c]; };          // (i = x, c = y)
   auto lx = [&](int i, int c) -> cplx { return lds[i * PAD + c]; };
   auto sx = [&](int i, int c, cplx v, int, int) { lds[i * PAD + c] = v; };
+  auto wx = [&](int i, int c, cplx v, int, int) { W[i * L + c] = v; };
   auto ly = [&](int i, int c) -> cplx { return lds[c * PAD + i]; };    // (i = y, c = x)
   auto sy = [&](int i, int c, cplx v, int, int) { lds[c * PAD + i] = v; };
-  run_plan<P, X0, X1, X2, L, NT>(a.tw, -1, false, gx, lx, sx, sx, true);  // x forward
-  // y forward back into LDS and out in order: from the last stage's registers a
-  // wave would write 16 bytes into each of 64 rows (the steepest descent at 64^3
-  // x 256 and its diagonalisation 59.9 ms so, 57.0 in order)
-  run_plan<P, X0, X1, X2, L, NT>(a.tw, -1, true, ly, ly, sy, sy, true);
-  for (int e = threadIdx.x; e < L * L; e += NT) W[e] = lds[e / L * PAD + e % L];
+  auto slot = [&](int k) {  // LDS slot of the plane's owned point k
+    const int xy = a.zxy[zo + k];
+    return (xy >> 16) * PAD + (xy & 0xffff);
+  };
+  if constexpr (GATHER) {
+    run_plan<P, X0, X1, X2, L, NT>(a.tw, +1, false, gx, lx, sx, sx, true);  // x inverse
+    run_plan<P, X0, X1, X2, L, NT>(a.tw, +1, true, ly, ly, sy, sy, true);   // y inverse
+    for (int k = threadIdx.x; k < zn; k += NT)
+      a.S[(long)(zo + k) * a.ldS + b] = cscale(a.scale, lds[slot(k)]);
+  } else {
+    // V at the outputs of the y inverse's last stage (point j + r NBL of
+    // butterfly j, column x), and the first owned point's V_nl psi, loaded under
+    // the transforms
+    double vp[NBF][RL];
+#pragma unroll
+    for (int q = 0; q < NBF; q++) {
+      const int w = threadIdx.x + q * NT;
+      const int j = w / L, c = w % L;
+#pragma unroll
+      for (int r = 0; r < RL; r++) {
+        const bool in = NBF * NT == NBL * L || w < NBL * L;
+        vp[q][r] = a.V[in ? ((long)c * L + j + r * NBL) * L + z : 0];
+      }
+    }
+    const int own0 = (int)threadIdx.x < zn ? a.zown[zo + threadIdx.x] : 0;
+    run_plan<P, X0, X1, X2, L, NT>(a.tw, +1, false, gx, lx, sx, sx, true);  // x inverse
+    cplx first = mk(0.0, 0.0);
+    if (own0) first = a.Qe[(long)(own0 >> OWN_COUNT_BITS) * a.ldQ + b];
+    auto sv = [&](int i, int c, cplx v, int q, int r) {
+      lds[c * PAD + i] = cscale(a.scale * vp[q][r], v);
+    };
+    run_plan<P, X0, X1, X2, L, NT>(a.tw, +1, true, ly, ly, sy, sv, true);  // y inverse
+    if (zn > 0) {
+      for (int k = threadIdx.x; k < zn; k += NT) {
+        const int own = k < NT ? own0 : a.zown[zo + k];
+        const int e0 = own >> OWN_COUNT_BITS, cnt = own & OWN_MAX_COUNT;
+        cplx v = k < NT ? first : a.Qe[(long)e0 * a.ldQ + b];
+        for (int j = 1; j < cnt; j++) v = cadd(v, a.Qe[(long)(e0 + j) * a.ldQ + b]);
+        const int e = slot(k);
+        lds[e] = cadd(lds[e], v);
+      }
+      __syncthreads();
+    }
+    run_plan<P, X0, X1, X2, L, NT>(a.tw, -1, true, ly, ly, sy, sy, true);   // y forward
+    run_plan<P, X0, X1, X2, L, NT>(a.tw, -1, true, lx, lx, sx, wx, false);  // x forward
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -405,9 +447,8 @@ __device__ __forceinline__ void xy_fwd_plane(const fft3_args &a, long plane, cpl
 // ---------------------------------------------------------------------------
 // ACC: the caller passes Taylor sums (acc1, perhaps acc2); without it they
 // must be null and the epilogue is a plain store.
-// GS (G-space Hpsi): no z transform (the first sweep made it), only the
-// transposing write, whose epilogue adds 1/2 |G+k+A|^2 kin_in instead of
-// V psi (no ownership entries, no scale).
+// GS (G-space Hpsi): z forward instead, and the epilogue adds 1/2 |G+k+A|^2
+// kin_in instead of V psi (no ownership entries).
 // FWD (Taylor chains): the tile then transforms its own hpsi forward in z
 // into W, in place of the next application's z_fwd sweep over the same tile
 // (the chunk's W region the tile read is the region it writes).
@@ -557,7 +598,7 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
   // The twiddle table (L entries) goes the same way into the L slots after
   // the tile, so that the transforms' twiddles are LDS reads.
   cplx *ltw = lds + L * Z_COLS;
-  if constexpr (!GS) {
+  {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lr = lane / Z_COLS, c = zswz(lane % Z_COLS);
     const int b = c / Z_TY, y = c % Z_TY;
@@ -640,28 +681,14 @@ __device__ __forceinline__ void z_bwd_epi_tile(const fft3_args &a, long t, cplx 
     if (a.Pc) vnl_expand_wave<NE, Z_TB>(a, gb0, own, osp, pre);
   }
 
-  auto gl = [&](int i, int c) -> cplx {
-    const int b = c / Z_TY, y = c % Z_TY;
-    return (y0 + y < NY && cb0 + b < a.nb) ? a.W[(((long)(cb0 + b) * L + i) * NX + x) * NY + y0 + y]
-                                          : mk(0.0, 0.0);
-  };
   auto ll = [&](int i, int c) -> cplx { return lds[i * Z_COLS + zswz(c)]; };
   auto ls = [&](int i, int c, cplx v, int, int) { lds[i * Z_COLS + zswz(c)] = v; };
-  if constexpr (GS) {
-    // the first sweep transformed z already: this sweep only transposes
-    for (int e = threadIdx.x; e < L * Z_COLS; e += NT) {
-      const int i = e / Z_COLS, c = e % Z_COLS;
-      lds[i * Z_COLS + zswz(c)] = gl(i, c);
-    }
-    __syncthreads();
-  } else {
-    // the W rows and twiddles loaded into LDS at the start: this wave's
-    // loads are complete (vmcnt 0), the barrier makes every wave's visible
-    __builtin_amdgcn_s_waitcnt(WAITCNT_VM0);
-    __syncthreads();
-    // (twiddles read at their products: pre[] is held through this transform)
-    run_plan<P, R0, R1, R2, Z_COLS, NT, false>(ltw, +1, true, ll, ll, ls, ls, true);
-  }
+  // the W rows and twiddles loaded into LDS at the start: this wave's
+  // loads are complete (vmcnt 0), the barrier makes every wave's visible
+  __builtin_amdgcn_s_waitcnt(WAITCNT_VM0);
+  __syncthreads();
+  // (twiddles read at their products: pre[] is held through this transform)
+  run_plan<P, R0, R1, R2, Z_COLS, NT, false>(ltw, GS ? -1 : +1, true, ll, ll, ls, ls, true);
 
   // projector_all::apply (projector_all.hpp:225-231): V_nl psi of the owned
   // points, its ownership entries summed in fixed (sphere, point) order.

@@ -620,24 +620,29 @@ void hamiltonian_apply(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld
 }
 
 // ks_hamiltonian::operator() on G-space orbitals (ks_hamiltonian.hpp:156-176)
-// for three-sweep grids: psi = to_real(phi), the projector on psi, then
-// H phi = to_fourier(V psi + V_nl psi) + 1/2 |G+k+A|^2 phi in three sweeps
-// per band chunk (z forward, x-y forward, transposing write with the kinetic
-// term).  The kinetic term acts on phi directly: the real-space
-// Hpsi followed by to_fourier would transform psi forward and back again.
+// for three-sweep grids: psi = to_real(phi), H phi = to_fourier(V psi + V_nl psi) +
+// 1/2 |G+k+A|^2 phi, the kinetic term on phi itself (to_fourier of the real-space
+// Hpsi would transform psi forward and back again).  Per band chunk: z inverse;
+// the planes to real space once for psi at the owned points alone, for the
+// projector; the planes again, to real space, x V and + V_nl psi, and back; z
+// forward.  128 N bytes per band, where to_real in three passes and three sweeps
+// of the potential terms moved 208: steepest descent at 40^3 x 48 bands 1824 ->
+// 1673 us, at 64^3 x 20 3546 -> 3303 us, at 48 x 50 x 54 x 40 3070 -> 2909 us, at
+// 64^3 x 256 (with the diagonalisation) 55.7 -> 52.2 ms; at 96^3 x 8, whose planes
+// have a CU each and are bound by their transforms, 6013 -> 6043 us.
 void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi, long hld,
                                 int nst, const cplx *line, long line_ld, double *part) {
-  fft3d(h, phi, ld, h.hn, nst, nst, +1, 1.0 / (double)h.npoint);
-  projector_phases(h, KA_CURRENT);
-  projector_project_expand(h, h.hn, nst, nst, h.vnl, nst, false);
+  const projector_tables &t = h.pt;
+  const bool project = t.nproj > 0 && t.nunique > 0;
+  if (project) projector_phases(h, KA_CURRENT);
   const band_chunks plan = chunk_plan(h, nst, ld, true);
   for (int c = 0; c < plan.n; c++) {
     const int b0 = plan.b0(c), nb = plan.nb(c);
     fft3_args a{};
     a.gskip = plan.gskip;
     a.glog = plan.glog;
-    a.psi = h.hn + b0;
-    a.ld = nst;
+    a.psi = phi + b0;
+    a.ld = ld;
     a.hpsi = hphi + b0;
     a.hld = hld;
     a.W = h.work;
@@ -650,14 +655,17 @@ void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi,
     a.ny = h.n[1];
     a.twx = h.axis[0].tw;
     a.twy = h.axis[1].tw;
-    a.scale = 1.0;
-    const projector_tables &t = h.pt;
-    if (t.nproj > 0 && t.nunique > 0) {
-      a.own = t.own;
-      a.Qe = h.vnl + b0;
-      a.ldQ = nst;
+    a.scale = 1.0 / (double)h.npoint;
+    if (project) {
+      a.zoff = t.zoff;
+      a.zxy = t.zxy;
+      a.zown = t.zown;
+      a.S = h.hn;
+      a.ldS = nb;
+      a.Qe = h.vnl;
+      a.ldQ = nb;
     }
-    a.xcd = nst % 8 != 0;
+    a.xcd = ld % 8 != 0 || hld % 8 != 0;
     a.kin_in = phi + b0;
     a.kin_ld = ld;
     if (line) {
@@ -667,10 +675,15 @@ void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi,
       a.mm_nst = nst;
       a.mm_band0 = b0;
     }
-    if (h.rect)
-      fft3_rect_fourier_hamiltonian(a, h.n, h.stream);
-    else
-      fft3_fourier_hamiltonian(a, h.n[0], h.stream);
+    auto run = [&](fourier_half half) {
+      if (h.rect)
+        fft3_rect_fourier_hamiltonian(a, h.n, h.stream, half);
+      else
+        fft3_fourier_hamiltonian(a, h.n[0], h.stream, half);
+    };
+    run(G_INVERSE);
+    if (project) projector_project_expand(h, h.hn, nb, nb, h.vnl, nb, false, t.zrow);
+    run(G_FORWARD);
   }
 }
 

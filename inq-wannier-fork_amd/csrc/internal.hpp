@@ -44,6 +44,11 @@ struct projector_tables {
   cplx *phase_ent = nullptr;  // [nent]
   int *ent = nullptr;         // [nproj][max_sphere] ownership entry of each sphere point
   int *own = nullptr;         // [N] (first entry << OWN_COUNT_BITS) | count, -1 if not owned
+  // the owned points by z plane, (x, y) ascending: plane z has rows [zoff[z],
+  // zoff[z + 1]) of zxy (x << 16 | y) and zown (own of the point); zrow: the
+  // row of each sphere point
+  int *zoff = nullptr, *zxy = nullptr, *zown = nullptr;
+  int *zrow = nullptr;        // [nproj][max_sphere]
   // per ownership entry, for expanding V_nl psi from the coefficients in the
   // Hpsi sweep (max_nlm <= 4 only; nullptr otherwise)
   int *ent_sph = nullptr;     // [nent] sphere
@@ -169,7 +174,7 @@ void projector_owned_sum(handle &h, cplx *Q, int nst, int slot);
 // projector_mfma.hip: gather + MFMA GEMM1 (-> P if write_P) + MFMA GEMM2 ->
 // per-entry V_nl psi in Qe (if Qe != nullptr)
 void projector_project_expand(handle &h, const cplx *psi, long ld, int nst, cplx *Qe, long ldQ,
-                              bool write_P);
+                              bool write_P, const int *point = nullptr);
 void mfma_selftest(double *out_device, hipStream_t stream);
 // P coefficients of all spheres and bands on the 4x4x4 FP64 MFMA (max_nlm <= 4)
 void projector_project_p4(handle &h, const cplx *psi, long ld, int nst);

@@ -262,6 +262,20 @@ void projector_upload(handle &h, int nproj, int max_sphere, int max_nlm, const i
     own[upoint[u]] = (uoff[u] << OWN_COUNT_BITS) | cnt;
   }
   for (size_t e = 0; e < uent.size(); e++) ent[uent[e]] = (int)e;
+  // the owned points by z plane (upoint ascends in (x, y, z))
+  std::vector<int> zoff(h.n[2] + 1, 0), zxy(upoint.size()), zown(upoint.size()), urow(upoint.size());
+  for (int g : upoint) zoff[g % h.n[2] + 1]++;
+  for (int z = 0; z < h.n[2]; z++) zoff[z + 1] += zoff[z];
+  std::vector<int> next(zoff.begin(), zoff.end() - 1);
+  for (size_t u = 0; u < upoint.size(); u++) {
+    const int g = upoint[u], xy = g / h.n[2], r = next[g % h.n[2]]++;
+    zxy[r] = (xy / h.n[1]) << 16 | xy % h.n[1];
+    zown[r] = own[g];
+    urow[u] = r;
+  }
+  std::vector<int> zrow(nk, -1);
+  for (long g = 0; g < nk; g++)
+    if (point[g] >= 0) zrow[g] = urow[owner[point[g]]];
   if (max_nlm <= 4 && !uent.empty()) {
     std::vector<int> esph(uent.size());
     std::vector<double> emat(uent.size() * 4, 0.0);
@@ -278,6 +292,10 @@ void projector_upload(handle &h, int nproj, int max_sphere, int max_nlm, const i
     t.ent_mat = upload(emat);
   }
   t.own = upload(own);
+  t.zoff = upload(zoff);
+  t.zxy = upload(zxy);
+  t.zown = upload(zown);
+  t.zrow = upload(zrow);
   t.ent = upload(ent);
   t.nent = (int)uent.size();
   t.owner = upload(owner);
@@ -301,6 +319,7 @@ void projector_free(handle &h) {
                   (void *)t.coeff_inq, (void *)t.size,
                   (void *)t.upoint, (void *)t.uoff, (void *)t.uent, (void *)t.owner,
                   (void *)t.phase_sph, (void *)t.phase_ent, (void *)t.own, (void *)t.ent,
+                  (void *)t.zoff, (void *)t.zxy, (void *)t.zown, (void *)t.zrow,
                   (void *)t.ent_sph, (void *)t.own_sph, (void *)t.ent_mat})
     if (p) (void)hipFree(p);
   t = projector_tables{};

@@ -88,7 +88,7 @@ __global__ void mfma_selftest_kernel(double *out) {
 }
 
 void projector_project_expand(handle &h, const cplx *psi, long ld, int nst, cplx *Qe, long ldQ,
-                              bool write_P) {
+                              bool write_P, const int *point) {
   const projector_tables &t = h.pt;
   if (t.nproj == 0) return;
   project_expand_args a;
@@ -97,7 +97,7 @@ void projector_project_expand(handle &h, const cplx *psi, long ld, int nst, cplx
   a.nst = nst;
   a.max_sphere = t.max_sphere;
   a.max_nlm = t.max_nlm;
-  a.point = t.point;
+  a.point = point ? point : t.point;
   a.size = t.size;
   a.mat = t.mat;
   a.coeff = t.coeff;
