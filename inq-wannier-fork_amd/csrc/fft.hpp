@@ -176,6 +176,10 @@ struct fft3_args {
   const int *zoff, *zxy, *zown;
   cplx *S;
   long ldS;
+  // and the preconditioner its first sweep applies to psi, in place (pre_kin ==
+  // nullptr: none): K(1/2 |G|^2 / pre_kin[16 b]) for the chunk's band at offset b
+  cplx *pre_psi;
+  const double *pre_kin;
   // and the partial sums of the line search over them (mm_phi == nullptr: none):
   // for each (x, y rows) of the grid and band mm_band0 + b, the eight of
   // line_sums over phi, kin_in and hpsi into mm_part[row][mm_nst][8]
@@ -184,6 +188,13 @@ struct fft3_args {
   double *mm_part;
   int mm_nst, mm_band0;
 };
+
+// K of Teter, Payne and Allan (preconditioner.hpp:30-37)
+__device__ __forceinline__ double tpa_k(double x) {
+  const double num = ((8.0 * x + 12.0) * x + 18.0) * x + 27.0;
+  const double den = (((16.0 * x + 8.0) * x + 12.0) * x + 18.0) * x + 27.0;
+  return num / den;
+}
 
 // <r|r>, <f|r>, <r|h>, <f|h> (real, imaginary) of one element
 // (steepest_descent.hpp:47-51)

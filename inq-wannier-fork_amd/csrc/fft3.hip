@@ -94,12 +94,12 @@ static void z_bwd_launch(const fft3_args &a, hipStream_t stream) {
 }
 
 // G-space Hpsi sweeps
-template <int R0, int R1, int R2, int TY>
+template <int R0, int R1, int R2, int TY, bool PRE>
 __global__ __launch_bounds__(z_threads(R0 * R1 * R2)) void z_inv_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
   constexpr int TB = Z_COLS / TY;
   const long t = a.xcd ? xcd_tile(blockIdx.x, gridDim.x, (a.nb + TB - 1) / TB) : (long)blockIdx.x;
-  z_fwd_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2), +1>(a, t, lds);
+  z_fwd_tile<R0, R1, R2, TY, z_threads(R0 * R1 * R2), +1, false, PRE>(a, t, lds);
 }
 
 template <int R0, int R1, int R2, int NT, bool GATHER>
@@ -154,7 +154,8 @@ static void prepare3() {
   ensure_lds(xy_kin_kernel<R0, R1, R2, plane_threads(L)>, xy_kin_lds<R0, R1, R2>());
   ensure_lds(xy_kin_kernel<R0, R1, R2, wide_threads(L)>, xy_kin_lds<R0, R1, R2>());
   if constexpr (L <= PROJ_MAX_LEN) ensure_lds(xy_proj_kernel<R0, R1, R2>, xy_proj_lds<R0, R1, R2>());
-  ensure_lds(z_inv_kernel<R0, R1, R2, 8>, zl);
+  ensure_lds(z_inv_kernel<R0, R1, R2, 8, false>, zl);
+  ensure_lds(z_inv_kernel<R0, R1, R2, 8, true>, zl);
   ensure_lds(z_kin_kernel<R0, R1, R2, 8, false>, z_bwd_lds(L));
   ensure_lds(z_kin_kernel<R0, R1, R2, 8, true>, z_bwd_lds(L));
   ensure_lds(xy_real_kernel<R0, R1, R2, wide_threads(L), true>, pl);
@@ -240,8 +241,13 @@ static void launch_fourier(const fft3_args &a, hipStream_t stream, fourier_half 
   const dim3 tiles((unsigned)z_tiles<8>(L, a.nb)), planes((unsigned)((long)a.nb * L));
   const size_t plds = (size_t)L * (L + 1) * sizeof(cplx);
   if (half == G_INVERSE) {
-    hipLaunchKernelGGL((z_inv_kernel<R0, R1, R2, 8>), tiles, dim3(z_threads(L)),
-                       (size_t)L * Z_COLS * sizeof(cplx), stream, a);
+    const size_t zlds = (size_t)L * Z_COLS * sizeof(cplx);
+    if (a.pre_kin)
+      hipLaunchKernelGGL((z_inv_kernel<R0, R1, R2, 8, true>), tiles, dim3(z_threads(L)), zlds,
+                         stream, a);
+    else
+      hipLaunchKernelGGL((z_inv_kernel<R0, R1, R2, 8, false>), tiles, dim3(z_threads(L)), zlds,
+                         stream, a);
     INQAMD_HIP_CHECK(hipGetLastError());
     if (a.zoff)
       hipLaunchKernelGGL((xy_real_kernel<R0, R1, R2, NT, true>), planes, dim3(NT), plds, stream, a);

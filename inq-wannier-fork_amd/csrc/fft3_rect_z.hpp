@@ -8,7 +8,7 @@ namespace inqamd {
 
 constexpr int RECT_TY = 8;  // y values of a 64-column tile (4 of a 32-column one)
 
-template <int R0, int R1, int R2, int SIGN>
+template <int R0, int R1, int R2, int SIGN, bool PRE>
 __global__ __launch_bounds__(z_threads(R0 * R1 * R2)) void rect_z_fwd_kernel(const fft3_args a) {
   extern __shared__ cplx lds[];
   constexpr int TB = Z_COLS / RECT_TY;
@@ -19,7 +19,7 @@ __global__ __launch_bounds__(z_threads(R0 * R1 * R2)) void rect_z_fwd_kernel(con
     return;
   }
   const long t = a.xcd ? xcd_tile(blockIdx.x, tiles, nbt) : (long)blockIdx.x;
-  z_fwd_tile<R0, R1, R2, RECT_TY, z_threads(R0 * R1 * R2), SIGN, true>(a, t, lds);
+  z_fwd_tile<R0, R1, R2, RECT_TY, z_threads(R0 * R1 * R2), SIGN, true, PRE>(a, t, lds);
 }
 
 template <int R0, int R1, int R2, bool ACC, bool FWD>
@@ -74,8 +74,9 @@ static void rect_z_run(const fft3_args &a, rect_z_kernel k, hipStream_t stream) 
   const long tiles = (long)a.nx * ((a.ny + RECT_TY - 1) / RECT_TY) * ((a.nb + TB - 1) / TB);
   const bool prep = k == RECT_Z_PREPARE;
   if (prep) {
-    rect_lds(rect_z_fwd_kernel<R0, R1, R2, -1>, zl);
-    rect_lds(rect_z_fwd_kernel<R0, R1, R2, +1>, zl);
+    rect_lds(rect_z_fwd_kernel<R0, R1, R2, -1, false>, zl);
+    rect_lds(rect_z_fwd_kernel<R0, R1, R2, +1, false>, zl);
+    rect_lds(rect_z_fwd_kernel<R0, R1, R2, +1, true>, zl);
     rect_lds(rect_z_kin_kernel<R0, R1, R2, false>, z_bwd_lds(L));
     rect_lds(rect_z_kin_kernel<R0, R1, R2, true>, z_bwd_lds(L));
   }
@@ -84,11 +85,14 @@ static void rect_z_run(const fft3_args &a, rect_z_kernel k, hipStream_t stream) 
   if (prep || k == RECT_Z_BWD_FWD) rect_z_bwd<R0, R1, R2, false, true>(a, stream, prep);
   if (prep || k == RECT_Z_BWD_ACC_FWD) rect_z_bwd<R0, R1, R2, true, true>(a, stream, prep);
   if (k == RECT_Z_FWD)
-    hipLaunchKernelGGL((rect_z_fwd_kernel<R0, R1, R2, -1>),
+    hipLaunchKernelGGL((rect_z_fwd_kernel<R0, R1, R2, -1, false>),
                        dim3((unsigned)(tiles + phase_blocks(a, z_threads(L)))),
                        dim3(z_threads(L)), zl, stream, a);
-  if (k == RECT_Z_INV)
-    hipLaunchKernelGGL((rect_z_fwd_kernel<R0, R1, R2, +1>), dim3((unsigned)tiles),
+  if (k == RECT_Z_INV && a.pre_kin)
+    hipLaunchKernelGGL((rect_z_fwd_kernel<R0, R1, R2, +1, true>), dim3((unsigned)tiles),
+                       dim3(z_threads(L)), zl, stream, a);
+  if (k == RECT_Z_INV && !a.pre_kin)
+    hipLaunchKernelGGL((rect_z_fwd_kernel<R0, R1, R2, +1, false>), dim3((unsigned)tiles),
                        dim3(z_threads(L)), zl, stream, a);
   if (k == RECT_Z_KIN && a.mm_phi)
     hipLaunchKernelGGL((rect_z_kin_kernel<R0, R1, R2, true>), dim3((unsigned)tiles),

@@ -359,13 +359,6 @@ __global__ __launch_bounds__(256) void lambda_final(const double *part, long nch
   band[b * 16 + 6] = fabs(den) < 1e-15 ? 0.0 : 2.0 * cc / den;
 }
 
-// K of Teter, Payne and Allan (preconditioner.hpp:30-37)
-__device__ double tpa_k(double x) {
-  const double num = ((8.0 * x + 12.0) * x + 18.0) * x + 27.0;
-  const double den = (((16.0 * x + 8.0) * x + 12.0) * x + 18.0) * x + 27.0;
-  return num / den;
-}
-
 // pass 3: phi(G) *= K(1/2 |G|^2 / kinetic_b) (preconditioner.hpp:45-52).
 // A wave takes one grid point at a time, its lanes the bands: the point's
 // G vector is worked out once per point (the index divisions of a flat
@@ -517,11 +510,16 @@ void inner_products(handle &h, const cplx *A, long lda, const cplx *B, long ldb,
 // The K(1/2|G|^2/kinetic) scaling of operations::preconditioner for
 // fourier_space orbitals (preconditioner.hpp:39-55), given the residual-type
 // kinetic sums already in the band records.
-void precondition_apply(handle &h, cplx *phi, long ld, int nst) {
+void preconditioner_kinetic(handle &h, int nst) {
   gs_state &g = state(h);
   hipLaunchKernelGGL(kinetic_final, dim3(nst), dim3(256), 0, h.stream,
                      (const double *)g.part, shape(h, nst).nchunk, nst, g.band);
   check_launch();
+}
+
+void precondition_apply(handle &h, cplx *phi, long ld, int nst) {
+  gs_state &g = state(h);
+  preconditioner_kinetic(h, nst);
   const long waves = h.npoint < PRECOND_POINT_WAVES ? h.npoint : PRECOND_POINT_WAVES;
   hipLaunchKernelGGL(precondition_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
                      h.stream, geometry(h), phi, ld, nst, h.npoint, (const double *)g.band);
@@ -628,13 +626,19 @@ void steepest_descent(handle &h, cplx *phi, long ld, int nst, bool precond) {
     GS_REDUCE(residual_partial, rs, h.stream, geometry(h), (const cplx *)g.hphi, rl,
               (const cplx *)phi, ld, g.res, rl, (const double *)g.band, nst, h.npoint, rs.chunk,
               g.part);
-    if (precond) precondition_apply(h, g.res, rl, nst);
-    // H residual and pass 4, in one where the sweeps make H residual
+    // pass 3, H residual and pass 4: in the first and last of the sweeps where they
+    // make H residual
     long mm_rows = nchunk;
     if (gspace_sweeps(h)) {
-      hamiltonian_fourier_sweeps(h, g.res, rl, g.hres, rl, nst, phi, ld, g.part);
+      fourier_extra e{g.res, nullptr, phi, ld, g.part};
+      if (precond) {
+        preconditioner_kinetic(h, nst);
+        e.kinetic = g.band + 5;
+      }
+      hamiltonian_fourier_sweeps(h, g.res, rl, g.hres, rl, nst, &e);
       mm_rows = line_sum_rows(h.n[0], h.n[1]);
     } else {
+      if (precond) precondition_apply(h, g.res, rl, nst);
       hamiltonian_fourier(h, g.res, rl, g.hres, rl, nst);
       GS_REDUCE(mm_partial, rs, h.stream, (const cplx *)phi, ld, (const cplx *)g.res,
                 (const cplx *)g.hres, rl, nst, h.npoint, rs.chunk, g.part);

@@ -631,7 +631,7 @@ void hamiltonian_apply(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld
 // 64^3 x 256 (with the diagonalisation) 55.7 -> 52.2 ms; at 96^3 x 8, whose planes
 // have a CU each and are bound by their transforms, 6013 -> 6043 us.
 void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi, long hld,
-                                int nst, const cplx *line, long line_ld, double *part) {
+                                int nst, const fourier_extra *extra) {
   const projector_tables &t = h.pt;
   const bool project = t.nproj > 0 && t.nunique > 0;
   if (project) projector_phases(h, KA_CURRENT);
@@ -668,12 +668,16 @@ void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi,
     a.xcd = ld % 8 != 0 || hld % 8 != 0;
     a.kin_in = phi + b0;
     a.kin_ld = ld;
-    if (line) {
-      a.mm_phi = line + b0;
-      a.mm_ld = line_ld;
-      a.mm_part = part;
+    if (extra) {
+      a.mm_phi = extra->line + b0;
+      a.mm_ld = extra->line_ld;
+      a.mm_part = extra->part;
       a.mm_nst = nst;
       a.mm_band0 = b0;
+      if (extra->kinetic) {
+        a.pre_psi = extra->phi + b0;
+        a.pre_kin = extra->kinetic + 16 * b0;
+      }
     }
     auto run = [&](fourier_half half) {
       if (h.rect)

@@ -197,11 +197,19 @@ void mfma4_selftest(double *out_device, hipStream_t stream);
 void set_slot(handle &h, int slot, const double v[3]);
 void update_current_slot(handle &h);
 // G-space Hpsi on a three-sweep grid (phi and hphi distinct from the
-// handle's work arrays); with `line`, also the partial sums of the line search
-// over line (ld line_ld), phi and hphi into part (line_sum_rows rows)
+// handle's work arrays); with `extra`, phi (extra->phi) is first scaled in place by
+// K(1/2 |G|^2 / kinetic[16 b]) where kinetic is given, and the partial sums of the
+// line search over line (ld line_ld), phi and hphi go into part (line_sum_rows
+// rows)
+struct fourier_extra {
+  cplx *phi;
+  const double *kinetic;
+  const cplx *line;
+  long line_ld;
+  double *part;
+};
 void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi, long hld,
-                                int nst, const cplx *line = nullptr, long line_ld = 0,
-                                double *part = nullptr);
+                                int nst, const fourier_extra *extra = nullptr);
 void fft3d(handle &h, const cplx *in, long in_ld, cplx *out, long out_ld, int nst, int sign,
            double scale);
 void hamiltonian_apply(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld, int nst,
