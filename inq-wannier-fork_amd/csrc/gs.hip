@@ -16,7 +16,7 @@
 //   pass 4  <r|r>, <phi|r>, <r|Hr>, <phi|Hr> and the step lambda per band (on
 //           three-sweep grids in the sweep that writes H residual)
 //   pass 5  phi += lambda r, hphi += lambda Hr (with the next step's pass-1 sums)
-// orthogonalize forms S = dV Phi^H Phi (a split-K strided-batched ZGEMM),
+// orthogonalize forms S = dV Phi^H Phi (gram.hip),
 // factors it (S = R R^H, R lower: cholesky.hip) and applies Phi <- Phi R^-H
 // with ZGEMM; the subspace diagonalisation diagonalises dV Phi^H H Phi with
 // rocSOLVER ZHEEVD.
@@ -45,7 +45,6 @@ namespace {
 constexpr long GS_CHUNK = 512;
 constexpr long GS_CHUNK_MIN = 64;
 constexpr long GS_BLOCKS = 2048;
-constexpr int IP_BATCHES = 64;  // point chunks of the split-K inner products
 
 struct gs_state {
   cplx *hphi = nullptr, *res = nullptr, *hres = nullptr;  // [N][max_bands] each
@@ -56,7 +55,7 @@ struct gs_state {
   cplx *T = nullptr;        // [max_bands]^2 rotation of orthogonalize
   cplx *chol = nullptr;     // scratch of the Cholesky factorisation
   double *eig = nullptr;    // [2 max_bands] eigenvalues + tridiagonal work
-  cplx *ip_part = nullptr;  // [IP_BATCHES + 1][max_bands]^2 split-K inner-product partials
+  cplx *ip_part = nullptr;  // [max_bands]^2 scratch of inner products in one slice
   rocblas_int *info = nullptr;
 };
 
@@ -136,7 +135,7 @@ void ensure_blas(handle &h) {
   if (!g.eig) g.eig = (double *)dalloc((size_t)2 * h.max_bands * sizeof(double));
   if (!g.info) g.info = (rocblas_int *)dalloc(sizeof(rocblas_int));
   if (!g.ip_part)
-    g.ip_part = (cplx *)dalloc((size_t)(IP_BATCHES + 1) * h.max_bands * h.max_bands * sizeof(cplx));
+    g.ip_part = (cplx *)dalloc((size_t)h.max_bands * h.max_bands * sizeof(cplx));
   GS_BLAS_CHECK(rocblas_set_stream(g.blas, h.stream));
 }
 
@@ -461,50 +460,14 @@ __global__ __launch_bounds__(256) void sd_update_eig_norm(cplx *__restrict__ phi
 
 void check_launch() { INQAMD_HIP_CHECK(hipGetLastError()); }
 
-// out[i] = sum over the partial slices of part (fixed order)
-__global__ __launch_bounds__(256) void slice_sum_kernel(const cplx *__restrict__ part, int nslice,
-                                                        long n, cplx *__restrict__ out) {
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-    cplx s = part[i];
-    for (int k = 1; k < nslice; k++) s = cadd(s, part[(long)k * n + i]);
-    out[i] = s;
-  }
-}
-
-// Row-major M[r][c] = alpha sum_p conj(A[p][r]) B[p][c] over all grid points
-// (operations::overlap, overlap.hpp:26-60, as a BLAS gemm H(A) B).  The
-// point sum is long and the output small, so it is split over IP_BATCHES
-// point chunks (a strided-batched ZGEMM; one gemm over all points would keep
-// only (nst/64)^2 workgroups busy) and the chunk results are summed in order.
+// Row-major Hermitian M[r][c] = alpha sum_p conj(A[p][r]) B[p][c] over all grid
+// points (operations::overlap, overlap.hpp:26-60).  Uses hn2.
 void inner_products(handle &h, const cplx *A, long lda, const cplx *B, long ldb, int nst,
                     double alpha, cplx *out) {
   ensure_blas(h);
-  gs_state &g = state(h);
-  const long N = h.npoint;
-  const int nb = (int)(N >= 256L * IP_BATCHES ? IP_BATCHES : 1);
-  const long kc = N / nb, rem = N - kc * nb;
-  const rocblas_stride sc = (rocblas_stride)nst * nst;
-  const rocblas_double_complex a = {alpha, 0.0}, zero = {0.0, 0.0};
-  // column-major C_b(c, r) = sum_{p in chunk b} B[p][c] conj(A[p][r]) is the
-  // row-major M_b[r][c]
-  GS_BLAS_CHECK(rocblas_zgemm_strided_batched(
-      g.blas, rocblas_operation_none, rocblas_operation_conjugate_transpose, nst, nst,
-      (rocblas_int)kc, &a, reinterpret_cast<const rocblas_double_complex *>(B), (int)ldb,
-      (rocblas_stride)(kc * ldb), reinterpret_cast<const rocblas_double_complex *>(A), (int)lda,
-      (rocblas_stride)(kc * lda), &zero, reinterpret_cast<rocblas_double_complex *>(g.ip_part),
-      nst, sc, nb));
-  int nslice = nb;
-  if (rem > 0) {
-    GS_BLAS_CHECK(rocblas_zgemm(
-        g.blas, rocblas_operation_none, rocblas_operation_conjugate_transpose, nst, nst,
-        (rocblas_int)rem, &a, reinterpret_cast<const rocblas_double_complex *>(B + kc * nb * ldb),
-        (int)ldb, reinterpret_cast<const rocblas_double_complex *>(A + kc * nb * lda), (int)lda,
-        &zero, reinterpret_cast<rocblas_double_complex *>(g.ip_part + (long)nb * sc), nst));
-    nslice++;
-  }
-  hipLaunchKernelGGL(slice_sum_kernel, dim3(grid1(sc)), dim3(256), 0, h.stream,
-                     (const cplx *)g.ip_part, nslice, (long)sc, out);
-  check_launch();
+  // (several slices take at most a quarter of hn2)
+  cplx *part = gram_slices(h.npoint, nst) > 1 ? h.hn2 : state(h).ip_part;
+  gram(A, lda, B, ldb, nst, h.npoint, alpha, part, out, h.stream);
 }
 
 // The K(1/2|G|^2/kinetic) scaling of operations::preconditioner for

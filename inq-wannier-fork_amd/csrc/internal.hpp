@@ -196,6 +196,11 @@ void mfma4_selftest(double *out_device, hipStream_t stream);
 // hamiltonian.hip
 void set_slot(handle &h, int slot, const double v[3]);
 void update_current_slot(handle &h);
+// gram.hip: row-major Hermitian out[r][c] = alpha sum_p conj(A[p][r]) B[p][c], with
+// gram_slices(npoint, nst) nst^2 values of scratch in part
+int gram_slices(long npoint, int nst);
+void gram(const cplx *A, long lda, const cplx *B, long ldb, int nst, long npoint, double alpha,
+          cplx *part, cplx *out, hipStream_t stream);
 // G-space Hpsi on a three-sweep grid (phi and hphi distinct from the
 // handle's work arrays); with `extra`, phi (extra->phi) is first scaled in place by
 // K(1/2 |G|^2 / kinetic[16 b]) where kinetic is given, and the partial sums of the
