@@ -15,9 +15,9 @@
 // order.
 //
 // A strided-batched library product formed the whole square and idled most of its
-// 64 x 64 tiles at few bands: 40^3 x 48 bands 118 -> 35 us, 96^3 x 8 1506 us -> a
-// tenth of it; steepest descent there 1623 -> 1534 and 5246 -> 3805 us, at 64^3 x
-// 20 3134 -> 2726 us, at 30 x 36 x 40 x 130 3396 -> 3246 us, the ground-state step
+// 64 x 64 tiles at few bands: 40^3 x 48 bands 118 -> 35 us, 96^3 x 8 1506 -> about
+// 65 us; steepest descent there 1623 -> 1534 and 5246 -> 3805 us, at 64^3 x 20
+// 3134 -> 2726 us, at 30 x 36 x 40 x 130 3396 -> 3246 us, the ground-state step
 // at 64^3 x 256 50.7 -> 49.4 ms.
 #include "internal.hpp"
 #include "projector_dev.hpp"

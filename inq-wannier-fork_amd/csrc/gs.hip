@@ -15,7 +15,8 @@
 //   H residual (G-space Hpsi)
 //   pass 4  <r|r>, <phi|r>, <r|Hr>, <phi|Hr> and the step lambda per band (on
 //           three-sweep grids in the sweep that writes H residual)
-//   pass 5  phi += lambda r, hphi += lambda Hr (with the next step's pass-1 sums)
+//   pass 5  phi += lambda r, hphi += lambda Hr, with pass 2 of the next step, whose
+//           eig and norm follow from this step's sums
 // orthogonalize forms S = dV Phi^H Phi (gram.hip),
 // factors it (S = R R^H, R lower: cholesky.hip) and applies Phi <- Phi R^-H
 // with ZGEMM; the subspace diagonalisation diagonalises dV Phi^H H Phi with
@@ -338,7 +339,8 @@ __global__ __launch_bounds__(256) void kinetic_final(const double *part, long nc
   if (threadIdx.x == 0) band[b * 16 + 5] = t[0] / t[1];
 }
 
-// steepest_descent.hpp:56-68
+// lambda (steepest_descent.hpp:56-68), and the eig and norm of phi + lambda r from
+// those of phi and the same sums: <r|H phi> = conj(<phi|H r>), lambda is real
 __global__ __launch_bounds__(256) void lambda_final(const double *part, long nchunk, int nst,
                                                     double dV, double *band) {
   const int b = blockIdx.x;
@@ -355,7 +357,15 @@ __global__ __launch_bounds__(256) void lambda_final(const double *part, long nch
   const double cb = re(m5r, 0.0, m[4], m[5]) - re(m4r, m4i, m[0], m[1]);
   const double cc = re(m4r, m4i, m[2], m[3]) - re(m[6], m[7], m5r, 0.0);
   const double den = cb + sqrt(cb * cb - 4.0 * ca * cc);
-  band[b * 16 + 6] = fabs(den) < 1e-15 ? 0.0 : 2.0 * cc / den;
+  const double lam = fabs(den) < 1e-15 ? 0.0 : 2.0 * cc / den;
+  band[b * 16 + 6] = lam;
+  const double er = m4r + lam * (2.0 * m[6] + lam * m[4]), ei = m4i - lam * lam * m[5];
+  const double nn = m5r + lam * (2.0 * m[2] + lam * m[0]);
+  band[b * 16 + 0] = er;
+  band[b * 16 + 1] = ei;
+  band[b * 16 + 2] = nn;
+  band[b * 16 + 3] = er / nn;
+  band[b * 16 + 4] = ei / nn;
 }
 
 // pass 3: phi(G) *= K(1/2 |G|^2 / kinetic_b) (preconditioner.hpp:45-52).
@@ -418,21 +428,23 @@ __global__ __launch_bounds__(256) void sd_update_phi(cplx *__restrict__ phi, lon
   }
 }
 
-// pass 5 of a step fused with pass 1 of the next (the partial sums of
-// eig_norm_partial over the updated phi and hphi, in its order), for steps
-// that update hphi
+// pass 5 of a step fused with pass 2 of the next: the residual of the updated phi
+// and hphi over the old one.  Seven arrays move instead of the nine of an update
+// with the sums of eig and norm and a residual pass after it: steepest descent at
+// 40^3 x 48 bands 1535 -> 1479 us, at 64^3 x 256 with the diagonalisation 49.5 ->
+// 48.0 ms.
 template <int BT>
-__global__ __launch_bounds__(256) void sd_update_eig_norm(cplx *__restrict__ phi, long ld,
-                                                          const cplx *__restrict__ res,
+__global__ __launch_bounds__(256) void sd_update_residual(gspace geo, cplx *__restrict__ phi,
+                                                          long ld, cplx *__restrict__ res,
                                                           cplx *__restrict__ hphi,
                                                           const cplx *__restrict__ hres, long rld,
                                                           int nst, long npoint,
                                                           const double *__restrict__ band,
                                                           long chunk, double *part) {
-  band_partials<3, BT>(npoint, chunk, nst, part, [&](long p, int b, double *a) {
-    const double lam = band[b * 16 + 6];
+  band_partials<2, BT>(npoint, chunk, nst, part, [&](long p, int b, double *a) {
+    const double er = band[b * 16 + 3], ei = band[b * 16 + 4], lam = band[b * 16 + 6];
     cplx f = phi[p * ld + b];
-    const cplx r = res[p * rld + b];
+    cplx r = res[p * rld + b];
     cplx h = hphi[p * rld + b];
     const cplx hr = hres[p * rld + b];
     f.x += lam * r.x;
@@ -441,9 +453,15 @@ __global__ __launch_bounds__(256) void sd_update_eig_norm(cplx *__restrict__ phi
     h.y += lam * hr.y;
     phi[p * ld + b] = f;
     hphi[p * rld + b] = h;
-    a[0] += h.x * f.x + h.y * f.y;
-    a[1] += h.x * f.y - h.y * f.x;
-    a[2] += f.x * f.x + f.y * f.y;
+    r.x = h.x + (-1.0) * (er * f.x - ei * f.y);
+    r.y = h.y + (-1.0) * (er * f.y + ei * f.x);
+    res[p * rld + b] = r;
+    int m0, m1, m2;
+    geo.m_of(p, m0, m1, m2);
+    const double lap = -0.5 * (-geo.g2(m0, m1, m2));
+    const double r2 = r.x * r.x + r.y * r.y;
+    a[0] += lap * r2;
+    a[1] += r2;
   });
 }
 
@@ -578,17 +596,17 @@ void steepest_descent(handle &h, cplx *phi, long ld, int nst, bool precond) {
   hamiltonian_fourier(h, phi, ld, g.hphi, rl, nst);
   const int num_steps = 5;
   for (int istep = 0; istep < num_steps; istep++) {
-    // pass 1 (after the first step, the previous step's update made its sums)
+    // passes 1 and 2 (after the first step, pass 4's sums and the last update)
     if (istep == 0) {
       GS_REDUCE(eig_norm_partial, rs, h.stream, (const cplx *)g.hphi, rl, (const cplx *)phi, ld,
                 nst, h.npoint, rs.chunk, g.part);
+      hipLaunchKernelGGL(eig_norm_final, fg, dim3(256), 0, h.stream, (const double *)g.part,
+                         nchunk, nst, dV, g.band);
+      check_launch();
+      GS_REDUCE(residual_partial, rs, h.stream, geometry(h), (const cplx *)g.hphi, rl,
+                (const cplx *)phi, ld, g.res, rl, (const double *)g.band, nst, h.npoint, rs.chunk,
+                g.part);
     }
-    hipLaunchKernelGGL(eig_norm_final, fg, dim3(256), 0, h.stream, (const double *)g.part, nchunk,
-                       nst, dV, g.band);
-    check_launch();
-    GS_REDUCE(residual_partial, rs, h.stream, geometry(h), (const cplx *)g.hphi, rl,
-              (const cplx *)phi, ld, g.res, rl, (const double *)g.band, nst, h.npoint, rs.chunk,
-              g.part);
     // pass 3, H residual and pass 4: in the first and last of the sweeps where they
     // make H residual
     long mm_rows = nchunk;
@@ -610,7 +628,7 @@ void steepest_descent(handle &h, cplx *phi, long ld, int nst, bool precond) {
                        nst, dV, g.band);
     check_launch();
     if (istep != num_steps - 1)
-      GS_REDUCE(sd_update_eig_norm, rs, h.stream, phi, ld, (const cplx *)g.res, g.hphi,
+      GS_REDUCE(sd_update_residual, rs, h.stream, geometry(h), phi, ld, g.res, g.hphi,
                 (const cplx *)g.hres, rl, nst, h.npoint, (const double *)g.band, rs.chunk, g.part);
     else
       GS_REDUCE(sd_update_phi, rs, h.stream, phi, ld, (const cplx *)g.res, rl, nst, h.npoint,
