@@ -18,8 +18,8 @@
 //   pass 5  phi += lambda r, hphi += lambda Hr, with pass 2 of the next step, whose
 //           eig and norm follow from this step's sums
 // orthogonalize forms S = dV Phi^H Phi (gram.hip),
-// factors it (S = R R^H, R lower: cholesky.hip) and applies Phi <- Phi R^-H
-// with ZGEMM; the subspace diagonalisation diagonalises dV Phi^H H Phi with
+// factors it (S = R R^H, R lower: cholesky.hip) and applies Phi <- Phi R^-H in
+// place (rotate.hip); the subspace diagonalisation diagonalises dV Phi^H H Phi with
 // rocSOLVER ZHEEVD.
 
 #include <rocblas/rocblas.h>
@@ -554,6 +554,24 @@ void preconditioner(handle &h, cplx *phi, long ld, int nst) {
   precondition_apply(h, phi, ld, nst);
 }
 
+// Phi <- Phi T (row-major T, `upper` triangular with zeros below): out[p][j] =
+// sum_i phi[p][i] T[i][j].  Bands beyond LDS go through a ZGEMM into hn, as the
+// column-major out^T = T_cm * Phi^T.
+static void rotate_bands(handle &h, cplx *phi, long ld, int nst, bool upper) {
+  gs_state &g = state(h);
+  if (rotate_supported(nst, h.max_lds)) {
+    rotate(phi, ld, nst, h.npoint, g.T, upper, h.max_lds, h.stream);
+    return;
+  }
+  const rocblas_double_complex one = {1.0, 0.0}, zero = {0.0, 0.0};
+  GS_BLAS_CHECK(rocblas_zgemm(g.blas, rocblas_operation_none, rocblas_operation_none, nst,
+                              (rocblas_int)h.npoint, nst, &one,
+                              reinterpret_cast<const rocblas_double_complex *>(g.T), nst,
+                              reinterpret_cast<const rocblas_double_complex *>(phi), (int)ld,
+                              &zero, reinterpret_cast<rocblas_double_complex *>(h.hn), nst));
+  copy(h, h.hn, nst, phi, ld, nst);
+}
+
 // operations::orthogonalize (orthogonalize.hpp:25-32): S = dV Phi^H Phi,
 // S = R R^H (R lower: zpotrf on the row-major S, cholesky.hpp:29-80),
 // Phi <- Phi R^-H (invert_triangular + rotate, rotate.hpp:147-156).
@@ -571,15 +589,7 @@ void orthogonalize(handle &h, cplx *phi, long ld, int nst, double dV) {
   if (band >= 0)
     throw error{ERR_ARGUMENT, "orthogonalize: overlap matrix is not positive definite (band " +
                                   std::to_string(band) + ")"};
-  // out[p][j] = sum_i phi[p][i] T[i][j]: column-major out^T = T_cm * Phi^T
-  // with T_cm (ld nst) the row-major T read column-major
-  const rocblas_double_complex one = {1.0, 0.0}, zero = {0.0, 0.0};
-  GS_BLAS_CHECK(rocblas_zgemm(g.blas, rocblas_operation_none, rocblas_operation_none, nst,
-                              (rocblas_int)h.npoint, nst, &one,
-                              reinterpret_cast<const rocblas_double_complex *>(g.T), nst,
-                              reinterpret_cast<const rocblas_double_complex *>(phi), (int)ld,
-                              &zero, reinterpret_cast<rocblas_double_complex *>(h.hn), nst));
-  copy(h, h.hn, nst, phi, ld, nst);
+  rotate_bands(h, phi, ld, nst, true);
 }
 
 // eigensolvers::steepest_descent (steepest_descent.hpp:23-88) on
@@ -649,19 +659,13 @@ void subspace_diagonalization(handle &h, cplx *phi, long ld, int nst, double *ei
   // H_sub[r][c] = dV sum_p conj(phi[p][r]) hphi[p][c], row-major (dV = V/N);
   // read as a column-major matrix that is conj(H_sub)
   inner_products(h, phi, ld, g.hphi, nst, nst, h.volume / (double)h.npoint, g.S);
-  const rocblas_double_complex zero = {0.0, 0.0}, one = {1.0, 0.0};
   // eigenvectors w_k of conj(H_sub) are conj(v_k), v_k those of H_sub
   GS_BLAS_CHECK(rocsolver_zheevd(g.blas, rocblas_evect_original, rocblas_fill_upper, nst,
                                  reinterpret_cast<rocblas_double_complex *>(g.S), nst, g.eig,
                                  g.eig + h.max_bands, g.info));
-  // out[p][k] = sum_i phi[p][i] v_k[i] = sum_i phi[p][i] conj(W(i, k)):
-  // column-major out^T = W^H Phi^T
-  GS_BLAS_CHECK(rocblas_zgemm(g.blas, rocblas_operation_conjugate_transpose,
-                              rocblas_operation_none, nst, (rocblas_int)h.npoint, nst, &one,
-                              reinterpret_cast<const rocblas_double_complex *>(g.S), nst,
-                              reinterpret_cast<const rocblas_double_complex *>(phi), (int)ld,
-                              &zero, reinterpret_cast<rocblas_double_complex *>(h.hn), nst));
-  copy(h, h.hn, nst, phi, ld, nst);
+  // out[p][k] = sum_i phi[p][i] v_k[i] = sum_i phi[p][i] conj(W(i, k))
+  adjoint_matrix(g.S, nst, g.T, h.stream);
+  rotate_bands(h, phi, ld, nst, false);
   rocblas_int info = 0;
   INQAMD_HIP_CHECK(hipMemcpyAsync(eig_host, g.eig, (size_t)nst * sizeof(double),
                                   hipMemcpyDeviceToHost, h.stream));

@@ -201,6 +201,13 @@ void update_current_slot(handle &h);
 int gram_slices(long npoint, int nst);
 void gram(const cplx *A, long lda, const cplx *B, long ldb, int nst, long npoint, double alpha,
           cplx *part, cplx *out, hipStream_t stream);
+// rotate.hip: phi <- phi M in place, M row-major nst x nst (upper triangular with
+// zeros below, or full), where 16 rows of phi fit in LDS
+bool rotate_supported(int nst, size_t max_lds);
+void rotate(cplx *phi, long ld, int nst, long npoint, const cplx *M, bool upper, size_t max_lds,
+            hipStream_t stream);
+// out[i][k] = conj(W[k][i]), both row-major n x n
+void adjoint_matrix(const cplx *W, int n, cplx *out, hipStream_t stream);
 // G-space Hpsi on a three-sweep grid (phi and hphi distinct from the
 // handle's work arrays); with `extra`, phi (extra->phi) is first scaled in place by
 // K(1/2 |G|^2 / kinetic[16 b]) where kinetic is given, and the partial sums of the
