@@ -245,4 +245,9 @@ bool fft3_rect_projector(const int n[3], int nb);
 void fft3_rect_fourier_hamiltonian(const fft3_args &a, const int n[3], hipStream_t stream,
                                    fourier_half half);
 
+// G-space moments of the chunk's bands from W after the z forward sweep, rows
+// [nb n[2]][8] (fft3_rect.hip; cubic grids too); where both plane axes have plans
+bool fft3_moments_supported(const int n[3], size_t max_lds);
+void fft3_moments(const fft3_args &a, const int n[3], double *rows, hipStream_t stream);
+
 }  // namespace inqamd

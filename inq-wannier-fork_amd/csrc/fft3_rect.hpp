@@ -8,10 +8,11 @@
 // Five pencil passes move 176 B per point and band and add V_nl psi and the
 // Taylor terms in passes of their own; the three sweeps move 112 with both
 // fused.  Against the pencil passes: Hpsi at 48 x 60 x 72 x 101 bands 817 -> 738
-// us, at 25 x 45 x 27 x 45 86 -> 67 us, at 80 x 90 x 96 x 20 508 -> 499 us; the
-// ETRS step at 32 x 25 x 90 x 60 1519 -> 1295 us, the interacting step at 60 x
-// 36 x 27 x 43 2.53 -> 2.07 ms, the adjoint of 8 steps at 20 x 60 x 36 x 12
-// (whose fused half steps need the sweeps) 20.1 -> 11.3 ms.
+// us (674 since its z tiles are dealt per XCD), at 25 x 45 x 27 x 45 86 -> 67 us,
+// at 80 x 90 x 96 x 20 508 -> 499 us; the ETRS step at 32 x 25 x 90 x 60 1519 ->
+// 1295 us, the interacting step at 60 x 36 x 27 x 43 2.53 -> 2.07 ms, the adjoint
+// of 8 steps at 20 x 60 x 36 x 12 (whose fused half steps need the sweeps) 20.1 ->
+// 11.3 ms.
 #pragma once
 
 #include "fft3_tiles.hpp"

@@ -691,6 +691,28 @@ void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi,
   }
 }
 
+bool gspace_sums_supported(const handle &h) {
+  return h.three_sweep && fft3_moments_supported(h.n, h.max_lds);
+}
+
+void gspace_sums(handle &h, const cplx *psi, long ld, int nst, double *rows) {
+  const band_chunks plan = chunk_plan(h, nst, ld, true);
+  for (int c = 0; c < plan.n; c++) {
+    const int b0 = plan.b0(c), nb = plan.nb(c);
+    local_passes(h, psi + b0, ld, nullptr, 0, nb, KA_CURRENT, b0, nst, nullptr, 0, h.stream, h.work,
+                 plan.gskip, plan.glog);
+    fft3_args a{};
+    a.W = h.work;
+    a.nb = nb;
+    a.nx = h.n[0];
+    a.ny = h.n[1];
+    a.twx = h.axis[0].tw;
+    a.twy = h.axis[1].tw;
+    fft3_moments(a, h.n, rows, h.stream);
+    rows += (long)nb * h.n[2] * 8;
+  }
+}
+
 void shift(handle &h, std::complex<double> c, const cplx *x, long xld, cplx *y, long yld,
                   int nst) {
   const long total = h.npoint * nst;

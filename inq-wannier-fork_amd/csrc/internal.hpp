@@ -222,6 +222,10 @@ struct fourier_extra {
 };
 void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi, long hld,
                                 int nst, const fourier_extra *extra = nullptr);
+// G-space moments sum_G |psi^|^2 m_c of each (band, z plane) into rows
+// [nst n[2]][8] on three-sweep grids with gspace_sums_supported; uses work
+bool gspace_sums_supported(const handle &h);
+void gspace_sums(handle &h, const cplx *psi, long ld, int nst, double *rows);
 void fft3d(handle &h, const cplx *in, long in_ld, cplx *out, long out_ld, int nst, int sign,
            double scale);
 void hamiltonian_apply(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld, int nst,

@@ -687,6 +687,20 @@ static void gspace_record(handle &h, const cplx *Xh, const cplx *Yh, long ld, in
   INQAMD_HIP_CHECK(hipGetLastError());
 }
 
+// The same of psi with itself (record[0..7], imaginary parts 0); uses work and hn
+static void psi_record(handle &h, const cplx *psi, long ld, int nst, double *rec) {
+  if (!gspace_sums_supported(h)) {
+    fft3d(h, psi, ld, h.work, nst, nst, -1, 1.0);
+    gspace_record(h, h.work, h.work, nst, nst, rec);
+    return;
+  }
+  double *rows = reinterpret_cast<double *>(h.hn);
+  gspace_sums(h, psi, ld, nst, rows);
+  hipLaunchKernelGGL(sum_rows_kernel, dim3(8), dim3(SUM_ROWS_NT), 0, h.stream,
+                     (const double *)rows, nst * h.n[2], 8, rec);
+  INQAMD_HIP_CHECK(hipGetLastError());
+}
+
 // record[8..25] = sphere pair sums of (mX, mY), weighted by coeff
 // [nproj][max_nlm] (the KB coefficients, or commutator_coeff's)
 static void nl_record(handle &h, const cplx *mX, const cplx *mY, int nb, double *rec,
@@ -1201,9 +1215,8 @@ int inqamd_current(inqamd_hamiltonian_t h, const void *psi, int nst, int ld, dou
     INQAMD_REQUIRE(J_cov && J_cart, "outputs are null");
     const cplx *f = (const cplx *)psi;
     double *rec = obs_record(*h, 0);
-    // G-space moments of |psi^|^2 (transform.hpp:337-367 into the workspace)
-    fft3d(*h, f, ld, h->work, nst, nst, -1, 1.0);
-    gspace_record(*h, h->work, h->work, nst, nst, rec);
+    // G-space moments of |psi^|^2 (transform.hpp:337-367)
+    psi_record(*h, f, ld, nst, rec);
     // sphere moments with the Cartesian components of the relative positions
     double L[9];
     for (int c = 0; c < 3; c++)
@@ -1333,8 +1346,7 @@ int inqamd_td_forward(inqamd_td_t td, const double *coeff, const void *psi0, int
     double L[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     lattice_dot(*h, d.direction, L);
     double *rec = obs_record(*h, 0);
-    fft3d(*h, state, nst, h->work, nst, nst, -1, 1.0);
-    gspace_record(*h, h->work, h->work, nst, nst, rec);
+    psi_record(*h, state, nst, nst, rec);
     sphere_moments(*h, state, nst, nst, L, false, h->mom_a);
     nl_record(*h, h->mom_a, h->mom_a, nst, rec, commutator_coeff(*h, d.commutator));
     pair_weights w = make_weights(*h, d.direction, kT);
