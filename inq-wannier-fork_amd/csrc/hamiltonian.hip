@@ -443,6 +443,16 @@ static void local_passes(handle &h, const cplx *psi, long ld, cplx *hpsi, long h
   fft_launch_pass(ep, FFT_EPILOGUE, h.stream);
 }
 
+// The library's own choice of bands per chunk
+static int default_band_chunk(const handle &h, int nst) {
+  // at least 192 MiB of intermediate and 24 bands per chunk: measured
+  // fastest at 64^3 x 256 (48 bands; 32 and 64 were 6 % slower) and at
+  // 96^3 x 512 (24 bands; 8 and 16 were 4-9 % slower)
+  long c = (192L << 20) / (h.npoint * (long)sizeof(cplx));
+  c = c < 24 ? 24 : c / 8 * 8;
+  return c < nst ? (int)c : nst;
+}
+
 // Bands per chunk of the local passes (0: all bands at once).  A chunk's
 // intermediate array can stay cache-resident between passes.
 static int band_chunk(const handle &h, int nst) {
@@ -452,12 +462,7 @@ static int band_chunk(const handle &h, int nst) {
   }();
   if (h.tune_chunk > 0) return h.tune_chunk < nst ? h.tune_chunk : nst;
   if (forced >= 0) return forced == 0 ? nst : forced;
-  // at least 192 MiB of intermediate and 24 bands per chunk: measured
-  // fastest at 64^3 x 256 (48 bands; 32 and 64 were 6 % slower) and at
-  // 96^3 x 512 (24 bands; 8 and 16 were 4-9 % slower)
-  long c = (192L << 20) / (h.npoint * (long)sizeof(cplx));
-  c = c < 24 ? 24 : c / 8 * 8;
-  return c < nst ? (int)c : nst;
+  return default_band_chunk(h, nst);
 }
 
 // Band chunks of the three-sweep Hpsi.  Where rows are a multiple of 4 KB
@@ -630,6 +635,11 @@ void hamiltonian_apply(handle &h, const cplx *psi, long ld, cplx *hpsi, long hld
 // 1673 us, at 64^3 x 20 3546 -> 3303 us, at 48 x 50 x 54 x 40 3070 -> 2909 us, at
 // 64^3 x 256 (with the diagonalisation) 55.7 -> 52.2 ms; at 96^3 x 8, whose planes
 // have a CU each and are bound by their transforms, 6013 -> 6043 us.
+//
+// The projector's point sums are split as for the library's own chunk whatever the
+// chunk in use, so that no band's bits depend on it (by all bands the spheres of
+// 64 atoms would go unsplit from 57 bands on and a chunk's launch leave half the
+// chip idle).
 void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi, long hld,
                                 int nst, const fourier_extra *extra) {
   const projector_tables &t = h.pt;
@@ -686,7 +696,9 @@ void hamiltonian_fourier_sweeps(handle &h, const cplx *phi, long ld, cplx *hphi,
         fft3_fourier_hamiltonian(a, h.n[0], h.stream, half);
     };
     run(G_INVERSE);
-    if (project) projector_project_expand(h, h.hn, nb, nb, h.vnl, nb, false, t.zrow);
+    if (project)
+      projector_project_expand(h, h.hn, nb, nb, h.vnl, nb, false, t.zrow,
+                               default_band_chunk(h, nst));
     run(G_FORWARD);
   }
 }

@@ -172,9 +172,12 @@ void projector_apply_coefficients(handle &h, cplx *hpsi, long ld, int nst, int s
 // Q[u][b] = the same sum for every owned grid point u (compact, ld = nst)
 void projector_owned_sum(handle &h, cplx *Q, int nst, int slot);
 // projector_mfma.hip: gather + MFMA GEMM1 (-> P if write_P) + MFMA GEMM2 ->
-// per-entry V_nl psi in Qe (if Qe != nullptr)
+// per-entry V_nl psi in Qe (if Qe != nullptr).  The order of the point sum follows
+// from nst_split bands (0: nst), not from nst: a caller that comes band chunk by
+// band chunk passes the same nst_split for each, and a band gets the same bits in
+// any chunk.
 void projector_project_expand(handle &h, const cplx *psi, long ld, int nst, cplx *Qe, long ldQ,
-                              bool write_P, const int *point = nullptr);
+                              bool write_P, const int *point = nullptr, int nst_split = 0);
 void mfma_selftest(double *out_device, hipStream_t stream);
 // P coefficients of all spheres and bands on the 4x4x4 FP64 MFMA (max_nlm <= 4)
 void projector_project_p4(handle &h, const cplx *psi, long ld, int nst);

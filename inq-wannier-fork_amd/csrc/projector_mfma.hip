@@ -88,9 +88,30 @@ __global__ void mfma_selftest_kernel(double *out) {
 }
 
 void projector_project_expand(handle &h, const cplx *psi, long ld, int nst, cplx *Qe, long ldQ,
-                              bool write_P, const int *point) {
+                              bool write_P, const int *point, int nst_split) {
   const projector_tables &t = h.pt;
   if (t.nproj == 0) return;
+  if (nst_split == 0) nst_split = nst;
+  // few (sphere, band tile) pairs: split the sphere points over workgroups
+  const long tiles = (long)((nst_split + PE_BANDS - 1) / PE_BANDS) * t.nproj;
+  int nc = 1;
+  if (tiles < 512 && h.proj_part) {
+    nc = (int)((1024 + tiles - 1) / tiles);
+    const int by_points = t.max_sphere / 256 > 1 ? t.max_sphere / 256 : 1;
+    if (nc > by_points) nc = by_points;
+    if (nc > PROJ_MAX_CHUNKS) nc = PROJ_MAX_CHUNKS;
+    if (tiles * nc > PROJ_PART_TILES) nc = (int)(PROJ_PART_TILES / tiles);
+    if (nc < 1) nc = 1;
+  }
+  // (more bands than nst_split: in ranges whose partial tiles fit)
+  const int fit = nc == 1 ? nst : (int)(PROJ_PART_TILES / ((long)nc * t.nproj)) * PE_BANDS;
+  if (nst > fit) {
+    INQAMD_REQUIRE(!write_P, "projector coefficients need nst_split = nst");
+    for (int b = 0; b < nst; b += fit)
+      projector_project_expand(h, psi + b, ld, nst - b < fit ? nst - b : fit, Qe + b, ldQ, false,
+                               point, nst_split);
+    return;
+  }
   project_expand_args a;
   a.psi = psi;
   a.ld = ld;
@@ -108,17 +129,6 @@ void projector_project_expand(handle &h, const cplx *psi, long ld, int nst, cplx
   a.Qe = Qe;
   a.ldQ = ldQ;
   const int nbt = (nst + PE_BANDS - 1) / PE_BANDS;
-  const long tiles = (long)nbt * t.nproj;
-  // few (sphere, band tile) pairs: split the sphere points over workgroups
-  int nc = 1;
-  if (tiles < 512 && h.proj_part) {
-    nc = (int)((1024 + tiles - 1) / tiles);
-    const int by_points = t.max_sphere / 256 > 1 ? t.max_sphere / 256 : 1;
-    if (nc > by_points) nc = by_points;
-    if (nc > PROJ_MAX_CHUNKS) nc = PROJ_MAX_CHUNKS;
-    if (tiles * nc > PROJ_PART_TILES) nc = (int)(PROJ_PART_TILES / tiles);
-    if (nc < 1) nc = 1;
-  }
   if (nc == 1) {
     dim3 grid(nbt, t.nproj);
     hipLaunchKernelGGL(project_expand_kernel, grid, dim3(PE_NT), 0, h.stream, a);
