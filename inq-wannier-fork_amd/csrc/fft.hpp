@@ -246,7 +246,8 @@ void fft3_rect_fourier_hamiltonian(const fft3_args &a, const int n[3], hipStream
                                    fourier_half half);
 
 // G-space moments of the chunk's bands from W after the z forward sweep, rows
-// [nb n[2]][8] (fft3_rect.hip; cubic grids too); where both plane axes have plans
+// [nst n[2]][8] offset to the chunk's first band, bands at the offsets that they
+// have in psi (fft3_rect.hip; cubic grids too); where both plane axes have plans
 bool fft3_moments_supported(const int n[3], size_t max_lds);
 void fft3_moments(const fft3_args &a, const int n[3], double *rows, hipStream_t stream);
 

@@ -283,8 +283,9 @@ __device__ __forceinline__ void rect_real_plane(const fft3_args &a, int nz, long
 
 // Plane `plane` = band * nz + z of W (psi transformed in z): the sums of |psi^|^2 m_c
 // over the plane, m_0 = 1 and m_1..3 the symmetric indices (x, y, z), into
-// rows[plane][8] (complex, like the other G-space moments).  Nothing is written
-// back: two sweeps, 48 N bytes per band, where three pencil passes and a pass over
+// rows[offset of the band in psi x nz + z][8] (complex, like the other G-space
+// moments), so that the order of their sum is the same for any chunks.  Nothing is
+// written back: two sweeps, 48 N bytes per band, where three pencil passes and a pass over
 // their result moved 112 (density, dipole, energies and current of 36 x 36 x 90 x 48
 // bands 540 -> 496 us, of 64^3 x 64 1130 -> 1033 us, of 96^3 x 8 878 -> 827 us).
 template <int NT>
@@ -330,11 +331,12 @@ __device__ __forceinline__ void rect_moments_plane(const fft3_args &a, int nz, l
   if (threadIdx.x != 0) return;
   for (int w = 1; w < NT / 64; w++)
     for (int k = 0; k < 3; k++) s[k] += red[w * 3 + k];
-  double *r = rows + plane * 8;
+  const int cb = (int)(plane / nz), z = (int)(plane - (long)cb * nz);
+  double *r = rows + ((long)(cb + (cb >> (3 + a.glog)) * a.gskip) * nz + z) * 8;
   r[0] = s[0];
   r[2] = s[1];
   r[4] = s[2];
-  r[6] = symmetric_index((int)(plane % nz), nz) * s[0];
+  r[6] = symmetric_index(z, nz) * s[0];
   r[1] = r[3] = r[5] = r[7] = 0.0;
 }
 

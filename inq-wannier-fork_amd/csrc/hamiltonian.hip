@@ -720,8 +720,9 @@ void gspace_sums(handle &h, const cplx *psi, long ld, int nst, double *rows) {
     a.ny = h.n[1];
     a.twx = h.axis[0].tw;
     a.twy = h.axis[1].tw;
-    fft3_moments(a, h.n, rows, h.stream);
-    rows += (long)nb * h.n[2] * 8;
+    a.gskip = plan.gskip;
+    a.glog = plan.glog;
+    fft3_moments(a, h.n, rows + (long)b0 * h.n[2] * 8, h.stream);
   }
 }
 
