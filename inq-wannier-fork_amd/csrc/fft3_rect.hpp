@@ -36,6 +36,28 @@ bool rect_z_launch_a(const fft3_args &a, int nz, rect_z_kernel k, hipStream_t st
 bool rect_z_launch_b(const fft3_args &a, int nz, rect_z_kernel k, hipStream_t stream);
 bool rect_z_launch_c(const fft3_args &a, int nz, rect_z_kernel k, hipStream_t stream);
 
+// Kernels of the x-y planes, by threads of their workgroups (explicitly instantiated
+// over the fft3_rect_x*.hip)
+enum rect_planes : int {
+  RECT_KINETIC,    // forward, 1/2 |G+k+A|^2, back
+  RECT_GATHER,     // psi at the owned points (G-space Hpsi)
+  RECT_POTENTIAL,  // to real space, V psi + V_nl psi, back (G-space Hpsi)
+  RECT_MOMENTS,    // sums of |psi^|^2 into rows (fft3_moments)
+  RECT_XY_PREPARE  // LDS attributes of the first three
+};
+
+// Most elements of a plane for a workgroup of NT threads
+constexpr int rect_elements(int NT) {
+  return NT == 128 ? 1280 : (NT == 256 ? 3072 : (NT == 512 ? 5120 : 10240));
+}
+
+inline size_t rect_xy_lds(const int n[3]) { return (size_t)n[0] * (n[1] | 1) * sizeof(cplx); }
+
+// Launches `what` for planes of n[0] x n[1] <= rect_elements(NT)
+template <int NT>
+void rect_xy_launch(const fft3_args &a, const int n[3], rect_planes what, double *rows,
+                    hipStream_t stream);
+
 // (length, radices of the z tiles): the lengths up to 96 that two or three
 // butterflies reach, from 20 on (shorter axes leave the sweeps' tiles mostly
 // empty), the cubic grids' with their plans
