@@ -249,6 +249,8 @@ void fft3_rect_fourier_hamiltonian(const fft3_args &a, const int n[3], hipStream
 // [nst n[2]][8] offset to the chunk's first band, bands at the offsets that they
 // have in psi (fft3_rect.hip; cubic grids too); where both plane axes have plans
 bool fft3_moments_supported(const int n[3], size_t max_lds);
+// Sets their LDS attributes (once, before any launch; fft3_rect_prepare does too)
+void fft3_moments_prepare(const int n[3]);
 void fft3_moments(const fft3_args &a, const int n[3], double *rows, hipStream_t stream);
 
 }  // namespace inqamd

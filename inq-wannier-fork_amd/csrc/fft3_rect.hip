@@ -68,7 +68,7 @@ void fft3_rect_prepare(const int n[3]) {
   if (lds > 65536)
     INQAMD_HIP_CHECK(hipFuncSetAttribute((const void *)rect_xy_proj_kernel,
                                          hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
-  rect_xy(fft3_args{}, n, RECT_XY_PREPARE, nullptr);
+  fft3_moments_prepare(n);
   rect_z(fft3_args{}, n[2], RECT_Z_PREPARE, nullptr);
 }
 
@@ -102,6 +102,8 @@ bool fft3_moments_supported(const int n[3], size_t max_lds) {
   return rect_length(n[0]) && rect_length(n[1]) && n[0] * n[1] <= rect_elements(1024) &&
          rect_xy_lds(n) <= max_lds;
 }
+
+void fft3_moments_prepare(const int n[3]) { rect_xy(fft3_args{}, n, RECT_XY_PREPARE, nullptr); }
 
 void fft3_moments(const fft3_args &a, const int n[3], double *rows, hipStream_t stream) {
   rect_xy(a, n, RECT_MOMENTS, stream, rows);

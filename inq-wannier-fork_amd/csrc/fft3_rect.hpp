@@ -43,7 +43,7 @@ enum rect_planes : int {
   RECT_GATHER,     // psi at the owned points (G-space Hpsi)
   RECT_POTENTIAL,  // to real space, V psi + V_nl psi, back (G-space Hpsi)
   RECT_MOMENTS,    // sums of |psi^|^2 into rows (fft3_moments)
-  RECT_XY_PREPARE  // LDS attributes of the first three
+  RECT_XY_PREPARE  // LDS attributes of them all
 };
 
 // Most elements of a plane for a workgroup of NT threads

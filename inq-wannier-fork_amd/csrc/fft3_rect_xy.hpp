@@ -372,13 +372,13 @@ void rect_xy_launch(const fft3_args &a, const int n[3], rect_planes what, double
       hipLaunchKernelGGL((rect_xy_kernel<NT, RECT_POTENTIAL>), planes, nt, lds, stream, a, n[2]);
       break;
     case RECT_MOMENTS:
-      attribute((const void *)rect_moments_kernel<NT>);  // (cubic handles prepare no planes)
       hipLaunchKernelGGL(rect_moments_kernel<NT>, planes, nt, lds, stream, a, n[2], rows);
       break;
     case RECT_XY_PREPARE:
       attribute((const void *)rect_xy_kernel<NT, RECT_KINETIC>);
       attribute((const void *)rect_xy_kernel<NT, RECT_GATHER>);
       attribute((const void *)rect_xy_kernel<NT, RECT_POTENTIAL>);
+      attribute((const void *)rect_moments_kernel<NT>);
       return;
   }
   INQAMD_HIP_CHECK(hipGetLastError());

@@ -129,7 +129,10 @@ void ensure_workspace(handle &h) {
 
 void ensure_blas(handle &h) {
   gs_state &g = state(h);
-  if (!g.blas) GS_BLAS_CHECK(rocblas_create_handle(&g.blas));
+  if (!g.blas) {
+    rotate_prepare();
+    GS_BLAS_CHECK(rocblas_create_handle(&g.blas));
+  }
   if (!g.S) g.S = (cplx *)dalloc((size_t)h.max_bands * h.max_bands * sizeof(cplx));
   if (!g.T) g.T = (cplx *)dalloc((size_t)h.max_bands * h.max_bands * sizeof(cplx));
   if (!g.chol) g.chol = (cplx *)dalloc((size_t)cholesky_scratch(h.max_bands) * sizeof(cplx));

@@ -1125,6 +1125,7 @@ static void create(handle &h, const inqamd_system_desc &d, hipStream_t stream) {
         fft3_rect_prepare(h.n);
       else
         fft3_prepare(h.n[0]);
+      if (!h.rect && gspace_sums_supported(h)) fft3_moments_prepare(h.n);
       INQAMD_HIP_CHECK(hipStreamCreateWithFlags(&h.aux, hipStreamNonBlocking));
       INQAMD_HIP_CHECK(hipEventCreateWithFlags(&h.ev_fork, hipEventDisableTiming));
       INQAMD_HIP_CHECK(hipEventCreateWithFlags(&h.ev_join, hipEventDisableTiming));

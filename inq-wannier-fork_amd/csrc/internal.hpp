@@ -207,6 +207,8 @@ void gram(const cplx *A, long lda, const cplx *B, long ldb, int nst, long npoint
 // rotate.hip: phi <- phi M in place, M row-major nst x nst (upper triangular with
 // zeros below, or full), where 16 rows of phi fit in LDS
 bool rotate_supported(int nst, size_t max_lds);
+// Sets the kernels' LDS attributes (once, before any launch)
+void rotate_prepare();
 void rotate(cplx *phi, long ld, int nst, long npoint, const cplx *M, bool upper, size_t max_lds,
             hipStream_t stream);
 // out[i][k] = conj(W[k][i]), both row-major n x n

@@ -119,11 +119,6 @@ void rotate_launch(cplx *phi, long ld, int nst, long npoint, const cplx *M, bool
                    hipStream_t stream) {
   constexpr int P = 16 * RT * RG;
   const size_t lds = (size_t)P * rotate_stride(nst) * sizeof(cplx);
-  const void *k = tri ? (const void *)rotate_kernel<RT, RG, NW, true>
-                      : (const void *)rotate_kernel<RT, RG, NW, false>;
-  if (lds > 65536)
-    INQAMD_HIP_CHECK(
-        hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
   const dim3 grid((unsigned)((npoint + P - 1) / P));
   if (tri)
     hipLaunchKernelGGL((rotate_kernel<RT, RG, NW, true>), grid, dim3(64 * NW), lds, stream, phi,
@@ -135,6 +130,16 @@ void rotate_launch(cplx *phi, long ld, int nst, long npoint, const cplx *M, bool
 }
 
 }  // namespace
+
+void rotate_prepare() {
+  for (const void *k : {(const void *)rotate_kernel<1, 4, 4, true>,
+                        (const void *)rotate_kernel<1, 4, 4, false>,
+                        (const void *)rotate_kernel<2, 1, 8, true>,
+                        (const void *)rotate_kernel<2, 1, 8, false>,
+                        (const void *)rotate_kernel<1, 1, 8, true>,
+                        (const void *)rotate_kernel<1, 1, 8, false>})
+    INQAMD_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
+}
 
 bool rotate_supported(int nst, size_t max_lds) {
   return (size_t)16 * rotate_stride(nst) * sizeof(cplx) <= max_lds;
