@@ -804,11 +804,12 @@ void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int s
     INQAMD_HIP_CHECK(hipEventRecord(h.ev_fork, h.stream));
     INQAMD_HIP_CHECK(hipStreamWaitEvent(h.aux, h.ev_fork, 0));
   }
-  // power n sits in buffer (n - 1) % 3: of the (at most three) powers pending at
-  // order n only the oldest shares its buffer, and the sweep reads that one at
+  // power n sits in buffer (n - 1) % keep: of the (at most `keep`) powers pending
+  // at order n only the oldest shares its buffer, and the sweep reads that one at
   // each point before it writes there
   static_assert(TAYLOR_PENDING == 3, "one buffer per pending power");
   cplx *buf[TAYLOR_PENDING] = {h.hn, h.hn2, h.hn3};
+  const int keep = h.hn3 ? 3 : 2;
   for (int c = 0; c < plan.n; c++) {
     const int b0 = plan.b0(c), nb = plan.nb(c);
     hipStream_t s = two && (c & 1) ? h.aux : h.stream;
@@ -817,9 +818,9 @@ void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int s
     long sld = ild;
     int first = 1;  // first power that no sum holds yet
     for (int n = 1; n <= order; n++) {
-      auto power = [&](int m) { return outs && outs[m - 1] ? outs[m - 1] : buf[(m - 1) % 3]; };
+      auto power = [&](int m) { return outs && outs[m - 1] ? outs[m - 1] : buf[(m - 1) % keep]; };
       cplx *dst = power(n) + b0;
-      const bool keep = n < order || (outs && outs[n - 1]);
+      const bool stored = n < order || (outs && outs[n - 1]);
       project_expand_args pa;
       if (beside)
         pa = projector_chunk_args(h, src, sld, nst, b0, nb, plan.gskip, plan.glog);
@@ -827,7 +828,7 @@ void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int s
         projector_project_p4_chunk(h, src, sld, nst, b0, nb, plan.gskip, plan.glog, s,
                                    two ? (c & 1) : 0);
       taylor_acc acc;
-      if (n == order || n - first == TAYLOR_PENDING) {
+      if (n == order || n - first == keep) {
         acc.p1 = p1;
         acc.ld1 = ld1;
         if (init1 && first == 1) acc.src1 = in, acc.lds1 = ild;
@@ -852,7 +853,7 @@ void taylor_chain(handle &h, const cplx *in, long ild, int nst, int order, int s
       local_passes(h, src, sld, dst, nst, nb, slot, b0, nst, &acc, 1, s, W, plan.gskip, plan.glog,
                    false, false, beside ? &pa : nullptr);
       local_passes(h, src, sld, dst, nst, nb, slot, b0, nst, &acc, 2, s, W, plan.gskip, plan.glog,
-                   n < order, !keep);
+                   n < order, !stored);
       src = dst;
       sld = nst;
     }
@@ -1028,6 +1029,15 @@ static void *dalloc(size_t bytes) {
   return p;
 }
 
+// Whether an array that only saves time may be allocated: where it takes at most an
+// eighth of the free memory, so that a run whose other arrays fill the device still
+// finds room for them
+static bool spare(size_t bytes) {
+  size_t free = 0, total = 0;
+  INQAMD_HIP_CHECK(hipMemGetInfo(&free, &total));
+  return bytes <= free / 8;
+}
+
 static void release(handle &h) {
   gs_release(h);
   td_release(h);
@@ -1146,7 +1156,6 @@ static void create(handle &h, const inqamd_system_desc &d, hipStream_t stream) {
   h.work = (cplx *)dalloc(orb);
   h.hn = (cplx *)dalloc(orb);
   h.hn2 = (cplx *)dalloc(orb);
-  if (h.three_sweep) h.hn3 = (cplx *)dalloc(orb);
   const long nchunk = (h.npoint + EN_CHUNK - 1) / EN_CHUNK;
   h.npartial = nchunk * h.max_bands * 2;
   h.partial = (double *)dalloc(h.npartial * sizeof(double));
@@ -1154,8 +1163,13 @@ static void create(handle &h, const inqamd_system_desc &d, hipStream_t stream) {
                    d.coeff, d.nlm, d.sphere_size);
   if (h.pt.nproj > 0)
     h.proj = (cplx *)dalloc((size_t)h.pt.nproj * h.pt.max_nlm * h.max_bands * sizeof(cplx));
-  if (h.pt.nproj > 0 && h.pt.nunique > 0 && h.three_sweep)
-    h.vnl = (cplx *)dalloc((size_t)h.pt.nent * h.max_bands * sizeof(cplx));
+  if (h.pt.nproj > 0 && h.pt.nunique > 0 && h.three_sweep) {
+    const size_t vnl = (size_t)h.pt.nent * h.max_bands * sizeof(cplx);
+    if (h.rect && !spare(vnl))
+      h.rect = h.three_sweep = false;  // (the pencil passes need no such array)
+    else
+      h.vnl = (cplx *)dalloc(vnl);
+  }
   if (h.pt.nproj > 0) {
     const size_t mom = (size_t)h.pt.nproj * h.pt.max_nlm * 4 * h.max_bands * sizeof(cplx);
     h.mom_a = (cplx *)dalloc(mom);
@@ -1166,6 +1180,8 @@ static void create(handle &h, const inqamd_system_desc &d, hipStream_t stream) {
     h.proj_part = (double *)dalloc(PROJ_PART_TILES * 256 * sizeof(double));
   }
   h.obs = (double *)dalloc(observables_scratch_doubles(h) * sizeof(double));
+  // (last, and only a luxury: without it Taylor chains keep two powers)
+  if (h.three_sweep && spare(orb)) h.hn3 = (cplx *)dalloc(orb);
 }
 
 }  // namespace inqamd

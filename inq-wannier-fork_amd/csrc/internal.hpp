@@ -126,7 +126,8 @@ struct inqamd_hamiltonian {
   inqamd::cplx *work = nullptr; // [N][max_bands] FFT intermediate
   inqamd::cplx *hn = nullptr;   // [N][max_bands] Taylor H^n psi
   inqamd::cplx *hn2 = nullptr;  // [N][max_bands] Taylor ping-pong
-  inqamd::cplx *hn3 = nullptr;  // [N][max_bands] third power of a Taylor chain (three-sweep)
+  inqamd::cplx *hn3 = nullptr;  // [N][max_bands] third power of a Taylor chain (three-sweep,
+                                // where memory is not short)
   inqamd::cplx *proj = nullptr; // [nproj][max_nlm][max_bands]
   inqamd::cplx *vnl = nullptr;  // [nent][max_bands] V_nl psi per ownership entry
   double *partial = nullptr;    // reduction partials
