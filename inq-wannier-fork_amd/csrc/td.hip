@@ -1265,13 +1265,24 @@ int inqamd_td_create(inqamd_hamiltonian_t h, const inqamd_td_desc *desc, inqamd_
     td->nb = d.band_slice == 0 || d.band_slice > d.nst ? d.nst : d.band_slice;
     td->nseg = (d.nsteps + d.checkpoint_every - 1) / d.checkpoint_every;
     lattice_dot(*h, d.direction, td->dir_cov);
-    td->fused = h->three_sweep && d.store_powers;
-    td->nstore = td->fused ? 2 * d.order : (d.store_powers ? d.order : 1);
     const long N = h->npoint;
     const size_t full = (size_t)N * d.nst * sizeof(cplx);
     const size_t slice = (size_t)N * td->nb * sizeof(cplx);
     const int K = d.checkpoint_every < (d.nsteps > 0 ? d.nsteps : 1) ? d.checkpoint_every
                                                                       : (d.nsteps > 0 ? d.nsteps : 1);
+    // The fused half steps keep the transforms of the powers too, twice the tape.  On
+    // a non-cubic grid, where the powers alone do without them, only if that fits.
+    td->fused = h->three_sweep && d.store_powers;
+    if (td->fused && h->rect) {
+      size_t free = 0, total = 0;
+      INQAMD_HIP_CHECK(hipMemGetInfo(&free, &total));
+      const size_t mom = (size_t)h->pt.nproj * h->pt.max_nlm * 4 * td->nb * sizeof(cplx);
+      const size_t sph = (size_t)h->pt.nproj * h->pt.max_sphere * td->nb * sizeof(cplx);
+      const size_t need = full * (td->nseg + 1) + slice * (4 * (size_t)K * d.order + 2 * d.order + 4) +
+                          2 * mom * d.order + sph + (size_t)N * sizeof(double);
+      td->fused = need <= free - free / 64;  // (a little is lost to the allocator's pages)
+    }
+    td->nstore = td->fused ? 2 * d.order : (d.store_powers ? d.order : 1);
     td->ckpt = (cplx *)td_alloc(td, full * (td->nseg + 1));
     td->tape = (cplx *)td_alloc(td, slice * 2 * K * td->nstore);
     td->cur = (cplx *)td_alloc(td, slice);
