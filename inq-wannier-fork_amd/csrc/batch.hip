@@ -701,14 +701,15 @@ void batch_run(inqamd_batch *b) {
     void *args[] = {(void *)&pc, (void *)&np, (void *)&cnt, (void *)&total};
     INQAMD_HIP_CHECK(hipLaunchKernel(k, dim3(grid), dim3(nt), args, lds, cs));
   };
-  if (b->group_by_grid) {
-    // The groups (one grid length each) are independent: the largest first, each
-    // with its three sweeps in a row on the stream with the least work so far,
-    // so that the small groups, which leave most of the chip idle, run beside
-    // others and a group's W is read back soon after it is written (every group's
-    // first sweep, then every second and third, chunk by chunk: 1177 us for eight
-    // systems of 24^3 to 72^3 with 9 to 64 bands, 1124 so).  The main stream starts
-    // behind: it runs the projector first.
+  if (b->group_by_grid && (int)b->chunks.size() < ns) {
+    // Fewer chunks than streams: the groups (one grid length each) are independent,
+    // so the largest first, each with its three sweeps in a row on the stream with
+    // the least work so far.  The small groups, which leave most of the chip idle,
+    // run beside others and a group's W is read back soon after it is written: eight
+    // systems of 24^3 to 72^3 with 9 to 64 bands take 1115 us, 1177 in the order
+    // below.  The main stream starts behind: it runs the projector first.  Where the
+    // chunks fill the streams that order keeps more of W in cache: 24 systems in six
+    // chunks take 4.67 ms so and 4.73 by groups.
     std::vector<int> order(b->groups.size());
     for (size_t i = 0; i < order.size(); i++) order[i] = (int)i;
     auto work = [&](int gi) { return (long)b->groups[gi].zitems * b->groups[gi].L; };
