@@ -119,8 +119,8 @@ __device__ __forceinline__ void gram_block(const gram_args &a, int rb, int cb, l
 
 // Workgroup: slice blockIdx.x, pair of band blocks blockIdx.y (those off the
 // diagonal, which have more tiles, first).  The pairs of a slice run at about the
-// same time on one XCD (gridDim.x is a multiple of 8 wherever there are several)
-// and share its loads in L2.  OFF: there are pairs off the diagonal (their tiles'
+// same time on one XCD where gridDim.x is a multiple of 8, and share its loads in
+// L2.  OFF: there are pairs off the diagonal (their tiles'
 // registers would cost a lone block its other waves).
 template <int T, bool SAME, bool OFF>
 __global__ __launch_bounds__(256) void gram_kernel(const gram_args a) {
@@ -178,13 +178,17 @@ constexpr int GRAM_BLOCKS = 1024;  // workgroups of a launch, about
 }  // namespace
 
 // Slices of the point sum: about GRAM_BLOCKS workgroups over the pairs of band
-// blocks, results of at most a quarter of the bands' own size, whole multiples of 8
+// blocks, results of at most a quarter of the bands' own size; whole multiples of 8
+// where there are that many, any number below (one slice for all of them there took
+// 28.7 ms where an orthogonalisation at 48^3 x 961 bands takes 22.4, and 2990 us for
+// 1490 at 24^3 x 433)
 int gram_slices(long npoint, int nst) {
   const int nblk = (nst + 63) / 64, pairs = nblk * (nblk + 1) / 2;
   long c = GRAM_BLOCKS / pairs;
   if (c > npoint / (4L * nst)) c = npoint / (4L * nst);
   if (c > 512) c = 512;
-  return c < 8 ? 1 : (int)(c / 8 * 8);
+  if (c >= 8) c = c / 8 * 8;
+  return c < 1 ? 1 : (int)c;
 }
 
 // part: gram_slices nst^2 values of scratch

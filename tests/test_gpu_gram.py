@@ -1,6 +1,6 @@
 """The inner products of the eigensolver at the edges of their tiles (16 bands) and
-blocks (64 bands), on grids that leave a short last slice or allow only one, in
-both uses: the overlap matrix of orthogonalize against the CPU oracle, and the
+blocks (64 bands), on grids that leave a short last slice, allow a few or only
+one, in both uses: the overlap matrix of orthogonalize against the CPU oracle, and the
 subspace Hamiltonian by its eigenvalues against numpy's of the same matrix.
 
 Tolerance 1e-12 relative: sums over up to 5e4 points in another order, times a
@@ -22,7 +22,7 @@ TOL = 1e-12
 @pytest.mark.parametrize("n,nst", [((12, 10, 14), 1), ((12, 10, 14), 16), ((12, 11, 10), 17),
                                    ((24, 24, 24), 33), ((32, 27, 25), 48), ((24, 25, 20), 49),
                                    ((12, 11, 10), 64), ((32, 27, 25), 65), ((36, 36, 36), 97),
-                                   ((36, 36, 36), 130)])
+                                   ((36, 36, 36), 130), ((12, 12, 12), 60), ((8, 10, 9), 97)])
 def test_inner_products(device, n, nst):
     print("[gpu-test] gram", n, nst, flush=True)
     lat = np.diag([0.4 * m for m in n])
