@@ -19,7 +19,8 @@ TOL = 1e-12
 
 @pytest.mark.parametrize("n,nst", [((12, 10, 14), 1), ((12, 10, 14), 16), ((12, 10, 14), 63),
                                    ((12, 11, 10), 64), ((12, 10, 14), 65), ((64, 64, 64), 3),
-                                   ((72, 80, 90), 50), ((60, 60, 50), 17)])
+                                   ((72, 80, 90), 50), ((60, 60, 50), 17),
+                                   ((50, 50, 54), 130)])
 def test_preconditioner_shapes(device, n, nst):
     """operations::preconditioner: the kinetic sums and their use."""
     print("[gpu-test] reductions", n, nst, flush=True)

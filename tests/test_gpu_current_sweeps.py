@@ -20,7 +20,7 @@ TOL = 1e-12
 @pytest.mark.parametrize("n,nst,chunk", [
     ((20, 20, 20), 1, 0), ((20, 25, 24), 11, 8), ((24, 24, 24), 9, 0),
     ((36, 32, 27), 5, 0), ((48, 48, 48), 4, 0), ((72, 75, 20), 3, 0),
-    ((96, 96, 20), 2, 0), ((80, 80, 80), 2, 0),
+    ((96, 96, 20), 2, 0), ((80, 80, 80), 2, 0), ((60, 64, 24), 5, 0), ((64, 64, 64), 3, 0),
 ])
 def test_current(device, n, nst, chunk):
     print("[gpu-test] current", n, nst, chunk, flush=True)

@@ -58,6 +58,7 @@ def test_every_length_on_every_axis(device, length):
 @pytest.mark.parametrize("n,nst,natoms", [
     ((96, 96, 20), 3, 2), ((64, 90, 25), 9, 3), ((48, 50, 36), 17, 4), ((24, 27, 80), 8, 3),
     ((25, 25, 25), 11, 2), ((90, 90, 90), 2, 0), ((20, 20, 20), 5, 1),
+    ((60, 64, 20), 3, 0), ((72, 70, 24), 5, 0), ((60, 64, 20), 9, 3), ((72, 70, 24), 3, 2),
 ])
 def test_hpsi_gspace_and_etrs(device, n, nst, natoms):
     s, psi, osys, ham, d, kA = check(device, n, nst, natoms)
