@@ -68,7 +68,8 @@ typedef struct {
  * Replaces ks_hamiltonian's constructor (ks_hamiltonian.hpp:79-89) and
  * projector_all(projectors) (projector_all.hpp:86-94).  `stream` is a
  * hipStream_t (NULL = default stream).  Allocates every workspace the later
- * calls need, so they allocate nothing -- except the ground-state calls
+ * calls need (and, where that takes at most an eighth of the free memory, one
+ * more orbital array that only saves time), so they allocate nothing -- except the ground-state calls
  * (orthogonalize, preconditioner, steepest_descent, subspace_diagonalization)
  * and the interacting TDDFT calls (density ... etrs_scf_step), which allocate their own
  * workspace on first use. */
@@ -108,9 +109,11 @@ int inqamd_stream_probe(int kind, const void *src, void *dst, long rows, int ld,
  *   xy_threads       x-y plane workgroups of 1 or 2 x plane_threads(L)
  *   band_chunk       bands per chunk of the sweeps (multiple of 8, <= max_bands)
  *   projector_bands  bands per workgroup of the projector coefficients (16/32/64)
- * z_tile_y, band_chunk and projector_bands change no result bit; xy_threads
- * selects another instantiation of the plane kernel, whose floating-point
- * contraction may differ in the last bits. */
+ * z_tile_y and xy_threads act on cubic grids only.  z_tile_y, band_chunk and
+ * projector_bands change no result bit; xy_threads selects another instantiation
+ * of the plane kernel, whose floating-point contraction may differ in the last
+ * bits, and, with few projectors, whether their point sums run beside the planes
+ * (unsplit) or in launches of their own. */
 typedef struct {
   int z_tile_y;
   int xy_threads;
@@ -138,8 +141,8 @@ int inqamd_hamiltonian_apply(inqamd_hamiltonian_t h, const void *psi, void *hpsi
  * forward transform of the real-space orbitals), same layout.  Must not alias. */
 int inqamd_hamiltonian_apply_fourier(inqamd_hamiltonian_t h, const void *phi, void *hphi,
                                      int nst, int ld);
-/* Diagnostic: one Hpsi (as inqamd_hamiltonian_apply, three-sweep path only)
- * with HIP events around each kernel on the handle's stream.  ms[0]: the
+/* Diagnostic: one Hpsi (as inqamd_hamiltonian_apply, the three-sweep path of cubic
+ * grids only, the projector always in launches of its own) with HIP events around each kernel on the handle's stream.  ms[0]: the
  * projector (phases + gather/MFMA/expand), ms[1..3]: the z-forward, x-y and
  * z-backward sweeps summed over band chunks; launches[] the kernel launches
  * each figure covers.  Synchronises.  No reference counterpart. */
@@ -375,7 +378,9 @@ typedef struct {
   double direction[3];      /* Cartesian polarisation of A and of the loss */
   int checkpoint_every;     /* steps per checkpoint segment (>= 1) */
   int band_slice;           /* bands per backward slice (0: all) */
-  int store_powers;         /* 1: keep H^j phi of a segment's half steps; 0: recompute */
+  int store_powers;         /* 1: keep H^j phi of a segment's half steps, with their
+                               transforms on three-sweep grids (twice the tape; on
+                               non-cubic ones where that fits); 0: recompute */
   int commutator;           /* the loss's [V_nl, r] form: INQAMD_COMMUTATOR_INQ (0) or
                                INQAMD_COMMUTATOR_CORRECTED (see inqamd_current) */
 } inqamd_td_desc;

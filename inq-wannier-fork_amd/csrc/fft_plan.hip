@@ -18,8 +18,8 @@
 // every axis; 64^3 x 128 1239 -> 1222 us, and one field of 64^3 (nst = 1, 15 of
 // 16 lanes idle before) 381 -> 237 us for its Hartree and PBE potentials.
 //
-// Instantiated for the lengths that factor into the butterflies below up to
-// 128; other lengths go to fft_dense.hip and fft.hip.
+// Instantiated for the lengths tabulated below; the others (98 and 105 among them)
+// go to fft_dense.hip and fft.hip.
 
 #include "fft.hpp"
 #include "fft_dft.hpp"

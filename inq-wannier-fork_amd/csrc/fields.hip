@@ -381,6 +381,11 @@ struct field_launch {
 
 }  // namespace
 
+// All lengths that the product takes.  Its work grows with the length, but the
+// passes still win where they end: PBE of 120^3 353 us against 426 with a pass for
+// each step, of 144^3 1475 against 1675, of 180^3 2916 against 3140, of 191 x 190 x
+// 187 1918 against 2214 (only 128^3, whose strides are powers of two, 555 against
+// 486); Poisson of 144^3 340 against 669, of 180^3 596 against 1160.
 bool fields_supported(const handle &h) {
   return h.n[0] <= DENSE_MAX_LEN && h.n[1] <= DENSE_MAX_LEN && h.n[2] <= DENSE_MAX_LEN;
 }

@@ -11,7 +11,8 @@ z-tile shape, chunk and projector bands change no result bit (the sweeps'
 arithmetic per column is the same for every shape, and the projector's point
 chunking follows from the band count alone); the x-y thread count selects
 another instantiation of the plane kernel, whose floating-point contraction
-may differ in the last bits.  The table is a speed choice.
+may differ in the last bits (and whether few projectors' point sums run beside
+the planes).  The table is a speed choice.
 """
 import itertools
 import json
