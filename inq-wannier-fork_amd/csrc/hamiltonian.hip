@@ -754,7 +754,8 @@ void copy(handle &h, const cplx *x, long xld, cplx *y, long yld, int nst) {
 // The sums are formed in one sweep out of every four: up to three powers wait
 // in buffers of their own (H^n in is written in any case) and the fourth
 // order's sweep reads them with the sums' old values and adds all four terms,
-// in the order of the recurrence.  Adding each power in its own sweep reads and
+// in the order of the recurrence (one sweep in three where memory left the handle
+// without hn3).  Adding each power in its own sweep reads and
 // writes every sum in every order: a Taylor-4 sum moved 496 B per point and
 // band where this moves 448, and the 2-for-1 sum 608 where this moves 464 (HBM
 // bounds every sweep): the interacting step of 64^3 x 256 bands 23.70 -> 20.53
